@@ -54,6 +54,10 @@ struct bes_ctx {
   std::vector<double> node_xyz;      // [nnode][nd] mesh nodes (solution files)
   std::vector<int64_t> cell_nodes;   // [ncell][nd+1] cell vertices (solution files)
   std::vector<int64_t> perm, iperm;  // perm[new] = old cell, iperm[old] = new
+  int *diperm = nullptr;             // iperm on the device
+  double *stage = nullptr;           // staging of the host copies, callers' layout (grown on demand)
+  size_t stage_bytes = 0;
+  unsigned long long *hmon = nullptr;  // pinned: Linf monitors [nv][B] and the failing-face word
   int nd = 0, nv = 0, k = 0, N = 0;
   bes::GasConst gc{};
   double venkat_k = 5.0;
@@ -86,8 +90,8 @@ struct bes_ctx {
   std::vector<char> lim_frozen;      // [B]
   int lim_epoch = 0;                 // changes with the freeze state (graph captures hold it)
   // reduction scratch: [0, 64) global-dt minimum per condition, [64, 64 + nv*B)
-  // Linf bit patterns [v][B]
-  static constexpr int kRedWords = 64 + 5 * kMaxBatch;
+  // Linf bit patterns [v][B] and the failing-face word after them
+  static constexpr int kRedWords = 64 + 5 * kMaxBatch + 1;
   unsigned long long *red = nullptr;
   unsigned long long *lbits = nullptr;  // Linf monitor words [kLinfSlots][nv][B] (see kernels_common.hpp)
   unsigned long long *err = nullptr;   // first failing device face, ~0 if none

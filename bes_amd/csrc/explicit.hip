@@ -503,13 +503,12 @@ __global__ void k_linf_decode(const unsigned long long *bits, double *out, int n
   if (dit && q == 0) *dit = it + 1;
 }
 
-// bits[q] = max over the Linf copies (copy 0 in place)
-__global__ void k_linf_reduce(unsigned long long *bits, int nq) {
+// out[q] = max over the Linf copies, out[nq] = the failing-face word
+__global__ void k_linf_reduce(const unsigned long long *bits, int nq, const unsigned long long *err,
+                              unsigned long long *out) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < nq) {
-    const unsigned long long m = linf_slots_max(bits, nq, q);
-    bits[q] = m;
-  }
+  if (q < nq) out[q] = linf_slots_max(bits, nq, q);
+  if (q == 0) out[nq] = *err;
 }
 
 // Persistent form of bes_explicit_run for one condition with local time
@@ -572,6 +571,47 @@ __global__ __launch_bounds__(256) void k_explicit_persistent(PersistStep a, DevM
       double *t = U0;
       U0 = Ua;
       Ua = t;
+    }
+  }
+}
+
+// Rows between the device layout (cells in Morton order, value q of cell i and
+// condition b at (q*sq + i*si)*B + b) and a staging buffer in the callers'
+// layout ([B][ne][ncomp], cells e0 .. e0+ne-1 in mesh order).  A block moves
+// kMoveRows (cell, condition) rows through LDS, so both sides are read and
+// written in runs: B values of one cell on the device side, the block's cells
+// of one condition on the staging side.  Bound by the PCIe copy beside it; the
+// permutation in a serial host loop took 27 ns per row (64 conditions x 31k
+// tetrahedra, 79 MB: state in and out 108 ms, with the kernel 7 ms).
+constexpr int kMoveRows = 256;
+template <bool TO_HOST>
+__global__ __launch_bounds__(256) void k_move_rows(double *__restrict__ dev, size_t sq, size_t si,
+                                                   double *__restrict__ stage, const int *__restrict__ iperm, int e0,
+                                                   int ne, int ncomp, int lgB) {
+  extern __shared__ double sm_rows[];
+  const int B = 1 << lgB, ct = kMoveRows >> lgB;   // cells of a block
+  const int eb = blockIdx.x * ct, nc = min(ct, ne - eb), run = nc * ncomp;
+  const int nval = kMoveRows * ncomp;
+  if constexpr (!TO_HOST) {
+    for (int t = threadIdx.x; t < run << lgB; t += blockDim.x) {
+      const int b = t / run, r = t - b * run;
+      sm_rows[t] = stage[((size_t)b * ne + eb) * ncomp + r];
+    }
+    __syncthreads();
+  }
+  for (int t = threadIdx.x; t < nval; t += blockDim.x) {
+    const int q = t / kMoveRows, r = t & (kMoveRows - 1), e = r >> lgB, b = r & (B - 1);
+    if (e >= nc) continue;
+    const size_t at = ((q * sq + (size_t)iperm[e0 + eb + e] * si) << lgB) + b;
+    const int l = (b * nc + e) * ncomp + q;
+    if constexpr (TO_HOST) sm_rows[l] = dev[at];
+    else dev[at] = sm_rows[l];
+  }
+  if constexpr (TO_HOST) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < run << lgB; t += blockDim.x) {
+      const int b = t / run, r = t - b * run;
+      stage[((size_t)b * ne + eb) * ncomp + r] = sm_rows[t];
     }
   }
 }
@@ -795,6 +835,14 @@ static int create_from_input(const MeshInput &in, int geom_mode, const bes_gas *
     bes_ctx_destroy(c);
     return s;
   }
+  he = hipHostMalloc((void **)&c->hmon, (5 * bes_ctx::kMaxBatch + 1) * sizeof(unsigned long long),
+                     hipHostMallocDefault);
+  if (he != hipSuccess) {
+    c->hmon = nullptr;
+    s = hip_fail(he, "hipHostMalloc");
+    bes_ctx_destroy(c);
+    return s;
+  }
   // default freestream: Mach 0 (Config.cpp:481-487 form)
   double fi[6] = {1.0, 0, 0, 0, 0, 0};
   fi[nd + 1] = 1.0 / c->gc.gamma;
@@ -812,16 +860,21 @@ static int reset_err(bes_ctx *c) {
   return BES_OK;
 }
 
-static int check_err(bes_ctx *c) {
-  unsigned long long e = 0;
-  BES_HIP(hipMemcpyAsync(&e, c->err, sizeof(e), hipMemcpyDeviceToHost, c->stream));
-  BES_HIP(hipStreamSynchronize(c->stream));
+// status of a pass from its failing-face word
+static int face_status(bes_ctx *c, unsigned long long e) {
   if (e != ~0ull) {
     c->last_err_face = e < c->fref.size() ? (long)c->fref[e] : -1;   // device face -> reference id
     set_error("non-finite flux at face " + std::to_string(c->last_err_face));
     return BES_ERR_NAN;
   }
   return BES_OK;
+}
+
+static int check_err(bes_ctx *c) {
+  unsigned long long e = 0;
+  BES_HIP(hipMemcpyAsync(&e, c->err, sizeof(e), hipMemcpyDeviceToHost, c->stream));
+  BES_HIP(hipStreamSynchronize(c->stream));
+  return face_status(c, e);
 }
 
 // launch helpers shared with the implicit path
@@ -935,31 +988,99 @@ int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int 
   return BES_OK;
 }
 
-// device (Morton order, [comp][N][B]) <-> host (reference order, [B][ncell][comp])
-int state_to_host(bes_ctx *c, const double *dsoa, int ncomp, double *host) {
-  const size_t N = c->N, B = c->B;
-  std::vector<double> tmp(ncomp * N * B);
-  BES_HIP(hipMemcpyAsync(tmp.data(), dsoa, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+// Staging of the host copies: grown on demand to at most kStageBytes (larger
+// arrays go through it in chunks of cells), kept by the context.
+constexpr size_t kStageBytes = (size_t)128 << 20;
+// Arrays up to this size are permuted on the host: the values sit in the CPU's
+// caches, while the kernel adds a launch and a copy that must wait for it (9k
+// triangles, 0.28 MB: state out 34 us by the loop, 60 by the kernel; 40k
+// triangles, 1.2 MB: 202 and 135).
+constexpr size_t kHostLoopBytes = (size_t)512 << 10;
+static int stage_room(bes_ctx *c, size_t want) {
+  want = std::min(want, kStageBytes);
+  if (c->stage_bytes >= want) return BES_OK;
   BES_HIP(hipStreamSynchronize(c->stream));
-  for (size_t b = 0; b < B; b++)
-    for (size_t i = 0; i < N; i++) {
-      const int64_t e = c->perm[i];
-      for (int q = 0; q < ncomp; q++) host[(b * N + e) * ncomp + q] = tmp[((size_t)q * N + i) * B + b];
-    }
+  if (c->stage) hipFree(c->stage);
+  c->stage = nullptr;
+  c->stage_bytes = 0;
+  hipError_t e = hipMalloc((void **)&c->stage, want);
+  while (e == hipErrorOutOfMemory && want > ((size_t)1 << 20)) {   // less room: more chunks
+    (void)hipGetLastError();
+    want /= 2;
+    e = hipMalloc((void **)&c->stage, want);
+  }
+  if (e != hipSuccess) { c->stage = nullptr; return hip_fail(e, "hipMalloc(staging)"); }
+  c->stage_bytes = want;
   return BES_OK;
 }
 
-int state_to_device(bes_ctx *c, const double *host, int ncomp, double *dsoa) {
-  const size_t N = c->N, B = c->B;
-  std::vector<double> tmp(ncomp * N * B);
-  for (size_t b = 0; b < B; b++)
-    for (size_t i = 0; i < N; i++) {
-      const int64_t e = c->perm[i];
-      for (int q = 0; q < ncomp; q++) tmp[((size_t)q * N + i) * B + b] = host[(b * N + e) * ncomp + q];
+// device rows (value q of cell i, condition b at (q*sq + i*si)*B + b) <-> host
+// array [B][ncell][ncomp] in mesh order
+template <bool TO_HOST>
+static int move_rows(bes_ctx *c, double *dev, size_t sq, size_t si, int ncomp, double *host) {
+  const size_t N = c->N, B = c->B, row = (size_t)ncomp * sizeof(double);
+  if (N * B * row <= kHostLoopBytes) {
+    std::vector<double> tmp(N * B * ncomp);
+    // value q of the row of cell i, condition b
+    auto at = [&](size_t q, size_t i, size_t b) { return (q * sq + i * si) * B + b; };
+    if (TO_HOST) {
+      BES_HIP(hipMemcpyAsync(tmp.data(), dev, N * B * row, hipMemcpyDeviceToHost, c->stream));
+      BES_HIP(hipStreamSynchronize(c->stream));
     }
-  BES_HIP(hipMemcpyAsync(dsoa, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    for (size_t b = 0; b < B; b++)
+      for (size_t i = 0; i < N; i++) {
+        double *h = host + (b * N + c->perm[i]) * ncomp;
+        for (int q = 0; q < ncomp; q++) {
+          if (TO_HOST) h[q] = tmp[at(q, i, b)];
+          else tmp[at(q, i, b)] = h[q];
+        }
+      }
+    if (!TO_HOST) {
+      BES_HIP(hipMemcpyAsync(dev, tmp.data(), N * B * row, hipMemcpyHostToDevice, c->stream));
+      BES_HIP(hipStreamSynchronize(c->stream));
+    }
+    return BES_OK;
+  }
+  int s = stage_room(c, std::max((size_t)kMoveRows * row, N * B * row));
+  if (s) return s;
+  if (!c->diperm) {
+    const std::vector<int> ip(c->iperm.begin(), c->iperm.end());
+    if ((s = upload(&c->diperm, ip))) return s;
+  }
+  const size_t ct = kMoveRows / B, cells = std::max<size_t>(c->stage_bytes / (B * row) / ct, 1) * ct;
+  for (size_t e0 = 0; e0 < N; e0 += cells) {
+    const size_t ne = std::min(cells, N - e0);
+    auto kernel = [&]() {
+      hipLaunchKernelGGL(k_move_rows<TO_HOST>, dim3((unsigned)((ne + ct - 1) / ct)), dim3(256), kMoveRows * row,
+                         c->stream, dev, sq, si, c->stage, c->diperm, (int)e0, (int)ne, ncomp, c->lgB);
+      return hipGetLastError();
+    };
+    if (TO_HOST) BES_HIP(kernel());
+    // one copy for all conditions when the chunk is the whole mesh
+    const size_t ncopy = ne == N ? 1 : B, len = (ne == N ? B : 1) * ne * row;
+    for (size_t b = 0; b < ncopy; b++) {
+      double *h = host + (b * N + e0) * ncomp, *d = c->stage + b * ne * ncomp;
+      if (TO_HOST) BES_HIP(hipMemcpyAsync(h, d, len, hipMemcpyDeviceToHost, c->stream));
+      else BES_HIP(hipMemcpyAsync(d, h, len, hipMemcpyHostToDevice, c->stream));
+    }
+    if (!TO_HOST) BES_HIP(kernel());
+  }
   BES_HIP(hipStreamSynchronize(c->stream));
   return BES_OK;
+}
+
+// device (Morton order, [comp][N][B]) <-> host (reference order, [B][ncell][comp])
+int state_to_host(bes_ctx *c, const double *dsoa, int ncomp, double *host) {
+  return move_rows<true>(c, const_cast<double *>(dsoa), (size_t)c->N, 1, ncomp, host);
+}
+
+int state_to_device(bes_ctx *c, const double *host, int ncomp, double *dsoa) {
+  return move_rows<false>(c, dsoa, (size_t)c->N, 1, ncomp, const_cast<double *>(host));
+}
+
+// device vector [N][nv][B] -> host [B][ncell][nv]
+int vector_to_host(bes_ctx *c, const double *dvec, double *host) {
+  return move_rows<true>(c, const_cast<double *>(dvec), 1, (size_t)c->nv, c->nv, host);
 }
 
 static void drop_graph(bes_ctx *c) {
@@ -1059,10 +1180,11 @@ int bes_ctx_destroy(bes_ctx *c) {
                   c->dm.af, c->dm.cfd, c->dm.info, c->dm.cfq, c->dm.saq, c->dm.fo, c->dm.fnb, c->dm.fnr,
                   c->dm.frs, c->dm.frn,
                   c->FF, c->U0, c->Ua, c->Ub, c->LG, c->G, c->phi, c->phi_frz,
-                  c->dt, c->dtg, c->R, c->red, c->lbits, c->err, c->linf, c->dfinf, c->dit};
+                  c->dt, c->dtg, c->R, c->diperm, c->stage, c->red, c->lbits, c->err, c->linf, c->dfinf, c->dit};
   drop_graph(c);
   for (void *p : ptrs)
     if (p) hipFree(p);
+  if (c->hmon) hipHostFree(c->hmon);
   for (auto &p : c->ev_pending) { c->ev_pool.push_back(p.a); c->ev_pool.push_back(p.b); }
   for (hipEvent_t e : c->ev_pool) if (e) hipEventDestroy(e);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -1236,16 +1358,19 @@ int bes_compute_residual(bes_ctx *c, double *R_out, double *maxabs_out) {
   int s;
   if ((s = reset_err(c)) || (s = fill_bits(c, bits, kLinfSlots * nv * B, 0ull))) return s;
   if ((s = launch_residual(c, nullptr, nullptr, 0.0, 1, c->R, bits))) return s;
-  hipLaunchKernelGGL(k_linf_reduce, dim3(grid_for(nv * B, 64)), dim3(64), 0, c->stream, bits, nv * B);
-  if (maxabs_out) {
-    std::vector<unsigned long long> b(nv * B);
-    BES_HIP(hipMemcpyAsync(b.data(), bits, b.size() * 8, hipMemcpyDeviceToHost, c->stream));
+  // monitors and failing face in one copy, queued before the residual's: one wait
+  unsigned long long *out = c->red + 64;
+  hipLaunchKernelGGL(k_linf_reduce, dim3(grid_for(nv * B, 64)), dim3(64), 0, c->stream, bits, nv * B, c->err, out);
+  BES_HIP(hipMemcpyAsync(c->hmon, out, (size_t)(nv * B + 1) * 8, hipMemcpyDeviceToHost, c->stream));
+  if (R_out) {
+    if ((s = state_to_host(c, c->R, c->nv, R_out))) return s;
+  } else {
     BES_HIP(hipStreamSynchronize(c->stream));
-    for (int q = 0; q < B; q++)
-      for (int v = 0; v < nv; v++) std::memcpy(&maxabs_out[q * nv + v], &b[v * B + q], 8);
   }
-  if (R_out && (s = state_to_host(c, c->R, c->nv, R_out))) return s;
-  return check_err(c);
+  if (maxabs_out)
+    for (int q = 0; q < B; q++)
+      for (int v = 0; v < nv; v++) std::memcpy(&maxabs_out[q * nv + v], &c->hmon[v * B + q], 8);
+  return face_status(c, c->hmon[nv * B]);
 }
 
 // one pseudo-time step (SolverExplicit.cpp:259-393) on the context stream;

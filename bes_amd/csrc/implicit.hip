@@ -47,6 +47,7 @@ int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int 
                     unsigned long long *linf_bits);
 int state_to_host(bes_ctx *c, const double *dsoa, int ncomp, double *host);
 int state_to_device(bes_ctx *c, const double *host, int ncomp, double *dsoa);
+int vector_to_host(bes_ctx *c, const double *dvec, double *host);
 namespace lp {
 int lp_build(bes_ctx *c, Impl *im);
 int lp_release(Impl *im);
@@ -2065,15 +2066,7 @@ int bes_linear_solve(bes_ctx *c, int *iters, double *relres) {
 
 int bes_get_linear_solution(bes_ctx *c, double *x) {
   if (!c || !c->impl || !x) { set_error("no solution"); return BES_ERR_ARG; }
-  Impl *im = impl_of(c);
-  const int N = c->N, nv = c->nv, B = c->B;
-  std::vector<double> h((size_t)N * nv * B);
-  BES_HIP(hipMemcpy(h.data(), im->x, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int b = 0; b < B; b++)
-    for (int64_t e = 0; e < N; e++)
-      for (int v = 0; v < nv; v++)
-        x[((size_t)b * N + e) * nv + v] = h[((size_t)c->iperm[e] * nv + v) * B + b];
-  return BES_OK;
+  return vector_to_host(c, impl_of(c)->x, x);
 }
 
 int bes_amg_apply(bes_ctx *c, const double *r, double *z) {
