@@ -662,131 +662,453 @@ __device__ __forceinline__ void st_group(TV *__restrict__ v, size_t e, size_t n1
   }
 }
 
-// up to 8 dot products <V_(i0+q), w> and ||w||^2 per lane: S[(q*B + b)*L + l],
-// the norm in slot cnt
-template <typename TV>
-__global__ __launch_bounds__(256) void k_mdot(const TV *__restrict__ V, size_t stride, int i0, int cnt,
-                                              const TV *__restrict__ w, size_t n1, int lgB, int L,
-                                              double *__restrict__ S) {
-  const int B = 1 << lgB;
-  const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ((size_t)L << lgB)) return;
-  const size_t l = g >> lgB;
-  const int b = (int)(g & (B - 1));
-  double acc[9];
-#pragma unroll
-  for (int q = 0; q < 9; q++) acc[q] = 0;
-  for (size_t e = kLaneGroup * l; e < n1; e += (size_t)kLaneGroup * L) {
-    double wx[kLaneGroup];
-    ld_group(w, e, n1, lgB, b, wx);
-#pragma unroll
-    for (int q = 0; q < 8; q++)
-      if (q < cnt) {
-        double vx[kLaneGroup];
-        ld_group(V + (size_t)(i0 + q) * stride, e, n1, lgB, b, vx);
-#pragma unroll
-        for (int h = 0; h < kLaneGroup; h++) acc[q] += vx[h] * wx[h];
-      }
-#pragma unroll
-    for (int h = 0; h < kLaneGroup; h++) acc[8] += wx[h] * wx[h];
+// Rows of the reduced values in the dots buffer (B conditions each): the dot
+// products of the first Gram-Schmidt pass from row 0 and of the second from row
+// kDots2, product q at 9*(q/8) + q%8 with ||w||^2 at row 8 of each; ||w||^2
+// after the update the step ends with, and after its first pass.
+constexpr int kDots2 = 48, kDotNorm = 40, kDotNorm1 = 41, kDotRows = 96;
+__host__ __device__ constexpr int dot_row(int q) { return 9 * (q / 8) + q % 8; }
+
+// DGKS: condition b takes a second pass when the first left less than eta of
+// ||w||.  The kernels of that pass look this up themselves (Gate), so the host
+// queues them without waiting for the norms; with no condition in need every
+// block returns at once.
+struct Gate {
+  double eta = 0.0;              // 0: not a second pass
+  const double *dots = nullptr;
+  __device__ __forceinline__ bool second(int b, int B) const {
+    return sqrt(dots[kDotNorm1 * B + b]) < eta * sqrt(dots[8 * B + b]);
   }
-  for (int q = 0; q < cnt; q++) S[((size_t)q * B + b) * L + l] = acc[q];
-  S[((size_t)cnt * B + b) * L + l] = acc[8];
+  // every thread of the block must call it
+  __device__ __forceinline__ bool closed(int B) const {
+    return eta > 0.0 && !__syncthreads_or((int)threadIdx.x < B && second(threadIdx.x, B));
+  }
+};
+
+// Level 1 of the lane sums adds lanes x*1024 + t + 256k, k = 0..3 in order, for
+// each t < 256, then the 64 values of each wave by the shuffle tree: four
+// partial sums per group of 1024 lanes, which level 2 adds in order.  One
+// condition's kernels give a block of 256 threads the lanes of one partial sum:
+// block 4x + v, thread 64k + t takes lane x*1024 + 256k + 64v + t, so the block
+// reduces them itself (grid: at least 4 blocks; lanes past L count zero).
+__device__ __forceinline__ int lane_of(int blk, int t) {
+  return (blk >> 2) * 1024 + (t >> 6) * 256 + (blk & 3) * 64 + (t & 63);
+}
+// thread t's sum of a block's lane values in LDS ([k][64])
+__device__ __forceinline__ double lanes4(const double *sm, int t) {
+  double s = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) s += sm[k * 64 + t];
+  return s;
 }
 
-// level 1 of the lane sums: block (x, qb) adds lanes x*1024 + t + 256k of row
-// qb (k = 0..3 in order, thread t), then a fixed tree over the block.  With
-// one block per row (L <= 1024) the result is final and goes to
-// out[q'*out_stride_q + b] (qb = q*B + b; q' = 8 for q = qnorm, else q);
-// otherwise to S2[qb*G + x] for level 2.
-__global__ __launch_bounds__(256) void k_sum_lanes1(const double *__restrict__ S, int L, double *__restrict__ dst,
-                                                    int out_stride_q, int qnorm, int lgB) {
-  const int x = blockIdx.x, qb = blockIdx.y, G = gridDim.x, B = 1 << lgB;
+// the lane group at element e for VB neighbouring conditions b .. b+VB-1
+// (x[h][k], zeros past n1), loaded without a branch so that the loads of
+// several vectors and groups are in flight together: addresses past n1 are
+// clamped (B > 1) or lie in the vector's padding (B = 1)
+template <typename TV, int VB>
+__device__ __forceinline__ void ld_lanes(const TV *__restrict__ v, size_t e, size_t n1, int lgB, int b,
+                                         double x[kLaneGroup][VB]) {
+  if constexpr (VB == 1) {
+    if (lgB == 0) {
+      TV r[kLaneGroup];
+      if constexpr (sizeof(TV) == 8) {
+        const double2 p = *reinterpret_cast<const double2 *>(v + e), q = *reinterpret_cast<const double2 *>(v + e + 2);
+        r[0] = p.x; r[1] = p.y; r[2] = q.x; r[3] = q.y;
+      } else {
+        const float4 p = *reinterpret_cast<const float4 *>(v + e);
+        r[0] = p.x; r[1] = p.y; r[2] = p.z; r[3] = p.w;
+      }
+#pragma unroll
+      for (int h = 0; h < kLaneGroup; h++) x[h][0] = e + h < n1 ? (double)r[h] : 0.0;
+    } else {
+#pragma unroll
+      for (int h = 0; h < kLaneGroup; h++) {
+        const size_t at = e + h < n1 ? e + h : n1 - 1;
+        const double t = (double)v[(at << lgB) + b];
+        x[h][0] = e + h < n1 ? t : 0.0;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int h = 0; h < kLaneGroup; h++) {
+      const size_t at = e + h < n1 ? e + h : n1 - 1;
+      double t[4];
+      const TV *src = v + (at << lgB) + b;
+      if constexpr (sizeof(TV) == 8) {
+        const double2 p = *reinterpret_cast<const double2 *>(src), q = *reinterpret_cast<const double2 *>(src + 2);
+        t[0] = p.x; t[1] = p.y; t[2] = q.x; t[3] = q.y;
+      } else {
+        const float4 p = *reinterpret_cast<const float4 *>(src);
+        t[0] = p.x; t[1] = p.y; t[2] = p.z; t[3] = p.w;
+      }
+#pragma unroll
+      for (int k = 0; k < VB; k++) x[h][k] = e + h < n1 ? t[k] : 0.0;
+    }
+  }
+}
+
+// Dot products <V_q, w>, q < cnt, and ||w||^2 (row cnt) per lane, all chunks
+// of Q vectors in one launch (blockIdx.y; w is read once per chunk).  A thread
+// is one lane of VB neighbouring conditions (VB = 4 where the batch allows it:
+// 16-byte loads).  One condition: the block's lanes (lane_of) are summed here
+// as level 1 of the lane sums does, out is S2[row][G][4]; a batch stores the
+// lane sums S[row*B + b][L].
+// Bound by HBM on the 2M wing; on small meshes by the number of waves (L is
+// 4096 for 40k triangles: 64 waves), hence Q: with fewer vectors a thread there
+// are more blocks and the same vectors are in flight at once.  40k triangles,
+// FP64: 11 us a step, where chunks of 8 took 19 us and two sum launches each;
+// 83k tetrahedra 15 against 28 us a chunk; unchanged on the 2M wing.
+template <typename TV, int VB, int Q>
+__global__ __launch_bounds__(256) void k_mdot(const TV *__restrict__ V, size_t stride, int cnt,
+                                               const TV *__restrict__ w, size_t n1, int lgB, int L,
+                                               double *__restrict__ out, Gate gate) {
+  const int B = 1 << lgB, lgU = VB == 1 ? lgB : lgB - 2;
+  if (gate.closed(B)) return;
+  const size_t u = lgB == 0 ? (size_t)lane_of(blockIdx.x, threadIdx.x) : (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t l = u >> lgU;
+  const int b = (int)(u & (((size_t)1 << lgU) - 1)) * VB;
+  const int i0 = blockIdx.y * Q;
+  const TV *v[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++) v[q] = V + (size_t)(i0 + q < cnt ? i0 + q : (cnt > 0 ? cnt - 1 : 0)) * stride;
+  double acc[Q + 1][VB];
+#pragma unroll
+  for (int q = 0; q <= Q; q++)
+#pragma unroll
+    for (int k = 0; k < VB; k++) acc[q][k] = 0;
+  if (l < (size_t)L) {
+#pragma unroll Q == 1 ? 4 : (Q <= 3 ? 2 : 1)
+    for (size_t e = kLaneGroup * l; e < n1; e += (size_t)kLaneGroup * L) {
+      double wx[kLaneGroup][VB], vx[Q][kLaneGroup][VB];
+      ld_lanes<TV, VB>(w, e, n1, lgB, b, wx);
+#pragma unroll
+      for (int q = 0; q < Q; q++) ld_lanes<TV, VB>(v[q], e, n1, lgB, b, vx[q]);
+#pragma unroll
+      for (int q = 0; q < Q; q++)
+#pragma unroll
+        for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+          for (int k = 0; k < VB; k++) acc[q][k] += vx[q][h][k] * wx[h][k];
+#pragma unroll
+      for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+        for (int k = 0; k < VB; k++) acc[Q][k] += wx[h][k] * wx[h][k];
+    }
+  }
+  const int nq = min(Q, cnt - i0);
+  if (lgB == 0) {
+    if constexpr (VB == 1) {
+      __shared__ double sm[4][256];
+      const int g = threadIdx.x >> 6, t = threadIdx.x & 63;
+#pragma unroll
+      for (int r0 = 0; r0 <= Q; r0 += 4) {   // four rows at a time, a wave each
+        if (r0) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (r0 + r <= Q) sm[r][threadIdx.x] = acc[r0 + r <= Q ? r0 + r : 0][0];
+        __syncthreads();
+        const int q = r0 + g;   // Q: the norm, from the first chunk only
+        const int row = q < Q ? (q < nq ? i0 + q : -1) : (q == Q && blockIdx.y == 0 ? cnt : -1);
+        if (row < 0) continue;
+        const double s = wave_sum(lanes4(sm[g], t));
+        if (t == 0) out[(size_t)row * gridDim.x + blockIdx.x] = s;
+      }
+    }
+    return;
+  }
+  if (l >= (size_t)L) return;
+#pragma unroll
+  for (int q = 0; q <= Q; q++) {
+    const int row = q < Q ? (q < nq ? i0 + q : -1) : (blockIdx.y == 0 ? cnt : -1);
+    if (row < 0) continue;
+#pragma unroll
+    for (int k = 0; k < VB; k++) out[((size_t)row * B + b + k) * L + l] = acc[q][k];
+  }
+}
+
+// level 1 of the lane sums of row qb, groups x, from stored lane sums
+__global__ __launch_bounds__(256) void k_sum_lanes1(const double *__restrict__ S, int L, double *__restrict__ S2) {
+  const int x = blockIdx.x, qb = blockIdx.y, G = gridDim.x;
   double s = 0;
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     const int l = x * 1024 + k * 256 + (int)threadIdx.x;
     if (l < L) s += S[(size_t)qb * L + l];
   }
-  __shared__ double sh[4];
   s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  const double r = sh[0] + sh[1] + sh[2] + sh[3];
-  if (G > 1) {
-    dst[(size_t)qb * G + x] = r;
-  } else {
-    const int q = qb >> lgB, qo = q == qnorm ? 8 : q;
-    dst[(size_t)qo * out_stride_q + (qb & (B - 1))] = r;
-  }
+  if ((threadIdx.x & 63) == 0) S2[((size_t)qb * G + x) * 4 + (threadIdx.x >> 6)] = s;
 }
 
-// level 2: out row qb = sum of its G level-1 sums, thread t adding t, t + 256,
-// ... in order, then a fixed tree (same output mapping as level 1)
-__global__ __launch_bounds__(256) void k_sum_lanes(const double *__restrict__ S, int L, double *__restrict__ out,
-                                                   int out_stride_q, int qnorm, int lgB) {
-  const int qb = blockIdx.x, B = 1 << lgB;
+// group x's four level-1 sums of a row
+__device__ __forceinline__ double group_sum(const double *__restrict__ row, int x) {
+  const double *p = row + (size_t)x * 4;
+  return p[0] + p[1] + p[2] + p[3];
+}
+
+// where the sum of row qb = q*B + b goes: the dots layout when qnorm >= 0
+// (row qnorm is ||w||^2), else row q
+__device__ __forceinline__ size_t sum_at(int qb, int qnorm, int lgB) {
+  const int q = qb >> lgB, qo = qnorm < 0 ? q : (q == qnorm ? 8 : dot_row(q));
+  return ((size_t)qo << lgB) + (qb & ((1 << lgB) - 1));
+}
+
+// level 2: row qb = sum of its G level-1 sums, thread t adding t, t + 256, ...
+// in order, then a fixed tree.  A closed gate passes the value at keep on.
+__global__ __launch_bounds__(256) void k_sum_lanes(const double *__restrict__ S2, int G, double *__restrict__ out,
+                                                   int qnorm, int lgB, Gate gate, const double *__restrict__ keep) {
+  const int qb = blockIdx.x;
+  if (gate.closed(1 << lgB)) {
+    if (keep && threadIdx.x == 0) out[sum_at(qb, qnorm, lgB)] = keep[qb];
+    return;
+  }
   double s = 0;
-  for (int l = threadIdx.x; l < L; l += 256) s += S[(size_t)qb * L + l];
+  for (int l = threadIdx.x; l < G; l += 256) s += group_sum(S2 + (size_t)qb * G * 4, l);
   __shared__ double sh[4];
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const int q = qb >> lgB, qo = q == qnorm ? 8 : q;
-    out[(size_t)qo * out_stride_q + (qb & (B - 1))] = sh[0] + sh[1] + sh[2] + sh[3];
-  }
+  if (threadIdx.x == 0) out[sum_at(qb, qnorm, lgB)] = sh[0] + sh[1] + sh[2] + sh[3];
 }
 
-// w -= sum_q h_q V_q per condition (h_q of condition b at h[(9*(q/8) + q%8)*B + b],
-// the multidot's layout) and ||w||^2 per lane into S[b*L + l]
-template <typename TV>
-__global__ __launch_bounds__(256) void k_orth_update(const TV *__restrict__ V, size_t stride, int cnt,
-                                                     const double *__restrict__ h, TV *__restrict__ w, size_t n1,
-                                                     int lgB, int L, double *__restrict__ S) {
-  const int B = 1 << lgB;
-  __shared__ double hs[32 * 64];
-  for (int q = threadIdx.x; q < cnt * B; q += blockDim.x) {
-    const int qq = q >> lgB, b = q & (B - 1);
-    hs[q] = h[(size_t)(9 * (qq >> 3) + (qq & 7)) * B + b];
+// both levels in one launch, a block per row, for G <= kRowGroups groups (the
+// sums are those of the two launches)
+constexpr int kRowGroups = 16;
+__global__ __launch_bounds__(1024) void k_sum_rows(const double *__restrict__ S, int L, double *__restrict__ out,
+                                                   int qnorm, int lgB, Gate gate, const double *__restrict__ keep) {
+  const int qb = blockIdx.x, G = (L + 1023) / 1024;
+  if (gate.closed(1 << lgB)) {
+    if (keep && threadIdx.x == 0) out[sum_at(qb, qnorm, lgB)] = keep[qb];
+    return;
+  }
+  __shared__ double sh[kRowGroups][4];
+  const int t = threadIdx.x & 255;
+#pragma unroll
+  for (int x0 = 0; x0 < kRowGroups; x0 += 4) {
+    if (x0 >= G) break;
+    const int x = x0 + (threadIdx.x >> 8);
+    double s = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int l = x * 1024 + k * 256 + t;
+      if (l < L) s += S[(size_t)qb * L + l];
+    }
+    s = wave_sum(s);
+    if ((t & 63) == 0) sh[x][t >> 6] = s;
   }
   __syncthreads();
-  const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ((size_t)L << lgB)) return;
-  const size_t l = g >> lgB;
-  const int b = (int)(g & (B - 1));
-  double nrm = 0;
-  for (size_t e = kLaneGroup * l; e < n1; e += (size_t)kLaneGroup * L) {
-    double wx[kLaneGroup];
-    ld_group(w, e, n1, lgB, b, wx);
-    int q = 0;
-    for (; q + 4 <= cnt; q += 4) {   // four vectors' loads in flight at once
-      double vx[4][kLaneGroup];
-#pragma unroll
-      for (int u = 0; u < 4; u++) ld_group(V + (size_t)(q + u) * stride, e, n1, lgB, b, vx[u]);
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const double hq = hs[((q + u) << lgB) + b];
-#pragma unroll
-        for (int k = 0; k < kLaneGroup; k++) wx[k] -= hq * vx[u][k];
+  if (threadIdx.x >= 64) return;
+  const double s = wave_sum((int)threadIdx.x < G ? group_sum(sh[0], threadIdx.x) : 0.0);
+  if (threadIdx.x == 0) out[sum_at(qb, qnorm, lgB)] = s;
+}
+
+// h of a Gram-Schmidt pass into hs[cnt][B].  With S2 (one condition, G <= 64)
+// every block does level 2 of the lane sums and block 0 writes it to dots;
+// without it h comes from dots.  In a second pass the conditions that need none
+// use h = 0.  A barrier must follow.
+__device__ __forceinline__ void orth_h(const double *__restrict__ S2, int G, double *dots, int cnt, int B,
+                                       const Gate &gate, double *hs) {
+  if (S2) {
+    const int lane = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q <= cnt; q += 4) {
+      const double s = wave_sum(lane < G ? group_sum(S2 + (size_t)q * G * 4, lane) : 0.0);
+      if (lane == 0) {
+        if (q < cnt) hs[q] = s;
+        if (blockIdx.x == 0) dots[q == cnt ? 8 : dot_row(q)] = s;
       }
     }
-    for (; q < cnt; q++) {
-      double vx[kLaneGroup];
-      ld_group(V + (size_t)q * stride, e, n1, lgB, b, vx);
-      const double hq = hs[(q << lgB) + b];
-#pragma unroll
-      for (int k = 0; k < kLaneGroup; k++) wx[k] -= hq * vx[k];
+  } else {
+    for (int q = threadIdx.x; q < cnt * B; q += blockDim.x) {
+      const int qq = q / B, b = q - qq * B;
+      const double h = dots[(size_t)dot_row(qq) * B + b];
+      hs[q] = gate.eta > 0.0 && !gate.second(b, B) ? 0.0 : h;
     }
-    TV r[kLaneGroup];
-#pragma unroll
-    for (int k = 0; k < kLaneGroup; k++) r[k] = (TV)wx[k];
-    st_group(w, e, n1, lgB, b, r);
-#pragma unroll
-    for (int k = 0; k < kLaneGroup; k++) nrm += (double)r[k] * (double)r[k];
   }
-  S[(size_t)b * L + l] = nrm;
+}
+
+// wx -= sum_q h_q V_q for one lane group of VB conditions, NU vectors' loads in
+// flight at once
+template <typename TV, int VB, int NU>
+__device__ __forceinline__ void orth_group(const TV *__restrict__ V, size_t stride, int cnt, const double *hs,
+                                           size_t e, size_t n1, int lgB, int b, double wx[kLaneGroup][VB]) {
+  auto sub = [&](auto nu, int q) {
+    constexpr int M = decltype(nu)::value;
+    double vx[M][kLaneGroup][VB];
+#pragma unroll
+    for (int i = 0; i < M; i++) ld_lanes<TV, VB>(V + (size_t)(q + i) * stride, e, n1, lgB, b, vx[i]);
+#pragma unroll
+    for (int i = 0; i < M; i++)
+#pragma unroll
+      for (int k = 0; k < VB; k++) {
+        const double hq = hs[((q + i) << lgB) + b + k];
+#pragma unroll
+        for (int h = 0; h < kLaneGroup; h++) wx[h][k] -= hq * vx[i][h][k];
+      }
+  };
+  int q = 0;
+  for (; q + NU <= cnt; q += NU) sub(std::integral_constant<int, NU>{}, q);
+  if constexpr (NU > 4)
+    if (q + 4 <= cnt) { sub(std::integral_constant<int, 4>{}, q); q += 4; }
+  if constexpr (NU > 2)
+    if (q + 2 <= cnt) { sub(std::integral_constant<int, 2>{}, q); q += 2; }
+  if (q < cnt) sub(std::integral_constant<int, 1>{}, q);
+}
+
+// the updated group stored, its squares (of the stored values) in r2
+template <typename TV, int VB>
+__device__ __forceinline__ void st_lanes(TV *__restrict__ w, size_t e, size_t n1, int lgB, int b,
+                                         const double wx[kLaneGroup][VB], double r2[kLaneGroup][VB]) {
+  TV r[kLaneGroup][VB];
+#pragma unroll
+  for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+    for (int k = 0; k < VB; k++) {
+      r[h][k] = (TV)wx[h][k];
+      r2[h][k] = (double)r[h][k] * (double)r[h][k];
+    }
+  if constexpr (VB == 1) {
+    TV t[kLaneGroup];
+#pragma unroll
+    for (int h = 0; h < kLaneGroup; h++) t[h] = r[h][0];
+    st_group(w, e, n1, lgB, b, t);
+  } else {
+#pragma unroll
+    for (int h = 0; h < kLaneGroup; h++)
+      if (e + h < n1) {
+        TV *dst = w + ((e + h) << lgB) + b;
+        if constexpr (sizeof(TV) == 8) {
+          reinterpret_cast<double2 *>(dst)[0] = make_double2(r[h][0], r[h][1]);
+          reinterpret_cast<double2 *>(dst)[1] = make_double2(r[h][2], r[h][3]);
+        } else {
+          *reinterpret_cast<float4 *>(dst) = make_float4(r[h][0], r[h][1], r[h][2], r[h][3]);
+        }
+      }
+  }
+}
+
+// w -= sum_q h_q V_q per condition and ||w||^2: one condition's level-1 sums
+// S2n[G][4], a batch's lane sums S[b][L].  A block is 256 lanes (VB conditions)
+// times SL slots; slot s takes the lane's groups s, s + SL, ..., and with SL > 1
+// their squares go through LDS, where the lane's first thread adds them in order.
+// Bound by HBM on the 2M wing (232 us, 5.2 TB/s), where SL = 1; with 2^16 lanes
+// one slot is one wave per SIMD, which waits for memory: 486k tetrahedra, FP32,
+// 54 us a call with one, 34 (4.6 TB/s) with four.
+template <typename TV, int VB, int SL>
+__global__ __launch_bounds__(256 * SL) void k_orth_lanes(const TV *__restrict__ V, size_t stride, int cnt,
+                                                         const double *__restrict__ S2, int G, double *dots,
+                                                         TV *__restrict__ w, size_t n1, int lgB, int L,
+                                                         double *__restrict__ S, Gate gate) {
+  const int B = 1 << lgB, lgU = VB == 1 ? lgB : lgB - 2;
+  if (gate.closed(B)) return;
+  extern __shared__ double hs[];   // [cnt][B]
+  __shared__ double sq[SL > 1 ? kLaneGroup * VB : 1][256 * SL];
+  orth_h(S2, G, dots, cnt, B, gate, hs);
+  __syncthreads();
+  const int t = threadIdx.x & 255, sl = threadIdx.x >> 8;
+  const size_t u = lgB == 0 ? (size_t)lane_of(blockIdx.x, t) : (size_t)blockIdx.x * 256 + t;
+  const size_t l = u >> lgU;
+  const int b = (int)(u & (((size_t)1 << lgU) - 1)) * VB;
+  const bool lane_ok = l < (size_t)L;
+  double nrm[VB];
+#pragma unroll
+  for (int k = 0; k < VB; k++) nrm[k] = 0;
+  for (size_t g0 = 0; g0 * L * kLaneGroup < n1; g0 += SL) {
+    const size_t e = kLaneGroup * (l + (size_t)L * (g0 + sl));
+    double r2[kLaneGroup][VB];
+#pragma unroll
+    for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+      for (int k = 0; k < VB; k++) r2[h][k] = 0;
+    if (lane_ok && e < n1) {
+      double wx[kLaneGroup][VB];
+      ld_lanes<TV, VB>(w, e, n1, lgB, b, wx);
+      orth_group<TV, VB, VB == 1 ? 4 : 2>(V, stride, cnt, hs, e, n1, lgB, b, wx);
+      st_lanes<TV, VB>(w, e, n1, lgB, b, wx, r2);
+    }
+    if constexpr (SL == 1) {
+#pragma unroll
+      for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+        for (int k = 0; k < VB; k++) nrm[k] += r2[h][k];
+    } else {
+      if (g0) __syncthreads();
+#pragma unroll
+      for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+        for (int k = 0; k < VB; k++) sq[h * VB + k][threadIdx.x] = r2[h][k];
+      __syncthreads();
+      if (sl == 0)
+#pragma unroll
+        for (int i = 0; i < SL; i++)
+#pragma unroll
+          for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+            for (int k = 0; k < VB; k++) nrm[k] += sq[h * VB + k][i * 256 + t];
+    }
+  }
+  if (lgB == 0) {
+    if constexpr (VB == 1) {
+      __shared__ double sm[256];
+      if (sl == 0) sm[t] = nrm[0];
+      __syncthreads();
+      if (threadIdx.x < 64) {
+        const double s = wave_sum(lanes4(sm, threadIdx.x));
+        if (threadIdx.x == 0) S[blockIdx.x] = s;
+      }
+    }
+  } else if (sl == 0 && lane_ok) {
+#pragma unroll
+    for (int k = 0; k < VB; k++) S[(size_t)(b + k) * L + l] = nrm[k];
+  }
+}
+
+// The same for few lanes, a thread per lane group: the kOrthSlots groups of a
+// lane sit in one block, their squares go through LDS and are added in the
+// lane's order; lane sums into S[b][L].  With a thread per lane small meshes
+// ran on a few waves, each waiting for memory once per four vectors and group
+// (40k triangles, 64 waves: 21 us a call, now 10; 83k tetrahedra 35, now 14).
+constexpr int kOrthSlots = 16;
+template <typename TV, int VB>
+__global__ __launch_bounds__(256) void k_orth_slots(const TV *__restrict__ V, size_t stride, int cnt,
+                                                    const double *__restrict__ S2, int G, double *dots,
+                                                    TV *__restrict__ w, size_t n1, int lgB, int L,
+                                                    double *__restrict__ S, Gate gate) {
+  const int B = 1 << lgB, lgU = VB == 1 ? lgB : lgB - 2;
+  if (gate.closed(B)) return;
+  extern __shared__ double hs[];   // [cnt][B]
+  __shared__ double sq[VB][kLaneGroup][256];
+  orth_h(S2, G, dots, cnt, B, gate, hs);
+  __syncthreads();
+  const int p = threadIdx.x & 15, sl = threadIdx.x >> 4;
+  const size_t u = (size_t)blockIdx.x * 16 + p, l = u >> lgU;
+  const int b = (int)(u & (((size_t)1 << lgU) - 1)) * VB;
+  const bool lane_ok = l < (size_t)L;
+  double nrm = 0;
+  for (size_t g0 = 0; g0 * L * kLaneGroup < n1; g0 += kOrthSlots) {
+    const size_t e = kLaneGroup * (l + (size_t)L * (g0 + sl));
+    double r2[kLaneGroup][VB];
+#pragma unroll
+    for (int h = 0; h < kLaneGroup; h++)
+#pragma unroll
+      for (int k = 0; k < VB; k++) r2[h][k] = 0;
+    if (lane_ok && e < n1) {
+      double wx[kLaneGroup][VB];
+      ld_lanes<TV, VB>(w, e, n1, lgB, b, wx);
+      orth_group<TV, VB, VB == 1 ? 8 : 2>(V, stride, cnt, hs, e, n1, lgB, b, wx);
+      st_lanes<TV, VB>(w, e, n1, lgB, b, wx, r2);
+    }
+    if (g0) __syncthreads();
+#pragma unroll
+    for (int k = 0; k < VB; k++)
+#pragma unroll
+      for (int h = 0; h < kLaneGroup; h++) sq[k][h][threadIdx.x] = r2[h][k];
+    __syncthreads();
+    if ((int)threadIdx.x < 16 * VB)   // thread (k, lane p): the lane's squares in order
+      for (int i = 0; i < kOrthSlots; i++)
+#pragma unroll
+        for (int h = 0; h < kLaneGroup; h++) nrm += sq[threadIdx.x >> 4][h][i * 16 + p];
+  }
+  if ((int)threadIdx.x < 16 * VB && lane_ok) S[(size_t)(b + (threadIdx.x >> 4)) * L + l] = nrm;
 }
 
 // r = b - y (b FP64) and ||r||^2 per lane into S[b*L + l]
@@ -841,16 +1163,28 @@ __device__ __forceinline__ void st4(T *p, const double x[4]) {
   }
 }
 
-// w = w / sqrt(n2[b]) per condition when n2[b] > 0 (the norm read on the
-// device, so the launch need not wait for the host)
+// w = w / sqrt(||w||^2) per condition when that is > 0, the norm (row kDotNorm
+// of dots) read on the device, so the launch need not wait for the host.  Block 0
+// hands the host the first ndots values of dots (a copy of its own took 2.7 us
+// a step and its gap).  (Summing the lane norms here too, by every block, took
+// 8.6 us where the sum and this take 7.3: 40k triangles.)
 template <typename TV>
-__global__ void k_scale_norm(TV *__restrict__ w, const double *__restrict__ n2, size_t n, int lgB) {
+__global__ __launch_bounds__(256) void k_scale_norm(TV *__restrict__ w, const double *__restrict__ dots,
+                                                    double *__restrict__ hdots, int ndots, size_t n, int lgB) {
   const size_t B = (size_t)1 << lgB, tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x,
                nt = (size_t)gridDim.x * blockDim.x, ng = n / 4;
+  const double *n2 = dots + kDotNorm * B;
+  if (blockIdx.x == 0)
+    for (int q = threadIdx.x; q < ndots; q += blockDim.x) hdots[q] = dots[q];
   double a[4];
   bool on[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) {
+    if (t > 0 && lgB == 0) {   // one condition: one reciprocal
+      a[t] = a[0];
+      on[t] = on[0];
+      continue;
+    }
     const double s2 = n2[(4 * tid + t) & (B - 1)];
     on[t] = s2 > 0;
     a[t] = on[t] ? 1.0 / sqrt(s2) : 1.0;
@@ -1189,10 +1523,13 @@ static int impl_alloc(bes_ctx *c, Impl *im) {
   BES_HIP(hipMalloc(&im->V, (size_t)std::max(im->restart + 1, 7) * im->vstride * es));
   BES_HIP(hipMalloc(&im->Z, 3 * im->vstride * es));
   BES_HIP(hipMalloc((void **)&im->part, 32 * kRedBlocks * sizeof(double)));
-  BES_HIP(hipMalloc((void **)&im->S, (size_t)9 * Bs * im->lanes * sizeof(double)));
-  BES_HIP(hipMalloc((void **)&im->S2, (size_t)9 * Bs * ((im->lanes + 1023) / 1024) * sizeof(double)));
-  BES_HIP(hipMalloc((void **)&im->dots, 64 * Bs * sizeof(double)));
-  BES_HIP(hipHostMalloc((void **)&im->hdots, 64 * Bs * sizeof(double), hipHostMallocDefault));
+  // lane sums: one condition keeps only a norm's, the dot products are summed
+  // to S2 in their kernel; a batch keeps those of every product of a step
+  const size_t nrow = (size_t)im->restart + 2;
+  BES_HIP(hipMalloc((void **)&im->S, (c->B == 1 ? 1 : nrow * Bs) * im->lanes * sizeof(double)));
+  BES_HIP(hipMalloc((void **)&im->S2, nrow * Bs * ((im->lanes + 1023) / 1024) * 4 * sizeof(double)));
+  BES_HIP(hipMalloc((void **)&im->dots, kDotRows * Bs * sizeof(double)));
+  BES_HIP(hipHostMalloc((void **)&im->hdots, kDotRows * Bs * sizeof(double), hipHostMallocDefault));
   BES_HIP(hipEventCreateWithFlags(&im->ev_dots, hipEventDisableTiming));
   BES_HIP(hipMalloc((void **)&im->bits, (size_t)kLinfSlots * 16 * Bs * sizeof(unsigned long long)));
   return BES_OK;
@@ -1391,35 +1728,117 @@ static int spmv(bes_ctx *c, Impl *im, const TV *x, TV *y) {
   return BES_OK;
 }
 
-// the lane sums of rows qb = q*B + b < nqb of S (L lanes each) into
-// out[q'*out_stride_q + b], q' = 8 for q = qnorm, else q: level 1 over groups
-// of 1024 lanes, then level 2 over the groups (skipped for L <= 1024)
-static void sum_lanes(bes_ctx *c, Impl *im, const double *S, int nqb, double *out, int out_stride_q, int qnorm) {
+// the lane sums S of nqb rows (q*B + b) into out (see sum_at): one launch for
+// up to kRowGroups groups of 1024 lanes, else two levels
+static void sum_lanes(bes_ctx *c, Impl *im, int nqb, double *out, int qnorm, Gate gate = Gate(),
+                      const double *keep = nullptr) {
   const int L = im->lanes, G = (L + 1023) / 1024;
-  if (G == 1) {
-    hipLaunchKernelGGL(k_sum_lanes1, dim3(1, nqb), dim3(256), 0, c->stream, S, L, out, out_stride_q, qnorm, c->lgB);
+  if (G <= kRowGroups) {
+    hipLaunchKernelGGL(k_sum_rows, dim3(nqb), dim3(1024), 0, c->stream, im->S, L, out, qnorm, c->lgB, gate, keep);
   } else {
-    hipLaunchKernelGGL(k_sum_lanes1, dim3(G, nqb), dim3(256), 0, c->stream, S, L, im->S2, out_stride_q, qnorm,
-                       c->lgB);
-    hipLaunchKernelGGL(k_sum_lanes, dim3(nqb), dim3(256), 0, c->stream, im->S2, G, out, out_stride_q, qnorm, c->lgB);
+    hipLaunchKernelGGL(k_sum_lanes1, dim3(G, nqb), dim3(256), 0, c->stream, im->S, L, im->S2);
+    hipLaunchKernelGGL(k_sum_lanes, dim3(nqb), dim3(256), 0, c->stream, im->S2, G, out, qnorm, c->lgB, gate, keep);
   }
 }
 
-// dots h_q = V_q^T w (q < cnt) and ||w||^2 of every condition: chunk ch of up to
-// 8 vectors reduces into dots[(9*ch + q)*B + b], its ||w||^2 into
-// dots[(9*ch + 8)*B + b] (the deterministic lane reductions)
+// dots h_q = V_q^T w (q < cnt) and ||w||^2 of every condition, reduced to row
+// at of the dots buffer (the deterministic lane reductions).  With defer, one
+// condition's last level may be left to k_orth_update: returns its S2 through
+// *S2 (null: the dots are done).
 template <typename TV>
-static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, const TV *w) {
-  const int B = c->B, lgB = c->lgB, L = im->lanes;
+static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, const TV *w, int at = 0,
+                    Gate gate = Gate(), const double **S2 = nullptr) {
+  const int B = c->B, lgB = c->lgB, L = im->lanes, G = (L + 1023) / 1024;
   const size_t n1 = (size_t)c->N * c->nv;
-  const int nchunk = std::max(1, (cnt + 7) / 8);
-  if (nchunk > 4) { set_error("too many basis vectors"); return BES_ERR_ARG; }
-  ProfScope ps(c, kProfKrylov, (double)(cnt + nchunk) * n1 * B * sizeof(TV));
-  const int nt = L * B, nb = grid_for(nt, 256);
-  for (int q = 0; q < nchunk; q++) {
-    const int i0 = q * 8, cc = std::max(0, std::min(8, cnt - i0));
-    hipLaunchKernelGGL((k_mdot<TV>), dim3(nb), dim3(256), 0, c->stream, V, stride, i0, cc, w, n1, lgB, L, im->S);
-    sum_lanes(c, im, im->S, (cc + 1) * B, im->dots + (size_t)9 * q * B, B, cc);
+  if (S2) *S2 = nullptr;
+  if (cnt > im->restart + 1) { set_error("too many basis vectors"); return BES_ERR_ARG; }
+  const bool quad = lgB >= 2;
+  // vectors per thread: as many as leave about four waves on every SIMD
+  const size_t units = (size_t)L * (quad ? B / 4 : B);
+  int qmax = quad ? 2 : 8;
+  while (qmax > 1 && units * ((cnt + qmax - 1) / qmax) < 262144) qmax /= 2;
+  const int ny = std::max(1, (cnt + qmax - 1) / qmax), Q = std::max(1, (cnt + ny - 1) / ny);
+  ProfScope ps(c, kProfKrylov, (double)(cnt + ny) * n1 * B * sizeof(TV));
+  double *out = B == 1 ? im->S2 : im->S;
+  const int bs = 256;
+  const dim3 grid(B == 1 ? 4 * G : (unsigned)((units + bs - 1) / bs), ny);
+  auto go = [&](auto vb, auto q) {
+    hipLaunchKernelGGL((k_mdot<TV, decltype(vb)::value, decltype(q)::value>), grid, dim3(bs), 0, c->stream, V, stride,
+                       cnt, w, n1, lgB, L, out, gate);
+  };
+  using std::integral_constant;
+  if (quad) {
+    if (Q == 1) go(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+    else go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+  } else {
+    const integral_constant<int, 1> one;
+    switch (Q) {
+      case 1: go(one, integral_constant<int, 1>{}); break;
+      case 2: go(one, integral_constant<int, 2>{}); break;
+      case 3: go(one, integral_constant<int, 3>{}); break;
+      case 4: go(one, integral_constant<int, 4>{}); break;
+      case 5: go(one, integral_constant<int, 5>{}); break;
+      case 6: go(one, integral_constant<int, 6>{}); break;
+      case 7: go(one, integral_constant<int, 7>{}); break;
+      default: go(one, integral_constant<int, 8>{}); break;
+    }
+  }
+  double *d = im->dots + (size_t)at * B;
+  if (B > 1) sum_lanes(c, im, (cnt + 1) * B, d, cnt, gate);
+  else if (S2 && G <= 64) *S2 = im->S2;
+  else hipLaunchKernelGGL(k_sum_lanes, dim3(cnt + 1), dim3(256), 0, c->stream, im->S2, G, d, cnt, 0, gate, nullptr);
+  BES_HIP(hipGetLastError());
+  return BES_OK;
+}
+
+// Up to this many lanes (times conditions over the kernel's VB) the update runs
+// a thread per lane group: past it a thread per lane gives at least a wave for
+// every other SIMD, and the sixteenfold blocks with their barrier cost more (486k
+// tetrahedra, 2^16 lanes, FP32: 79 us against 34; the 2M wing 371 against 232).
+constexpr size_t kSlotUnits = 16384;
+
+// one Gram-Schmidt pass of w against V_0 .. V_(cnt-1): dots into row at, w
+// updated, its ||w||^2 into row nat (a closed gate copies row kDotNorm1 there)
+template <typename TV>
+static int orthogonalise(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, TV *w, int at, int nat,
+                         Gate gate = Gate()) {
+  const int B = c->B, lgB = c->lgB, L = im->lanes, G = (L + 1023) / 1024;
+  const size_t n1 = (size_t)c->N * c->nv;
+  const double *S2 = nullptr;
+  int s = multidot<TV>(c, im, V, stride, cnt, w, at, gate, &S2);
+  if (s) return s;
+  ProfScope ps(c, kProfKrylov, (double)(cnt + 2) * n1 * B * sizeof(TV));
+  double *d = im->dots + (size_t)at * B;
+  const size_t units = (size_t)L * (lgB >= 2 ? B / 4 : B), lds = (size_t)cnt * B * sizeof(double);
+  double *out = im->dots + (size_t)nat * B;
+  const double *keep = im->dots + (size_t)kDotNorm1 * B;
+  if (units <= kSlotUnits) {
+    const dim3 grid((unsigned)((units + 15) / 16));
+    if (lgB >= 2)
+      hipLaunchKernelGGL((k_orth_slots<TV, 4>), grid, dim3(256), lds, c->stream, V, stride, cnt, S2, G, d, w, n1, lgB,
+                         L, im->S, gate);
+    else
+      hipLaunchKernelGGL((k_orth_slots<TV, 1>), grid, dim3(256), lds, c->stream, V, stride, cnt, S2, G, d, w, n1, lgB,
+                         L, im->S, gate);
+    sum_lanes(c, im, B, out, -1, gate, keep);
+  } else if (B == 1) {   // level 1 in the kernel (S2 may still be read: the sums go to S)
+    auto go = [&](auto sl) {
+      constexpr int SL = decltype(sl)::value;
+      hipLaunchKernelGGL((k_orth_lanes<TV, 1, SL>), dim3(4 * G), dim3(256 * SL), lds, c->stream, V, stride, cnt, S2, G,
+                         d, w, n1, lgB, L, im->S, gate);
+    };
+    if (L <= 65536) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 1>{});
+    hipLaunchKernelGGL(k_sum_lanes, dim3(1), dim3(256), 0, c->stream, im->S, G, out, -1, 0, gate, keep);
+  } else {
+    const dim3 grid((unsigned)((units + 255) / 256));
+    if (lgB >= 2)
+      hipLaunchKernelGGL((k_orth_lanes<TV, 4, 1>), grid, dim3(256), lds, c->stream, V, stride, cnt, S2, G, d, w, n1,
+                         lgB, L, im->S, gate);
+    else
+      hipLaunchKernelGGL((k_orth_lanes<TV, 1, 1>), grid, dim3(256), lds, c->stream, V, stride, cnt, S2, G, d, w, n1,
+                         lgB, L, im->S, gate);
+    sum_lanes(c, im, B, out, -1, gate, keep);
   }
   BES_HIP(hipGetLastError());
   return BES_OK;
@@ -1427,7 +1846,7 @@ static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, c
 
 // one lane-reduced norm per condition (S slot 0) into dots[at*B + b]
 static int sum_norms(bes_ctx *c, Impl *im, int at) {
-  sum_lanes(c, im, im->S, c->B, im->dots + (size_t)at * c->B, c->B, -1);
+  sum_lanes(c, im, c->B, im->dots + (size_t)at * c->B, -1);
   BES_HIP(hipGetLastError());
   return BES_OK;
 }
@@ -1466,7 +1885,9 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
   }
   hipMemsetAsync(xx, 0, n * sizeof(double), c->stream);
   const double *hd = im->hdots;
-  auto hdot = [&](int q, int b) { return hd[(size_t)(9 * (q / 8) + (q % 8)) * B + b]; };
+  const double eta = im->reorth_eta;
+  auto hdot = [&](int row, int q, int b) { return hd[(size_t)(row + dot_row(q)) * B + b]; };
+  const int scale_blocks = (int)std::min<size_t>(kRedBlocks, (n / 4 + 255) / 256 + 1);
   // ||b|| per condition
   hipLaunchKernelGGL((k_scale<double, TV>), dim3(kRedBlocks), dim3(256), 0, c->stream, bb, 1.0, Z, n);
   int s;
@@ -1531,81 +1952,40 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
         if ((s = spmv<TM, TV>(c, im, Z, w))) return s;
       }
       queued = false;
-      // classical Gram-Schmidt: the dots, the update and (without
-      // re-orthogonalisation) the normalisation are queued back to back and
-      // the host waits once, for h and ||w||
-      const bool dev_scale = !(im->reorth_eta > 0);
-      if ((s = multidot<TV>(c, im, V, vs, j + 1, w))) return s;
-      {
-        ProfScope ps(c, kProfKrylov, (double)(j + 3) * n * sizeof(TV));
-        hipLaunchKernelGGL((k_orth_update<TV>), dim3(nbl), dim3(256), 0, c->stream, V, vs, j + 1, im->dots, w, n1, lgB,
-                           L, im->S);
-        if ((s = sum_norms(c, im, 40))) return s;
+      // classical Gram-Schmidt: the dots, the update, with eta > 0 the second
+      // pass (its kernels look up which conditions need it) and the
+      // normalisation are queued back to back and the host waits once, for h
+      // and ||w||
+      if (eta > 0) {
+        if ((s = orthogonalise<TV>(c, im, V, vs, j + 1, w, 0, kDotNorm1))) return s;
+        Gate gate;
+        gate.eta = eta;
+        gate.dots = im->dots;
+        if ((s = orthogonalise<TV>(c, im, V, vs, j + 1, w, kDots2, kDotNorm, gate))) return s;
+      } else if ((s = orthogonalise<TV>(c, im, V, vs, j + 1, w, 0, kDotNorm))) {
+        return s;
       }
-      if (dev_scale)
-        hipLaunchKernelGGL((k_scale_norm<TV>), dim3(kRedBlocks), dim3(256), 0, c->stream, w, im->dots + (size_t)40 * B,
-                           n, lgB);
-      BES_HIP(hipMemcpyAsync(im->hdots, im->dots, (size_t)41 * B * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+      hipLaunchKernelGGL((k_scale_norm<TV>), dim3(scale_blocks), dim3(256), 0, c->stream, w, im->dots,
+                         im->hdots, (eta > 0 ? kDotRows : kDotNorm + 1) * B, n, lgB);
+      BES_HIP(hipGetLastError());
       BES_HIP(hipEventRecord(im->ev_dots, c->stream));
       // the next step's preconditioner and product need only the normalised w:
       // queue them before waiting, so the device works while the host reads h
       // and ||w|| (their results are discarded for conditions this step ends)
       bool more = false;
       for (int b = 0; b < B; b++) if (active[b] && total[b] + 1 < im->maxiter) more = true;
-      if (dev_scale && j + 1 < m && more) {
+      if (j + 1 < m && more) {
         if ((s = precond_apply<TM, TV>(c, im, w, Z, Z1))) return s;
         if ((s = spmv<TM, TV>(c, im, Z, V + (size_t)(j + 2) * vs))) return s;
         queued = true;
       }
       BES_HIP(hipEventSynchronize(im->ev_dots));
-      std::vector<double> wn2(B), w0n2(B);
-      for (int b = 0; b < B; b++) { w0n2[b] = hd[(size_t)8 * B + b]; wn2[b] = hd[(size_t)40 * B + b]; }
-      std::vector<double> hsave;
-      if (!dev_scale) {   // DGKS second pass for the conditions that need it (h2 = 0 for the rest: w unchanged)
-        bool any = false;
-        std::vector<char> re(B, 0);
-        for (int b = 0; b < B; b++)
-          if (active[b] && std::sqrt(wn2[b]) < im->reorth_eta * std::sqrt(w0n2[b])) { re[b] = 1; any = true; }
-        hsave.assign(hd, hd + (size_t)36 * B);
-        if (any) {
-          if ((s = multidot<TV>(c, im, V, vs, j + 1, w)) || (s = fetch_dots(c, im, (size_t)36 * B))) return s;
-          std::vector<double> h2(hd, hd + (size_t)36 * B);
-          for (int b = 0; b < B; b++)
-            for (int q = 0; q <= j; q++) {
-              const size_t at = (size_t)(9 * (q / 8) + (q % 8)) * B + b;
-              if (!re[b]) h2[at] = 0.0;
-            }
-          BES_HIP(hipMemcpyAsync(im->dots, h2.data(), h2.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-          for (int b = 0; b < B; b++)
-            if (re[b]) {
-              im->reorths++;
-              for (int q = 0; q <= j; q++) {
-                const size_t at = (size_t)(9 * (q / 8) + (q % 8)) * B + b;
-                hsave[at] += h2[at];
-              }
-            }
-          {
-            ProfScope ps(c, kProfKrylov, (double)(j + 3) * n * sizeof(TV));
-            hipLaunchKernelGGL((k_orth_update<TV>), dim3(nbl), dim3(256), 0, c->stream, V, vs, j + 1, im->dots, w, n1,
-                               lgB, L, im->S);
-            if ((s = sum_norms(c, im, 40))) return s;
-          }
-          BES_HIP(hipMemcpyAsync(im->hdots + (size_t)40 * B, im->dots + (size_t)40 * B, B * sizeof(double),
-                                 hipMemcpyDeviceToHost, c->stream));
-          BES_HIP(hipStreamSynchronize(c->stream));
-          for (int b = 0; b < B; b++) wn2[b] = hd[(size_t)40 * B + b];
-        }
-        for (int b = 0; b < B; b++) {
-          const double hn = std::sqrt(wn2[b]);
-          scl.c[b] = (active[b] && hn > 0) ? 1.0 / hn : 1.0;
-        }
-        hipLaunchKernelGGL((k_scale_b<TV, TV>), dim3(kRedBlocks), dim3(256), 0, c->stream, w, scl, w, n, lgB);
-      }
       for (int b = 0; b < B; b++) {
         if (!active[b]) continue;
-        for (int q = 0; q <= j; q++)
-          hcol[q] = dev_scale ? hdot(q, b) : hsave[(size_t)(9 * (q / 8) + (q % 8)) * B + b];
-        const double hn = std::sqrt(wn2[b]);
+        const double hn = std::sqrt(hd[(size_t)kDotNorm * B + b]);
+        const bool re = eta > 0 && std::sqrt(hd[(size_t)kDotNorm1 * B + b]) < eta * std::sqrt(hd[(size_t)8 * B + b]);
+        for (int q = 0; q <= j; q++) hcol[q] = re ? hdot(0, q, b) + hdot(kDots2, q, b) : hdot(0, q, b);
+        if (re) im->reorths++;
         hcol[j + 1] = hn;
         double *csb = &cs[(size_t)b * m], *snb = &sn[(size_t)b * m], *gb = &g[(size_t)b * (m + 1)];
         for (int q = 0; q < j; q++) {   // Givens rotations

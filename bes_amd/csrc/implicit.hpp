@@ -71,10 +71,10 @@ struct Impl {
   long extra_restarts = 0; // GMRES cycles whose Givens estimate met the target but the true residual did not
   double *part = nullptr;  // reduction partials [32][kRedBlocks] (BiCGStab)
   int lanes = 0;           // lanes L of the deterministic batched reductions
-  double *S = nullptr;     // their lane sums [9][B][L]
-  double *S2 = nullptr;    // level-1 sums of groups of 1024 lanes [9][B][L/1024]
-  double *dots = nullptr;  // [64][B] reduced dot products, condition fastest
-  double *hdots = nullptr; // [64][B] pinned host copy of dots (Arnoldi step)
+  double *S = nullptr;     // their lane sums: [L] (one condition), [restart + 2][B][L] (batch)
+  double *S2 = nullptr;    // level-1 sums of groups of 1024 lanes [restart + 2][B][L/1024]
+  double *dots = nullptr;  // [kDotRows][B] reduced dot products, condition fastest
+  double *hdots = nullptr; // [kDotRows][B] pinned host copy of dots (Arnoldi step)
   hipEvent_t ev_dots = nullptr;  // recorded after the copy into hdots
   unsigned long long *bits = nullptr;   // [2][8][B] Linf monitors of b and sum F*A, per variable and condition
   int ncolor = 0;
