@@ -336,25 +336,21 @@ __device__ __forceinline__ void face_state(const double *pk, const double *r, do
   }
 }
 
-// One thread per (face, condition), faces in device order: second-order states
-// of both sides from the cell packs, then the face flux per unit area
-// (FluxRoe.tpp:306-333, FluxFreestream.tpp:192-226, FluxSlipWall.tpp:32-53),
-// computed once per face and stored as a record of fs values (nv, padded to an
-// even count when B = 1 so the record moves in 16-byte pieces).  finf:
-// freestream primitive state per condition.
+// Flux per unit area of face f (owner o, neighbour j or a boundary code) for
+// condition b: second-order states of both sides from the cell packs, then
+// FluxRoe.tpp:306-333, FluxFreestream.tpp:192-226 or FluxSlipWall.tpp:32-53.
+// finf: freestream primitive state per condition.
 template <int ND, bool ONE>
-__device__ __forceinline__ void face_flux_thread(const double *__restrict__ PK, const DevMesh &dm, const GasConst &gc,
-                                                 const double *__restrict__ finf, double *__restrict__ FF, int fs,
-                                                 unsigned long long *__restrict__ err, int lgB, int t) {
+__device__ __forceinline__ void face_flux_value(const double *__restrict__ PK, const DevMesh &dm, const GasConst &gc,
+                                                const double *__restrict__ finf,
+                                                unsigned long long *__restrict__ err, int f, int o, int j, int b,
+                                                int B, double *out) {
   constexpr int NV = ND + 2;
-  const int F = dm.F, B = ONE ? 1 : 1 << lgB;
-  const int f = ONE ? t : t >> lgB, b = ONE ? 0 : t & (B - 1);
-  if (f >= F) return;
-  const int o = dm.fo[f], j = dm.fnb[f];
+  const int F = dm.F;
   // both sides' packs and the face geometry are requested before any of them
   // is used (a boundary face reads its owner's pack twice, from cache), so the
   // two gathers overlap instead of taking one memory round trip each
-  double nn[ND], rs[ND], rn[ND], ul[NV], out[NV + 1];
+  double nn[ND], rs[ND], rn[ND], ul[NV];
   double pko[(ND + 2) * (ND + 1)], pkn[(ND + 2) * (ND + 1)];
 #pragma unroll
   for (int d = 0; d < ND; d++) {
@@ -381,6 +377,21 @@ __device__ __forceinline__ void face_flux_thread(const double *__restrict__ PK, 
 #pragma unroll
   for (int v = 0; v < NV; v++) bad |= (out[v] != out[v]);
   if (bad) atomicMin(err, (unsigned long long)f);
+}
+
+// One thread per (face, condition), faces in device order: the flux, computed
+// once per face and stored as a record of fs values (nv, padded to an even count
+// when B = 1 so the record moves in 16-byte pieces).
+template <int ND, bool ONE>
+__device__ __forceinline__ void face_flux_thread(const double *__restrict__ PK, const DevMesh &dm, const GasConst &gc,
+                                                 const double *__restrict__ finf, double *__restrict__ FF, int fs,
+                                                 unsigned long long *__restrict__ err, int lgB, int t) {
+  constexpr int NV = ND + 2;
+  const int B = ONE ? 1 : 1 << lgB;
+  const int f = ONE ? t : t >> lgB, b = ONE ? 0 : t & (B - 1);
+  if (f >= dm.F) return;
+  double out[NV + 1];
+  face_flux_value<ND, ONE>(PK, dm, gc, finf, err, f, dm.fo[f], dm.fnb[f], b, B, out);
   out[NV] = 0.0;
   if constexpr (ONE) {   // fs = NV rounded up to even
     double2 *dst = reinterpret_cast<double2 *>(FF + (size_t)f * ((NV + 1) / 2 * 2));
@@ -509,6 +520,219 @@ __global__ void k_linf_reduce(const unsigned long long *bits, int nq, const unsi
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q < nq) out[q] = linf_slots_max(bits, nq, q);
   if (q == 0) out[nq] = *err;
+}
+
+// ---- few cells: a pass is one serial chain per thread on a few waves ----
+// A launch over some ten thousand cells takes the time of one thread's chain of
+// loads and FP64 operations plus the launch, whatever the arithmetic units could
+// do, so these forms shorten the chain and the number of launches instead of
+// the work: the gradient pass takes a thread per (cell, variable) and also does
+// the time step and the monitors' bookkeeping; the second pass computes each
+// face's flux from both of its cells (twice the fluxes, none stored) and sums
+// and updates in the same launch.  Every value comes from the same operations in
+// the same order as in the per-pass kernels.  An RK4 step on 3k triangles is 8
+// launches instead of 15, 41 us instead of 71.  Blocks are mapped so that an XCD
+// keeps one range of cells over all passes, whose data its L2 then still holds
+// (40k triangles, 70 -> 62 us a step; no difference at 3k).
+
+// what a gradient pass of an explicit run does besides
+struct StageAux {
+  double *dt = nullptr;                   // local time step at cfl (null: none)
+  double cfl = 0.0;
+  unsigned long long *clear = nullptr;    // monitor words to zero
+  const unsigned long long *bits = nullptr;   // monitor words of the iteration before, to be decoded
+  double *linf = nullptr;                 //   into row it - 1 of linf (it > 0)
+  int it = 0, cap = 0;
+  int *dit = nullptr;                     // device iteration counter (graph replays): it from there, then advanced
+};
+
+// by one block: rows of the monitors [v][B] of the iteration before, then the clear
+__device__ __forceinline__ void stage_aux_block(const StageAux &x, int nv, int B) {
+  const int nq = nv * B;
+  if (x.bits) {
+    const int it = x.dit ? *x.dit : x.it;
+    if (it > 0 && it <= x.cap) {
+      if (B == 1) {   // a wave per word, a lane per copy
+        for (int q = threadIdx.x >> 6; q < nq; q += blockDim.x >> 6) {
+          unsigned long long m = x.bits[(size_t)(threadIdx.x & 63) * nq + q];
+#pragma unroll
+          for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long y = __shfl_xor(m, o, 64);
+            m = y > m ? y : m;
+          }
+          if ((threadIdx.x & 63) == 0) x.linf[(size_t)(it - 1) * nq + q] = __longlong_as_double((long long)m);
+        }
+      } else {
+        for (int q = threadIdx.x; q < nq; q += blockDim.x) {
+          const int v = q / B, b = q - v * B;
+          x.linf[((size_t)(it - 1) * B + b) * nv + v] =
+              __longlong_as_double((long long)linf_slots_max(x.bits, nq, q));
+        }
+      }
+    }
+    __syncthreads();
+    if (x.dit && threadIdx.x == 0) *x.dit = it + 1;
+  }
+  if (x.clear)
+    for (int q = threadIdx.x; q < kLinfSlots * nq; q += blockDim.x) x.clear[q] = 0ull;
+}
+
+// gradlim_cell for one variable: blocks of 64 (cell, condition) units, wave v of
+// a block takes variable v; with aux.dt one more wave takes the time step.  The
+// last block does the bookkeeping.
+template <int ND>
+__global__ __launch_bounds__(64 * (ND + 3)) void k_gradlim_split(const double *__restrict__ U, DevMesh dm, GasConst gc,
+                                                                 double *__restrict__ PK, double *__restrict__ Gout,
+                                                                 double *__restrict__ Pout, double *__restrict__ frz,
+                                                                 CoefB fmask, int lgB, StageAux aux) {
+  constexpr int NV = ND + 2, K = ND + 1, GW = ND + 1;
+  const int N = dm.N, B = 1 << lgB;
+  if (blockIdx.x == gridDim.x - 1) {
+    stage_aux_block(aux, NV, B);
+    return;
+  }
+  const int v = threadIdx.x >> 6;   // wave-uniform
+  const int t = xcd_block_of(blockIdx.x, gridDim.x - 1) * 64 + (threadIdx.x & 63), i = t >> lgB, b = t & (B - 1);
+  if (i >= N) return;
+  if (v == NV) {
+    if (aux.dt) timestep_cell<ND>(U, dm, gc, aux.cfl, aux.dt, i, b, B);
+    return;
+  }
+  int nb[K];
+  double S[K][ND], w[K], uj[K], rl[K][ND];
+#pragma unroll
+  for (int m = 0; m < K; m++) {
+    nb[m] = dm.nbr[(size_t)m * N + i];
+    w[m] = dm.w[(size_t)m * N + i];
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+      S[m][d] = dm.Sg[((size_t)m * ND + d) * N + i];
+      rl[m][d] = dm.rl[((size_t)m * ND + d) * N + i];
+    }
+  }
+  const double V = dm.vol[i], eps2 = dm.eps2[i];
+  const double *Uv = U + (size_t)v * N * B + b;
+  const double u = Uv[(size_t)i * B];
+#pragma unroll
+  for (int m = 0; m < K; m++) uj[m] = Uv[(size_t)(nb[m] >= 0 ? nb[m] : i) * B];
+  double g[ND], mn = u, mx = u;
+#pragma unroll
+  for (int d = 0; d < ND; d++) g[d] = 0.0;
+#pragma unroll
+  for (int m = 0; m < K; m++) {
+    if (nb[m] >= 0) {
+      const double fv = w[m] * u + (1 - w[m]) * uj[m];
+#pragma unroll
+      for (int d = 0; d < ND; d++) g[d] += S[m][d] * fv;
+      mn = (uj[m] < mn) ? uj[m] : mn;
+      mx = (uj[m] > mx) ? uj[m] : mx;
+    } else {
+#pragma unroll
+      for (int d = 0; d < ND; d++) g[d] += S[m][d] * u;
+      if (nb[m] == -1 && v >= 1 && v <= ND) {   // slip wall: tangential momentum on the face
+        double nn[ND], mom[ND], vn = 0, na = 0;
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+          nn[d] = dm.nf[((size_t)m * ND + d) * N + i];
+          mom[d] = U[((size_t)(1 + d) * N + i) * B + b];
+        }
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+          vn += mom[d] * nn[d];
+          if (d == v - 1) na = nn[d];
+        }
+        const double tg = u - vn * na;
+#pragma unroll
+        for (int d = 0; d < ND; d++) g[d] += (tg * S[m][d] - u * S[m][d]);
+      }
+    }
+  }
+  const RcpDiv divV(V);
+#pragma unroll
+  for (int d = 0; d < ND; d++) g[d] = divV(g[d]);
+  double best = 1.0;
+  const size_t pq = ((size_t)v * N + i) * B + b;
+  if (frz && fmask.c[b] != 0.0) {
+    best = frz[pq];
+  } else {
+    const double dmin = mn - u, dmax = mx - u;
+#pragma unroll
+    for (int m = 0; m < K; m++) {
+      if (nb[m] < 0) continue;
+      double d2 = 0;
+#pragma unroll
+      for (int d = 0; d < ND; d++) d2 += g[d] * rl[m][d];
+      d2 /= 2.0;
+      const double f = face_limiter(dmin, dmax, d2, eps2);
+      best = (f < best) ? f : best;
+    }
+    if (frz) frz[pq] = best;
+  }
+  double *pk = PK + ((size_t)i * NV + v) * GW * B + b;
+  pk[0] = u;
+#pragma unroll
+  for (int d = 0; d < ND; d++) {
+    if (Gout) Gout[(((size_t)v * ND + d) * N + i) * B + b] = g[d];
+    pk[(size_t)(1 + d) * B] = best * g[d];
+  }
+  if (Pout) Pout[pq] = best;
+}
+
+// Face fluxes, residual, stage update and monitors of blocks of 64 (cell,
+// condition) units: wave q takes the units' q-th faces (reference face order),
+// the fluxes meet in LDS, then wave v sums and updates variable v.
+template <int ND, bool ONE>
+__global__ __launch_bounds__(64 * (ND + 2)) void k_residual_faces(
+    const double *__restrict__ PK, DevMesh dm, GasConst gc, const double *__restrict__ finf,
+    // U0 and Ud may be the same array (see cell_residual_block)
+    const double *U0, double *Ud, const double *__restrict__ dt, const double *__restrict__ dtg, double alpha,
+    double *__restrict__ Rout, unsigned long long *__restrict__ linf_bits, unsigned long long *__restrict__ err,
+    int lgB) {
+  constexpr int NV = ND + 2, K = ND + 1;
+  __shared__ double fx[K][NV][64];
+  const int N = dm.N, B = ONE ? 1 : 1 << lgB;
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = xcd_block() * 64 + lane, i = ONE ? t : t >> lgB, b = ONE ? 0 : t & (B - 1);
+  double aq[K];
+  if (i < N) {
+#pragma unroll
+    for (int q = 0; q < K; q++) aq[q] = dm.saq[(size_t)q * N + i];
+    if (wv < K) {
+      const uint32_t info = dm.info[i];
+      const int f = dm.cfq[(size_t)wv * N + i], m = (info >> (2 * wv)) & 3;
+      int j = 0;
+#pragma unroll
+      for (int mm = 0; mm < K; mm++) {
+        const int nb = dm.nbr[(size_t)mm * N + i];
+        j = mm == m ? nb : j;
+      }
+      const bool own = (info >> (8 + m)) & 1;
+      double out[NV];
+      face_flux_value<ND, ONE>(PK, dm, gc, finf, err, f, own ? i : j, own ? j : i, b, B, out);
+#pragma unroll
+      for (int v = 0; v < NV; v++) fx[wv][v][lane] = out[v];
+    }
+  }
+  __syncthreads();
+  const int v = wv;
+  double R = 0.0;
+  if (i < N) {
+#pragma unroll
+    for (int q = 0; q < K; q++) R += fx[q][v][lane] * aq[q];
+    const size_t q = ((size_t)v * N + i) * B + b;
+    if (Ud) {
+      const double c = alpha * (dtg ? dtg[b] : dt[(size_t)i * B + b]) / dm.vol[i];
+      Ud[q] = U0[q] - c * R;
+    }
+    if (Rout) Rout[q] = R;
+  }
+  if (linf_bits) {
+    double a = ::fabs(R);
+    for (int o = 32; o >= B; o >>= 1) a = fmax(a, __shfl_xor(a, o, 64));
+    if (lane < B)
+      atomicMax(&linf_slot_of(linf_bits, NV * B, blockIdx.x)[v * B + lane],
+                (unsigned long long)__double_as_longlong(a));
+  }
 }
 
 // Persistent form of bes_explicit_run for one condition with local time
@@ -923,14 +1147,35 @@ double gradlim_bytes(const bes_ctx *c) {
   return N * (8 * nv * B + k * (4 + 16 * nd + 8) + 16 + 8 * nv * (1 + nd) * B);
 }
 
-// one thread per (cell, condition)
-int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout) {
+// Up to this many (cell, condition) units a pass is bound by the length of a
+// thread's chain and by launches, and the split forms are taken.  RK4 step as a
+// graph, split against per-pass kernels: 3k triangles 41 / 71 us, 40k 62 / 86,
+// 102k 108 / 116, 160k 143 / 143; tetrahedra 3k 49 / 91, 48k 102 / 126, 64k
+// 130 / 134, 94k 176 / 168; 64 conditions x 1,200 triangles 71 / 114, 32
+// conditions x 3,840 tetrahedra 201 / 154.
+static bool split_pass(const bes_ctx *c) { return (long)c->N * c->B <= (c->nd == 2 ? 131072 : 65536); }
+
+// one thread per (cell, condition), or per (cell, condition, variable); aux is
+// for the split form only
+int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout, const StageAux *aux = nullptr) {
   const int bs = tuned_bs(c, kProfGradlim), nb = grid_for(c->N * c->B, bs);
   ProfScope ps(c, kProfGradlim, gradlim_bytes(c));
   CoefB fm;
   for (int b = 0; b < bes_ctx::kMaxBatch; b++)
     fm.c[b] = (b < (int)c->lim_frozen.size() && c->lim_frozen[b]) ? 1.0 : 0.0;
   double *frz = c->lim_freeze_on ? c->phi_frz : nullptr;
+  if (split_pass(c)) {
+    const StageAux ax = aux ? *aux : StageAux();
+    const dim3 grid(grid_for(c->N * c->B, 64) + 1), block(64 * (c->nv + (ax.dt ? 1 : 0)));
+    if (c->nd == 2)
+      hipLaunchKernelGGL(k_gradlim_split<2>, grid, block, 0, c->stream, U, c->dm, c->gc, c->LG, Gout, Pout, frz, fm,
+                         c->lgB, ax);
+    else
+      hipLaunchKernelGGL(k_gradlim_split<3>, grid, block, 0, c->stream, U, c->dm, c->gc, c->LG, Gout, Pout, frz, fm,
+                         c->lgB, ax);
+    BES_HIP(hipGetLastError());
+    return BES_OK;
+  }
   // one condition: the block's packs are staged in LDS
   const bool one = c->B == 1;
   const size_t lds = one ? (size_t)bs * c->nv * (c->nd + 1) * sizeof(double) : 0;
@@ -973,11 +1218,23 @@ double residual_bytes(const bes_ctx *c, bool update, bool rout) {
 // residual of the packs of the last gradient pass; with U0/Ud the stage update
 int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int local, double *Rout,
                     unsigned long long *linf_bits) {
+  const double *dtg = local ? nullptr : c->dtg;
+  const bool one = c->B == 1;
+  if (split_pass(c)) {
+    // the packs of both sides and the face records per cell face
+    ProfScope ps(c, kProfResidual, residual_bytes(c, U0 != nullptr, Rout != nullptr) + faceflux_bytes(c));
+    by_shape(c->nd, one, [&](auto nd, auto one_) {
+      constexpr int ND = decltype(nd)::value;
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual_faces<ND, decltype(one_)::value>), dim3(grid_for(c->N * c->B, 64)),
+                         dim3(64 * (ND + 2)), 0, c->stream, c->LG, c->dm, c->gc, c->dfinf, U0, Ud, c->dt, dtg, alpha,
+                         Rout, linf_bits, c->err, c->lgB);
+    });
+    BES_HIP(hipGetLastError());
+    return BES_OK;
+  }
   int s = launch_face_flux(c);
   if (s) return s;
   const int bs = tuned_bs(c, kProfResidual), nb = grid_for(c->N * c->B, bs);
-  const double *dtg = local ? nullptr : c->dtg;
-  const bool one = c->B == 1;
   ProfScope ps(c, kProfResidual, residual_bytes(c, U0 != nullptr, Rout != nullptr));
   by_shape(c->nd, one, [&](auto nd, auto one_) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_residual<decltype(nd)::value, decltype(one_)::value>),
@@ -1374,27 +1631,54 @@ int bes_compute_residual(bes_ctx *c, double *R_out, double *maxabs_out) {
 }
 
 // one pseudo-time step (SolverExplicit.cpp:259-393) on the context stream;
-// it_host < 0: the Linf row index comes from the device counter
+// it_host < 0: the Linf row index comes from the device counter.  The split form
+// decodes a step's monitors in the next step's first pass (explicit_last_linf
+// after the run decodes the last).
 static int explicit_iteration(bes_ctx *c, int nstage, const double *alpha, double cfl, int local, bool linf,
                               int it_host) {
   const int nv = c->nv, B = c->B;
+  const bool split = split_pass(c);
   unsigned long long *bits = c->lbits;
   int s;
-  if ((s = launch_timestep(c, c->U0, cfl, local))) return s;
+  if (!(split && local) && (s = launch_timestep(c, c->U0, cfl, local))) return s;
   for (int st = 0; st < nstage; st++) {
     const bool last = st == nstage - 1;
     const double *src = st == 0 ? c->U0 : ((st - 1) % 2 == 0 ? c->Ua : c->Ub);
     double *dst = (last && nstage > 1) ? c->U0 : (st % 2 == 0 ? c->Ua : c->Ub);
-    if ((s = launch_gradlim(c, src, nullptr, nullptr))) return s;
-    if (last && linf && (s = fill_bits(c, bits, kLinfSlots * nv * B, 0ull))) return s;
+    StageAux aux;
+    if (split) {
+      if (st == 0 && local) {
+        aux.dt = c->dt;
+        aux.cfl = cfl;
+      }
+      if (st == 0 && linf) {
+        aux.bits = bits;
+        aux.linf = c->linf;
+        aux.it = it_host;
+        aux.cap = c->linf_cap;
+        aux.dit = it_host < 0 ? c->dit : nullptr;
+      }
+      if (last && linf) aux.clear = bits;
+    }
+    if ((s = launch_gradlim(c, src, nullptr, nullptr, &aux))) return s;
+    if (last && linf && !split && (s = fill_bits(c, bits, kLinfSlots * nv * B, 0ull))) return s;
     if ((s = launch_residual(c, c->U0, dst, alpha[st], local, nullptr, (last && linf) ? bits : nullptr))) return s;
-    if (last && linf) {
+    if (last && linf && !split) {
       hipLaunchKernelGGL(k_linf_decode, dim3(1), dim3(nv * B), 0, c->stream, bits, c->linf, nv, B,
                          it_host < 0 ? 0 : it_host, c->linf_cap, it_host < 0 ? c->dit : nullptr);
       BES_HIP(hipGetLastError());
     }
     if (last && nstage == 1) std::swap(c->U0, c->Ua);
   }
+  return BES_OK;
+}
+
+// the monitors of the last step of a run of niter steps
+static int explicit_last_linf(bes_ctx *c, int niter) {
+  if (!split_pass(c) || niter < 1) return BES_OK;
+  hipLaunchKernelGGL(k_linf_decode, dim3(1), dim3(c->nv * c->B), 0, c->stream, c->lbits, c->linf, c->nv, c->B,
+                     niter - 1, c->linf_cap, nullptr);
+  BES_HIP(hipGetLastError());
   return BES_OK;
 }
 
@@ -1503,6 +1787,7 @@ int bes_explicit_run(bes_ctx *c, int niter, int nstage, const double *alpha, dou
     for (int it = 0; it < niter; it++)
       if ((s = explicit_iteration(c, nstage, alpha, cfl, local, linf_out != nullptr, it))) return s;
   }
+  if (linf_out && !persist && (s = explicit_last_linf(c, niter))) return s;
   if ((s = prof_collect(c))) return s;
   if (linf_out && niter > 0) {
     BES_HIP(hipMemcpyAsync(linf_out, c->linf, (size_t)niter * nv * B * sizeof(double), hipMemcpyDeviceToHost,

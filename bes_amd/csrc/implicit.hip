@@ -42,7 +42,8 @@ namespace bes {
 
 int launch_timestep(bes_ctx *c, const double *U, double cfl, int local, const double *cfl_b = nullptr);
 int launch_face_flux(bes_ctx *c);
-int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout);
+struct StageAux;   // explicit.hip
+int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout, const StageAux *aux = nullptr);
 int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int local, double *Rout,
                     unsigned long long *linf_bits);
 int state_to_host(bes_ctx *c, const double *dsoa, int ncomp, double *host);

@@ -9,12 +9,12 @@ namespace bes {
 // with its own L2.  Remap the hardware block id so that XCD x processes one
 // contiguous range of blocks: Morton-ordered neighbours then share an L2.
 // The map is a bijection on [0, gridDim.x) for any grid size.
-__device__ __forceinline__ int xcd_block() {
-  const int nb = gridDim.x, b = blockIdx.x;
+__device__ __forceinline__ int xcd_block_of(int b, int nb) {
   const int full = nb >> 3, rem = nb & 7, x = b & 7, q = b >> 3;
   const int start = x * full + (x < rem ? x : rem);
   return start + q;
 }
+__device__ __forceinline__ int xcd_block() { return xcd_block_of(blockIdx.x, gridDim.x); }
 
 __device__ __forceinline__ int cell_index() { return xcd_block() * blockDim.x + threadIdx.x; }
 
