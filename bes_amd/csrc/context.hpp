@@ -34,8 +34,13 @@ struct DevMesh {
   int *fo = nullptr;        // [F] owner cell
   int *fnb = nullptr;       // [F] neighbour cell, -1 slip wall, -2 far field
   double *fnr = nullptr;    // [nd][F] unit normal, owner -> neighbour
-  double *frs = nullptr;    // [nd][F] owner's reconstruction vector for the face
-  double *frn = nullptr;    // [nd][F] neighbour's reconstruction vector for the face
+  double *frs = nullptr;    // [nd][F] owner's reconstruction vector for the face (null where common)
+  double *frn = nullptr;    // [nd][F] neighbour's reconstruction vector for the face (null where common)
+  // meshes whose cells use one reconstruction vector, to local face 0, for all
+  // their faces but the mesh's face 0 (bes_ctx::common): that face, its cells
+  // and their states at it
+  int odd_face = -1, odd_owner = -1, odd_nbr = -1;
+  double *odd_state = nullptr;   // [2][nv][B] owner's, neighbour's
 };
 
 // Matrix storage of the implicit path (block CSR, own block first in each row).
@@ -71,7 +76,10 @@ struct bes_ctx {
   bes::DevMesh dm;
   hipStream_t stream = nullptr;
   double *U0 = nullptr, *Ua = nullptr, *Ub = nullptr;  // [nv][N][B]
-  double *LG = nullptr;        // [N][nv][1+nd][B] per-cell pack: per variable U_v, then phi*grad U_v [d]
+  double *LG = nullptr;        // [N][pw][B] per-cell record of the gradient pass: per variable U_v, then phi*grad
+                               // U_v [d]; where common the reconstructed state [nv] (even length for B = 1)
+  size_t pw = 0;               // its length
+  bool common = false;         // one reconstruction vector per cell (geom_mode without its bit 4)
   double *FF = nullptr;        // [F][fs][B] face fluxes per unit area (device face order)
   int fs = 0;                  // face-flux record length: nv, rounded up to even for B = 1 (16-byte access)
   std::vector<int64_t> fref;   // reference face id of each device face

@@ -139,9 +139,30 @@ __device__ __forceinline__ double face_limiter(double mn, double mx, double d2, 
   return (d2 > 0 || d2 < 0) ? r : 1.0;
 }
 
+// What the gradient pass leaves of a cell for the face pass.  In general the pack
+// [NV][1 + ND]: per variable U_v, then phi_v * grad U_v.  With RC (DevMesh::common:
+// every face of a cell but one uses the same reconstruction vector, the
+// reference's own lookup) the reconstructed state U + (phi*grad).r itself, NV
+// values instead of NV*(1 + ND); the operations and their order are the face
+// pass's, so the face states are the same bits.  Records of one condition are
+// padded to an even length (16-byte access).
+// Tetrahedra: 48 instead of 160 bytes a cell written and read, 48 bytes of
+// reconstruction vectors a face not read; on a 750k-tet box k_gradlim 84 -> 69 us,
+// k_face_flux 78 -> 44; 64 conditions x 31k tetrahedra 150 -> 129 and 164 -> 82.
+template <int ND, bool ONE, bool RC>
+struct PackW {
+  static constexpr int W = RC ? (ONE ? (ND + 3) / 2 * 2 : ND + 2) : (ND + 2) * (ND + 1);
+};
+
+// the reconstructed state of a cell that has the mesh's face 0, for that face
+// (its vector is the one to the cell's last face)
+__device__ __forceinline__ int odd_side(const DevMesh &dm, int i) {
+  return i == dm.odd_owner ? 0 : (i == dm.odd_nbr ? 1 : -1);
+}
+
 // the gradient, limiter and pack of one (cell, condition); the pack goes to
-// stage (PW doubles) when STAGE, else to PK
-template <int ND, bool STAGE>
+// stage (PackW doubles) when STAGE, else to PK
+template <int ND, bool STAGE, bool RC>
 __device__ __forceinline__ void gradlim_cell(const double *__restrict__ U, const DevMesh &dm,
                                              double *__restrict__ PK, double *__restrict__ Gout,
                                              double *__restrict__ Pout, double *__restrict__ frz,
@@ -242,7 +263,20 @@ __device__ __forceinline__ void gradlim_cell(const double *__restrict__ U, const
       pk[1 + d] = best * g[v][d];
     }
     if (Pout) Pout[pq] = best;
-    if constexpr (STAGE) {
+    if constexpr (RC) {
+      double uf = u[v];
+#pragma unroll
+      for (int d = 0; d < ND; d++) uf += pk[1 + d] * rl[0][d];
+      if constexpr (STAGE) stage[v] = uf;
+      else PK[((size_t)i * NV + v) * B + b] = uf;
+      const int side = odd_side(dm, i);
+      if (side >= 0) {
+        double uo = u[v];
+#pragma unroll
+        for (int d = 0; d < ND; d++) uo += pk[1 + d] * rl[K - 1][d];
+        dm.odd_state[((size_t)side * NV + v) * B + b] = uo;
+      }
+    } else if constexpr (STAGE) {
 #pragma unroll
       for (int q = 0; q < GW; q++) stage[v * GW + q] = pk[q];
     } else {
@@ -271,14 +305,15 @@ __device__ __forceinline__ void gradlim_cell(const double *__restrict__ U, const
 // apart and lines leave L2 partly written.
 // the cells of block blk (one condition), packs staged in sm (blockDim.x*PW
 // doubles); every thread of the block must call it
-template <int ND>
+template <int ND, bool RC>
 __device__ __forceinline__ void gradlim_block_one(const double *__restrict__ U, const DevMesh &dm,
                                                   double *__restrict__ PK, double *__restrict__ Gout,
                                                   double *__restrict__ Pout, double *__restrict__ frz,
                                                   const CoefB &fmask, int blk, double *sm) {
-  constexpr int PW = (ND + 2) * (ND + 1);
+  constexpr int PW = PackW<ND, true, RC>::W;
   const int N = dm.N, i0 = blk * blockDim.x, t = i0 + threadIdx.x;
-  if (t < N) gradlim_cell<ND, true>(U, dm, PK, Gout, Pout, frz, fmask, t, 0, 1, sm + threadIdx.x * PW);
+  if constexpr (RC && PW > ND + 2) sm[threadIdx.x * PW + PW - 1] = 0.0;
+  if (t < N) gradlim_cell<ND, true, RC>(U, dm, PK, Gout, Pout, frz, fmask, t, 0, 1, sm + threadIdx.x * PW);
   __syncthreads();
   const int nc = min((int)blockDim.x, N - i0);   // cells of this block (i0 < N: the blocks cover N)
   const double2 *src = reinterpret_cast<const double2 *>(sm);
@@ -287,29 +322,27 @@ __device__ __forceinline__ void gradlim_block_one(const double *__restrict__ U, 
   __syncthreads();   // sm is free again for the block's next call
 }
 
-template <int ND, bool ONE>
+template <int ND, bool ONE, bool RC>
 __global__ __launch_bounds__(256) void k_gradlim(const double *__restrict__ U, DevMesh dm,
                                                     double *__restrict__ PK, double *__restrict__ Gout,
                                                     double *__restrict__ Pout, double *__restrict__ frz,
                                                     CoefB fmask, int lgB) {
-  constexpr int NV = ND + 2, GW = ND + 1, PW = NV * GW;
   extern __shared__ double sm_pack[];
   const int N = dm.N;
   const int i0 = blockIdx.x * blockDim.x;   // dispatch order (see k_cell_residual)
   const int t = i0 + threadIdx.x;
   if constexpr (!ONE) {
     const int B = 1 << lgB, i = t >> lgB, b = t & (B - 1);
-    if (i < N) gradlim_cell<ND, false>(U, dm, PK, Gout, Pout, frz, fmask, i, b, B, nullptr);
+    if (i < N) gradlim_cell<ND, false, RC>(U, dm, PK, Gout, Pout, frz, fmask, i, b, B, nullptr);
   } else {
-    gradlim_block_one<ND>(U, dm, PK, Gout, Pout, frz, fmask, blockIdx.x, sm_pack);
+    gradlim_block_one<ND, RC>(U, dm, PK, Gout, Pout, frz, fmask, blockIdx.x, sm_pack);
   }
 }
 
-// a cell pack [NV][1 + ND] of one condition into registers (ONE: the
-// single-condition layout, the pack in 16-byte pieces)
-template <int ND, bool ONE>
+// a cell's record (PackW values) of condition b into registers (ONE: the
+// single-condition layout, in 16-byte pieces)
+template <int PW, bool ONE>
 __device__ __forceinline__ void load_pack(const double *__restrict__ PK, int cell, int b, int B, double *pk) {
-  constexpr int PW = (ND + 2) * (ND + 1);
   if constexpr (ONE) {
     const double2 *src = reinterpret_cast<const double2 *>(PK + (size_t)cell * PW);
 #pragma unroll
@@ -340,30 +373,46 @@ __device__ __forceinline__ void face_state(const double *pk, const double *r, do
 // condition b: second-order states of both sides from the cell packs, then
 // FluxRoe.tpp:306-333, FluxFreestream.tpp:192-226 or FluxSlipWall.tpp:32-53.
 // finf: freestream primitive state per condition.
-template <int ND, bool ONE>
+template <int ND, bool ONE, bool RC>
 __device__ __forceinline__ void face_flux_value(const double *__restrict__ PK, const DevMesh &dm, const GasConst &gc,
                                                 const double *__restrict__ finf,
                                                 unsigned long long *__restrict__ err, int f, int o, int j, int b,
                                                 int B, double *out) {
-  constexpr int NV = ND + 2;
+  constexpr int NV = ND + 2, PW = PackW<ND, ONE, RC>::W;
   const int F = dm.F;
   // both sides' packs and the face geometry are requested before any of them
   // is used (a boundary face reads its owner's pack twice, from cache), so the
   // two gathers overlap instead of taking one memory round trip each
-  double nn[ND], rs[ND], rn[ND], ul[NV];
-  double pko[(ND + 2) * (ND + 1)], pkn[(ND + 2) * (ND + 1)];
+  double nn[ND], rs[ND], rn[ND], ul[NV], ur[NV];
+  double pko[PW], pkn[PW];
 #pragma unroll
   for (int d = 0; d < ND; d++) {
     nn[d] = dm.fnr[(size_t)d * F + f];
-    rs[d] = dm.frs[(size_t)d * F + f];
-    rn[d] = dm.frn[(size_t)d * F + f];
+    if constexpr (!RC) {
+      rs[d] = dm.frs[(size_t)d * F + f];
+      rn[d] = dm.frn[(size_t)d * F + f];
+    }
   }
-  load_pack<ND, ONE>(PK, o, b, B, pko);
-  load_pack<ND, ONE>(PK, j >= 0 ? j : o, b, B, pkn);
-  face_state<ND>(pko, rs, ul);
+  load_pack<PW, ONE>(PK, o, b, B, pko);
+  load_pack<PW, ONE>(PK, j >= 0 ? j : o, b, B, pkn);
+  if constexpr (RC) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      ul[v] = pko[v];
+      ur[v] = pkn[v];
+    }
+    if (f == dm.odd_face) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        ul[v] = dm.odd_state[(size_t)v * B + b];
+        ur[v] = dm.odd_state[((size_t)NV + v) * B + b];
+      }
+    }
+  } else {
+    face_state<ND>(pko, rs, ul);
+    if (j >= 0) face_state<ND>(pkn, rn, ur);
+  }
   if (j >= 0) {
-    double ur[NV];
-    face_state<ND>(pkn, rn, ur);
     roe_flux<ND, double>(gc, ul, ur, nn, out);
   } else if (j == -1) {
     slip_flux<ND, double>(gc, ul, nn, out);
@@ -382,7 +431,7 @@ __device__ __forceinline__ void face_flux_value(const double *__restrict__ PK, c
 // One thread per (face, condition), faces in device order: the flux, computed
 // once per face and stored as a record of fs values (nv, padded to an even count
 // when B = 1 so the record moves in 16-byte pieces).
-template <int ND, bool ONE>
+template <int ND, bool ONE, bool RC>
 __device__ __forceinline__ void face_flux_thread(const double *__restrict__ PK, const DevMesh &dm, const GasConst &gc,
                                                  const double *__restrict__ finf, double *__restrict__ FF, int fs,
                                                  unsigned long long *__restrict__ err, int lgB, int t) {
@@ -391,7 +440,7 @@ __device__ __forceinline__ void face_flux_thread(const double *__restrict__ PK, 
   const int f = ONE ? t : t >> lgB, b = ONE ? 0 : t & (B - 1);
   if (f >= dm.F) return;
   double out[NV + 1];
-  face_flux_value<ND, ONE>(PK, dm, gc, finf, err, f, dm.fo[f], dm.fnb[f], b, B, out);
+  face_flux_value<ND, ONE, RC>(PK, dm, gc, finf, err, f, dm.fo[f], dm.fnb[f], b, B, out);
   out[NV] = 0.0;
   if constexpr (ONE) {   // fs = NV rounded up to even
     double2 *dst = reinterpret_cast<double2 *>(FF + (size_t)f * ((NV + 1) / 2 * 2));
@@ -403,12 +452,12 @@ __device__ __forceinline__ void face_flux_thread(const double *__restrict__ PK, 
   }
 }
 
-template <int ND, bool ONE>
+template <int ND, bool ONE, bool RC>
 __global__ __launch_bounds__(256) void k_face_flux(const double *__restrict__ PK, DevMesh dm, GasConst gc,
                                                    const double *__restrict__ finf, double *__restrict__ FF,
                                                    int fs, unsigned long long *__restrict__ err, int lgB) {
   // dispatch order (see k_cell_residual)
-  face_flux_thread<ND, ONE>(PK, dm, gc, finf, FF, fs, err, lgB, blockIdx.x * blockDim.x + threadIdx.x);
+  face_flux_thread<ND, ONE, RC>(PK, dm, gc, finf, FF, fs, err, lgB, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // One thread per (cell, condition): residual sum_f +-F*A over the cell's faces
@@ -580,7 +629,7 @@ __device__ __forceinline__ void stage_aux_block(const StageAux &x, int nv, int B
 // gradlim_cell for one variable: blocks of 64 (cell, condition) units, wave v of
 // a block takes variable v; with aux.dt one more wave takes the time step.  The
 // last block does the bookkeeping.
-template <int ND>
+template <int ND, bool RC>
 __global__ __launch_bounds__(64 * (ND + 3)) void k_gradlim_split(const double *__restrict__ U, DevMesh dm, GasConst gc,
                                                                  double *__restrict__ PK, double *__restrict__ Gout,
                                                                  double *__restrict__ Pout, double *__restrict__ frz,
@@ -668,12 +717,30 @@ __global__ __launch_bounds__(64 * (ND + 3)) void k_gradlim_split(const double *_
     }
     if (frz) frz[pq] = best;
   }
-  double *pk = PK + ((size_t)i * NV + v) * GW * B + b;
-  pk[0] = u;
+  double lg[ND];
 #pragma unroll
   for (int d = 0; d < ND; d++) {
     if (Gout) Gout[(((size_t)v * ND + d) * N + i) * B + b] = g[d];
-    pk[(size_t)(1 + d) * B] = best * g[d];
+    lg[d] = best * g[d];
+  }
+  if constexpr (RC) {
+    double uf = u;
+#pragma unroll
+    for (int d = 0; d < ND; d++) uf += lg[d] * rl[0][d];
+    if (lgB == 0) PK[(size_t)i * PackW<ND, true, RC>::W + v] = uf;
+    else PK[((size_t)i * NV + v) * B + b] = uf;
+    const int side = odd_side(dm, i);
+    if (side >= 0) {
+      double uo = u;
+#pragma unroll
+      for (int d = 0; d < ND; d++) uo += lg[d] * rl[K - 1][d];
+      dm.odd_state[((size_t)side * NV + v) * B + b] = uo;
+    }
+  } else {
+    double *pk = PK + ((size_t)i * NV + v) * GW * B + b;
+    pk[0] = u;
+#pragma unroll
+    for (int d = 0; d < ND; d++) pk[(size_t)(1 + d) * B] = lg[d];
   }
   if (Pout) Pout[pq] = best;
 }
@@ -681,7 +748,7 @@ __global__ __launch_bounds__(64 * (ND + 3)) void k_gradlim_split(const double *_
 // Face fluxes, residual, stage update and monitors of blocks of 64 (cell,
 // condition) units: wave q takes the units' q-th faces (reference face order),
 // the fluxes meet in LDS, then wave v sums and updates variable v.
-template <int ND, bool ONE>
+template <int ND, bool ONE, bool RC>
 __global__ __launch_bounds__(64 * (ND + 2)) void k_residual_faces(
     const double *__restrict__ PK, DevMesh dm, GasConst gc, const double *__restrict__ finf,
     // U0 and Ud may be the same array (see cell_residual_block)
@@ -708,7 +775,7 @@ __global__ __launch_bounds__(64 * (ND + 2)) void k_residual_faces(
       }
       const bool own = (info >> (8 + m)) & 1;
       double out[NV];
-      face_flux_value<ND, ONE>(PK, dm, gc, finf, err, f, own ? i : j, own ? j : i, b, B, out);
+      face_flux_value<ND, ONE, RC>(PK, dm, gc, finf, err, f, own ? i : j, own ? j : i, b, B, out);
 #pragma unroll
       for (int v = 0; v < NV; v++) fx[wv][v][lane] = out[v];
     }
@@ -754,7 +821,7 @@ struct PersistStep {
   int nstage, niter, linf_cap;
 };
 
-template <int ND>
+template <int ND, bool RC>
 __global__ __launch_bounds__(256) void k_explicit_persistent(PersistStep a, DevMesh dm, GasConst gc, CoefB fmask) {
   constexpr int NV = ND + 2, FS = (NV + 1) / 2 * 2;
   extern __shared__ double sm_pack[];
@@ -772,7 +839,7 @@ __global__ __launch_bounds__(256) void k_explicit_persistent(PersistStep a, DevM
       const double *src = st == 0 ? U0 : ((st - 1) % 2 == 0 ? Ua : a.Ub);
       double *dst = (last && a.nstage > 1) ? U0 : (st % 2 == 0 ? Ua : a.Ub);
       for (int blk = blockIdx.x; blk < nbc; blk += gridDim.x)
-        gradlim_block_one<ND>(src, dm, a.PK, nullptr, nullptr, a.frz, fmask, blk, sm_pack);
+        gradlim_block_one<ND, RC>(src, dm, a.PK, nullptr, nullptr, a.frz, fmask, blk, sm_pack);
       grid.sync();
       // the monitor words are cleared here: block 0 decoded the previous
       // step's before it reached the barrier above, and the adds come after
@@ -781,7 +848,7 @@ __global__ __launch_bounds__(256) void k_explicit_persistent(PersistStep a, DevM
         for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < kLinfSlots * NV; q += gridDim.x * blockDim.x)
           a.lbits[q] = 0ull;
       for (int blk = blockIdx.x; blk < nbf; blk += gridDim.x)
-        face_flux_thread<ND, true>(a.PK, dm, gc, a.finf, a.FF, FS, a.err, 0, blk * blockDim.x + threadIdx.x);
+        face_flux_thread<ND, true, RC>(a.PK, dm, gc, a.finf, a.FF, FS, a.err, 0, blk * blockDim.x + threadIdx.x);
       grid.sync();
       for (int blk = blockIdx.x; blk < nbc; blk += gridDim.x)
         cell_residual_block<ND, true>(a.FF, FS, U0, dst, a.dt, nullptr, a.alpha[st], dm, nullptr,
@@ -948,7 +1015,14 @@ static int build_device_mesh(bes_ctx *c) {
   }
   if ((int)dev2ref.size() != F) { set_error("face ownership is inconsistent"); return BES_ERR_MESH; }
   std::vector<int> fo(F), fnb(F);
-  std::vector<double> fnr((size_t)nd * F), frs((size_t)nd * F), frn((size_t)nd * F, 0.0);
+  // one reconstruction vector for all faces of a cell but the mesh's face 0
+  // (rsel, the reference's lookup), unless the mode gives every face its own
+  const bool common = !(g.mode & 4);
+  std::vector<double> fnr((size_t)nd * F), frs, frn;
+  if (!common) {
+    frs.assign((size_t)nd * F, 0.0);
+    frn.assign((size_t)nd * F, 0.0);
+  }
   // reconstruction vector a cell uses for one of its faces (rsel: Q22 in compat mode)
   auto recon = [&](int64_t cell, int64_t f, int d) -> double {
     for (int mm = 0; mm < k; mm++)
@@ -961,6 +1035,7 @@ static int build_device_mesh(bes_ctx *c) {
     fnb[q] = g.nbr[f] >= 0 ? (int)c->iperm[g.nbr[f]] : (g.btype[f] == kSlipWall ? -1 : -2);
     for (int d = 0; d < nd; d++) {
       fnr[(size_t)d * F + q] = g.n[f * nd + d];
+      if (common) continue;
       frs[(size_t)d * F + q] = recon(g.owner[f], f, d);
       if (g.nbr[f] >= 0) frn[(size_t)d * F + q] = recon(g.nbr[f], f, d);
     }
@@ -1007,6 +1082,12 @@ static int build_device_mesh(bes_ctx *c) {
   }
   DevMesh &dm = c->dm;
   dm.nd = nd; dm.k = k; dm.N = N; dm.F = F;
+  c->common = common;
+  if (common && F > 0) {
+    dm.odd_face = ref2dev[0];
+    dm.odd_owner = (int)c->iperm[g.owner[0]];
+    dm.odd_nbr = g.nbr[0] >= 0 ? (int)c->iperm[g.nbr[0]] : -1;
+  }
   int s;
   if ((s = upload(&dm.vol, vol)) || (s = upload(&dm.eps2, eps2)) || (s = upload(&dm.sproj, sproj)) ||
       (s = upload(&dm.nbr, nbr)) || (s = upload(&dm.Sg, Sg)) || (s = upload(&dm.w, w)) ||
@@ -1049,8 +1130,11 @@ static int create_from_input(const MeshInput &in, int geom_mode, const bes_gas *
   if (he != hipSuccess) { s = hip_fail(he, "hipStreamCreate"); delete c; return s; }
   const size_t N = c->N, nv = c->nv, nd = c->nd;
   c->fs = (int)((nv + 1) / 2 * 2);
-  if ((s = build_device_mesh(c)) || (s = dalloc(&c->U0, nv * N)) || (s = dalloc(&c->Ua, nv * N)) ||
-      (s = dalloc(&c->Ub, nv * N)) || (s = dalloc(&c->LG, nv * (1 + nd) * N)) ||
+  if ((s = build_device_mesh(c))) { bes_ctx_destroy(c); return s; }
+  c->pw = (size_t)(c->common ? c->fs : (int)(nv * (1 + nd)));
+  if ((s = dalloc(&c->U0, nv * N)) || (s = dalloc(&c->Ua, nv * N)) ||
+      (s = dalloc(&c->Ub, nv * N)) || (s = dalloc(&c->LG, c->pw * N)) ||
+      (s = dalloc(&c->dm.odd_state, 2 * 5 * (size_t)bes_ctx::kMaxBatch)) ||
       (s = dalloc(&c->FF, (size_t)c->fs * c->dm.F)) || (s = dalloc(&c->dt, N)) ||
       (s = dalloc(&c->dtg, bes_ctx::kMaxBatch)) || (s = dalloc(&c->red, bes_ctx::kRedWords)) ||
       (s = dalloc(&c->lbits, (size_t)kLinfSlots * 5 * bes_ctx::kMaxBatch)) ||
@@ -1126,25 +1210,26 @@ int launch_timestep(bes_ctx *c, const double *U, double cfl, int local, const do
   return BES_OK;
 }
 
-// calls f(integral_constant nd, bool_constant one) for the kernel instance
-// of the mesh dimension and of a single-condition (one) or batched launch
+// calls f(integral_constant nd, bool_constant one, bool_constant rc) for the
+// kernel instance of the mesh dimension, of a single-condition (one) or batched
+// launch and of the pack's form (rc: PackW)
 template <typename Fn>
-void by_shape(int nd, bool one, Fn &&f) {
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
-  if (nd == 2) {
-    if (one) f(I2{}, std::true_type{});
-    else f(I2{}, std::false_type{});
-  } else {
-    if (one) f(I3{}, std::true_type{});
-    else f(I3{}, std::false_type{});
-  }
+void by_mesh(const bes_ctx *c, Fn &&f) {
+  auto forms = [&](auto nd) {
+    const bool one = c->B == 1;
+    if (one && c->common) f(nd, std::true_type{}, std::true_type{});
+    else if (one) f(nd, std::true_type{}, std::false_type{});
+    else if (c->common) f(nd, std::false_type{}, std::true_type{});
+    else f(nd, std::false_type{}, std::false_type{});
+  };
+  if (c->nd == 2) forms(std::integral_constant<int, 2>{});
+  else forms(std::integral_constant<int, 3>{});
 }
 
 // algorithmic HBM bytes of one gradient+limiter launch: state, geometry, pack
 double gradlim_bytes(const bes_ctx *c) {
   const double N = c->N, B = c->B, nv = c->nv, nd = c->nd, k = c->k;
-  return N * (8 * nv * B + k * (4 + 16 * nd + 8) + 16 + 8 * nv * (1 + nd) * B);
+  return N * (8 * nv * B + k * (4 + 16 * nd + 8) + 16 + 8.0 * c->pw * B);
 }
 
 // Up to this many (cell, condition) units a pass is bound by the length of a
@@ -1167,20 +1252,18 @@ int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout, cons
   if (split_pass(c)) {
     const StageAux ax = aux ? *aux : StageAux();
     const dim3 grid(grid_for(c->N * c->B, 64) + 1), block(64 * (c->nv + (ax.dt ? 1 : 0)));
-    if (c->nd == 2)
-      hipLaunchKernelGGL(k_gradlim_split<2>, grid, block, 0, c->stream, U, c->dm, c->gc, c->LG, Gout, Pout, frz, fm,
-                         c->lgB, ax);
-    else
-      hipLaunchKernelGGL(k_gradlim_split<3>, grid, block, 0, c->stream, U, c->dm, c->gc, c->LG, Gout, Pout, frz, fm,
-                         c->lgB, ax);
+    by_mesh(c, [&](auto nd, auto one, auto rc) {
+      (void)one;
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gradlim_split<decltype(nd)::value, decltype(rc)::value>), grid, block, 0,
+                         c->stream, U, c->dm, c->gc, c->LG, Gout, Pout, frz, fm, c->lgB, ax);
+    });
     BES_HIP(hipGetLastError());
     return BES_OK;
   }
   // one condition: the block's packs are staged in LDS
-  const bool one = c->B == 1;
-  const size_t lds = one ? (size_t)bs * c->nv * (c->nd + 1) * sizeof(double) : 0;
-  by_shape(c->nd, one, [&](auto nd, auto one_) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gradlim<decltype(nd)::value, decltype(one_)::value>),
+  const size_t lds = c->B == 1 ? (size_t)bs * c->pw * sizeof(double) : 0;
+  by_mesh(c, [&](auto nd, auto one, auto rc) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gradlim<decltype(nd)::value, decltype(one)::value, decltype(rc)::value>),
                        dim3(nb), dim3(bs), lds, c->stream, U, c->dm, c->LG, Gout, Pout, frz, fm, c->lgB);
   });
   BES_HIP(hipGetLastError());
@@ -1189,17 +1272,16 @@ int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout, cons
 
 // face flux: face records, both cell packs (each pack read once overall), fluxes
 double faceflux_bytes(const bes_ctx *c) {
-  const double F = c->dm.F, N = c->N, B = c->B, nd = c->nd, nv = c->nv;
-  return F * (8 + 24 * nd + 8 * c->fs * B) + N * 8 * nv * (1 + nd) * B;
+  const double F = c->dm.F, N = c->N, B = c->B, nd = c->nd;
+  return F * (8 + (c->common ? 8 : 24) * nd + 8 * c->fs * B) + N * 8 * c->pw * B;
 }
 
 // face fluxes of the current packs (shared with the implicit assembly)
 int launch_face_flux(bes_ctx *c) {
   const int bs = tuned_bs(c, kProfFaceFlux), nb = grid_for(c->dm.F * c->B, bs);
-  const bool one = c->B == 1;
   ProfScope ps(c, kProfFaceFlux, faceflux_bytes(c));
-  by_shape(c->nd, one, [&](auto nd, auto one_) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_face_flux<decltype(nd)::value, decltype(one_)::value>),
+  by_mesh(c, [&](auto nd, auto one, auto rc) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_face_flux<decltype(nd)::value, decltype(one)::value, decltype(rc)::value>),
                        dim3(nb), dim3(bs), 0, c->stream, c->LG, c->dm, c->gc, c->dfinf, c->FF, c->fs, c->err,
                        c->lgB);
   });
@@ -1219,14 +1301,13 @@ double residual_bytes(const bes_ctx *c, bool update, bool rout) {
 int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int local, double *Rout,
                     unsigned long long *linf_bits) {
   const double *dtg = local ? nullptr : c->dtg;
-  const bool one = c->B == 1;
   if (split_pass(c)) {
     // the packs of both sides and the face records per cell face
     ProfScope ps(c, kProfResidual, residual_bytes(c, U0 != nullptr, Rout != nullptr) + faceflux_bytes(c));
-    by_shape(c->nd, one, [&](auto nd, auto one_) {
+    by_mesh(c, [&](auto nd, auto one, auto rc) {
       constexpr int ND = decltype(nd)::value;
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual_faces<ND, decltype(one_)::value>), dim3(grid_for(c->N * c->B, 64)),
-                         dim3(64 * (ND + 2)), 0, c->stream, c->LG, c->dm, c->gc, c->dfinf, U0, Ud, c->dt, dtg, alpha,
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual_faces<ND, decltype(one)::value, decltype(rc)::value>),
+                         dim3(grid_for(c->N * c->B, 64)), dim3(64 * (ND + 2)), 0, c->stream, c->LG, c->dm, c->gc, c->dfinf, U0, Ud, c->dt, dtg, alpha,
                          Rout, linf_bits, c->err, c->lgB);
     });
     BES_HIP(hipGetLastError());
@@ -1236,8 +1317,9 @@ int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int 
   if (s) return s;
   const int bs = tuned_bs(c, kProfResidual), nb = grid_for(c->N * c->B, bs);
   ProfScope ps(c, kProfResidual, residual_bytes(c, U0 != nullptr, Rout != nullptr));
-  by_shape(c->nd, one, [&](auto nd, auto one_) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_residual<decltype(nd)::value, decltype(one_)::value>),
+  by_mesh(c, [&](auto nd, auto one, auto rc) {
+    (void)rc;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_residual<decltype(nd)::value, decltype(one)::value>),
                        dim3(nb), dim3(bs), 0, c->stream, c->FF, c->fs, U0, Ud, c->dt, dtg, alpha, c->dm, Rout,
                        linf_bits, c->lgB);
   });
@@ -1365,8 +1447,9 @@ static int resize_batch(bes_ctx *c, int B) {
   const size_t N = c->N, nv = c->nv, nd = c->nd, Bs = B;
   int s;
   c->fs = B == 1 ? (int)((nv + 1) / 2 * 2) : (int)nv;
+  c->pw = (size_t)(c->common ? c->fs : (int)(nv * (1 + nd)));
   if ((s = dalloc(&c->U0, nv * N * Bs)) || (s = dalloc(&c->Ua, nv * N * Bs)) || (s = dalloc(&c->Ub, nv * N * Bs)) ||
-      (s = dalloc(&c->LG, nv * (1 + nd) * N * Bs)) || (s = dalloc(&c->FF, (size_t)c->fs * c->dm.F * Bs)) ||
+      (s = dalloc(&c->LG, c->pw * N * Bs)) || (s = dalloc(&c->FF, (size_t)c->fs * c->dm.F * Bs)) ||
       (s = dalloc(&c->dt, N * Bs)))
     return s;
   std::vector<double> fb((size_t)B * (nv + 1));
@@ -1435,7 +1518,7 @@ int bes_ctx_destroy(bes_ctx *c) {
   bes_implicit_free(c);
   void *ptrs[] = {c->dm.vol, c->dm.eps2, c->dm.sproj, c->dm.nbr, c->dm.Sg, c->dm.w, c->dm.rl, c->dm.nf,
                   c->dm.af, c->dm.cfd, c->dm.info, c->dm.cfq, c->dm.saq, c->dm.fo, c->dm.fnb, c->dm.fnr,
-                  c->dm.frs, c->dm.frn,
+                  c->dm.frs, c->dm.frn, c->dm.odd_state,
                   c->FF, c->U0, c->Ua, c->Ub, c->LG, c->G, c->phi, c->phi_frz,
                   c->dt, c->dtg, c->R, c->diperm, c->stage, c->red, c->lbits, c->err, c->linf, c->dfinf, c->dit};
   drop_graph(c);
@@ -1730,9 +1813,13 @@ static int explicit_run_persistent(bes_ctx *c, int niter, int nstage, const doub
   CoefB fm;
   for (int b = 0; b < bes_ctx::kMaxBatch; b++)
     fm.c[b] = (b < (int)c->lim_frozen.size() && c->lim_frozen[b]) ? 1.0 : 0.0;
-  const void *fn = c->nd == 2 ? (const void *)k_explicit_persistent<2> : (const void *)k_explicit_persistent<3>;
+  const void *fn = nullptr;
+  by_mesh(c, [&](auto nd, auto one, auto rc) {
+    (void)one;
+    fn = (const void *)k_explicit_persistent<decltype(nd)::value, decltype(rc)::value>;
+  });
   const int bs = 256;
-  const size_t lds = (size_t)bs * c->nv * (c->nd + 1) * sizeof(double);
+  const size_t lds = (size_t)bs * c->pw * sizeof(double);
   int dev = 0, ncu = 0, per_cu = 0;
   BES_HIP(hipGetDevice(&dev));
   BES_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
