@@ -326,16 +326,15 @@ template <int ND, bool ONE, bool RC>
 __global__ __launch_bounds__(256) void k_gradlim(const double *__restrict__ U, DevMesh dm,
                                                     double *__restrict__ PK, double *__restrict__ Gout,
                                                     double *__restrict__ Pout, double *__restrict__ frz,
-                                                    CoefB fmask, int lgB) {
+                                                    CoefB fmask, int lgB, int xcd) {
   extern __shared__ double sm_pack[];
-  const int N = dm.N;
-  const int i0 = blockIdx.x * blockDim.x;   // dispatch order (see k_cell_residual)
-  const int t = i0 + threadIdx.x;
+  const int N = dm.N, blk = xcd ? xcd_block() : blockIdx.x;
+  const int t = blk * blockDim.x + threadIdx.x;
   if constexpr (!ONE) {
     const int B = 1 << lgB, i = t >> lgB, b = t & (B - 1);
     if (i < N) gradlim_cell<ND, false, RC>(U, dm, PK, Gout, Pout, frz, fmask, i, b, B, nullptr);
   } else {
-    gradlim_block_one<ND, RC>(U, dm, PK, Gout, Pout, frz, fmask, blockIdx.x, sm_pack);
+    gradlim_block_one<ND, RC>(U, dm, PK, Gout, Pout, frz, fmask, blk, sm_pack);
   }
 }
 
@@ -455,20 +454,17 @@ __device__ __forceinline__ void face_flux_thread(const double *__restrict__ PK, 
 template <int ND, bool ONE, bool RC>
 __global__ __launch_bounds__(256) void k_face_flux(const double *__restrict__ PK, DevMesh dm, GasConst gc,
                                                    const double *__restrict__ finf, double *__restrict__ FF,
-                                                   int fs, unsigned long long *__restrict__ err, int lgB) {
-  // dispatch order (see k_cell_residual)
-  face_flux_thread<ND, ONE, RC>(PK, dm, gc, finf, FF, fs, err, lgB, blockIdx.x * blockDim.x + threadIdx.x);
+                                                   int fs, unsigned long long *__restrict__ err, int lgB,
+                                                   int xcd) {
+  const int blk = xcd ? xcd_block() : blockIdx.x;
+  face_flux_thread<ND, ONE, RC>(PK, dm, gc, finf, FF, fs, err, lgB, blk * blockDim.x + threadIdx.x);
 }
 
 // One thread per (cell, condition): residual sum_f +-F*A over the cell's faces
 // in the reference face order (SolverExplicit.cpp:325-341), fused with the
 // stage update U = U0 - alpha*dt/V*R (:364-375) and the Linf monitor (:356-362).
 // The faces come pre-sorted in that order with the area negated where the cell
-// is the neighbour (R + x*(-A) is R - x*A exactly).  Blocks run in dispatch
-// order (consecutive blocks on different XCDs): on the 2M-tet box this kernel,
-// the face flux and the gradient took 4%, 2% and 1% less time than with the
-// XCD-contiguous block map of cell_index(), whose shared-L2 reuse of
-// neighbour data does not pay for these gathers.
+// is the neighbour (R + x*(-A) is R - x*A exactly).  Block order: xcd_order.
 // the cells of block blk; every thread of the block must call it (the Linf
 // monitor is a block reduction)
 template <int ND, bool ONE>
@@ -540,8 +536,9 @@ __global__ __launch_bounds__(256) void k_cell_residual(const double *__restrict_
                                                        double *Ud, const double *__restrict__ dt,
                                                        const double *__restrict__ dtg, double alpha, DevMesh dm,
                                                        double *__restrict__ Rout,
-                                                       unsigned long long *__restrict__ linf_bits, int lgB) {
-  cell_residual_block<ND, ONE>(FF, fs, U0, Ud, dt, dtg, alpha, dm, Rout, linf_bits, lgB, blockIdx.x);
+                                                       unsigned long long *__restrict__ linf_bits, int lgB, int xcd) {
+  cell_residual_block<ND, ONE>(FF, fs, U0, Ud, dt, dtg, alpha, dm, Rout, linf_bits, lgB,
+                               xcd ? xcd_block() : blockIdx.x);
 }
 
 __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v) {
@@ -1234,11 +1231,19 @@ double gradlim_bytes(const bes_ctx *c) {
 
 // Up to this many (cell, condition) units a pass is bound by the length of a
 // thread's chain and by launches, and the split forms are taken.  RK4 step as a
-// graph, split against per-pass kernels: 3k triangles 41 / 71 us, 40k 62 / 86,
-// 102k 108 / 116, 160k 143 / 143; tetrahedra 3k 49 / 91, 48k 102 / 126, 64k
-// 130 / 134, 94k 176 / 168; 64 conditions x 1,200 triangles 71 / 114, 32
-// conditions x 3,840 tetrahedra 201 / 154.
-static bool split_pass(const bes_ctx *c) { return (long)c->N * c->B <= (c->nd == 2 ? 131072 : 65536); }
+// graph in us, split against per-pass kernels: 40k triangles 54 / 71, 90k 80 /
+// 97, 160k 112 / 123, 250k 152 / 154, 360k 200 / 192; tetrahedra 25k 60 / 88,
+// 48k 80 / 105, 83k 122 / 138, 105k 147 / 150, 132k 171 / 178, 179k 215 / 192;
+// batches: 8 x 10k tetrahedra 119 / 121, 32 x 3k 128 / 123, 64 x 2.4k triangles
+// 105 / 111, 64 x 4k 148 / 138.
+static bool split_pass(const bes_ctx *c) { return (long)c->N * c->B <= (c->nd == 2 ? 196608 : 90112); }
+
+// Block order of the per-pass kernels: up to this many units each XCD takes one
+// range of cells in every pass, so part of what a pass reads is still in its L2
+// (RK4 step: 360k triangles 208 -> 192 us, 444k tetrahedra 391 -> 372, 750k 637 ->
+// 625, 64 conditions x 10k 404 -> 384).  Past it dispatch order, which spreads
+// neighbouring cells over the XCDs: 2M tetrahedra 1594 us against 1608.
+static int xcd_order(const bes_ctx *c) { return (long)c->N * c->B <= (1 << 20); }
 
 // one thread per (cell, condition), or per (cell, condition, variable); aux is
 // for the split form only
@@ -1264,7 +1269,8 @@ int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout, cons
   const size_t lds = c->B == 1 ? (size_t)bs * c->pw * sizeof(double) : 0;
   by_mesh(c, [&](auto nd, auto one, auto rc) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_gradlim<decltype(nd)::value, decltype(one)::value, decltype(rc)::value>),
-                       dim3(nb), dim3(bs), lds, c->stream, U, c->dm, c->LG, Gout, Pout, frz, fm, c->lgB);
+                       dim3(nb), dim3(bs), lds, c->stream, U, c->dm, c->LG, Gout, Pout, frz, fm, c->lgB,
+                       xcd_order(c));
   });
   BES_HIP(hipGetLastError());
   return BES_OK;
@@ -1283,7 +1289,7 @@ int launch_face_flux(bes_ctx *c) {
   by_mesh(c, [&](auto nd, auto one, auto rc) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_face_flux<decltype(nd)::value, decltype(one)::value, decltype(rc)::value>),
                        dim3(nb), dim3(bs), 0, c->stream, c->LG, c->dm, c->gc, c->dfinf, c->FF, c->fs, c->err,
-                       c->lgB);
+                       c->lgB, xcd_order(c));
   });
   BES_HIP(hipGetLastError());
   return BES_OK;
@@ -1321,7 +1327,7 @@ int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int 
     (void)rc;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cell_residual<decltype(nd)::value, decltype(one)::value>),
                        dim3(nb), dim3(bs), 0, c->stream, c->FF, c->fs, U0, Ud, c->dt, dtg, alpha, c->dm, Rout,
-                       linf_bits, c->lgB);
+                       linf_bits, c->lgB, xcd_order(c));
   });
   BES_HIP(hipGetLastError());
   return BES_OK;

@@ -1,5 +1,5 @@
 """The two forms of the explicit passes, at the sizes where the dispatch changes
-(131,072 cell-conditions in 2D, 65,536 in 3D) and at the edges of their blocks, against the CPU
+(196,608 cell-conditions in 2D, 90,112 in 3D) and at the edges of their blocks, against the CPU
 oracle and against each condition's own run, bit for bit."""
 import numpy as np
 import pytest
@@ -22,7 +22,7 @@ def _case(md, seed=2):
 # fewer cells than a block's 64, one block, one past it, ragged; the last size of
 # the split form and the first of the other, in 2D and 3D
 @pytest.mark.parametrize("mesh", [("bump", 5, 4), ("bump", 8, 4), ("bump", 11, 3), ("box", 4, 3, 3), ("box", 5, 5, 3),
-                                  ("bump", 256, 256), ("bump", 331, 199), ("box", 21, 21, 24), ("box", 22, 22, 23)])
+                                  ("bump", 384, 256), ("bump", 331, 299), ("box", 25, 24, 25), ("box", 25, 25, 25)])
 @pytest.mark.parametrize("graph", [False, True])
 def test_steps_equal_the_oracle(mesh, graph):
     md = _mesh(*mesh)
@@ -64,8 +64,8 @@ def test_one_stage_and_global_steps(alpha, local):
 
 
 # batches on both sides of the line; frozen limiter values in one condition's place
-@pytest.mark.parametrize("mesh,B", [(("bump", 9, 4), 2), (("box", 4, 4, 3), 8), (("bump", 32, 32), 64),
-                                    (("bump", 33, 32), 64), (("box", 12, 12, 10), 8)])
+@pytest.mark.parametrize("mesh,B", [(("bump", 9, 4), 2), (("box", 4, 4, 3), 8), (("bump", 48, 32), 64),
+                                    (("bump", 49, 32), 64), (("box", 12, 12, 14), 8)])
 def test_batch_equals_single_runs(mesh, B):
     md = _mesh(*mesh)
     PU = [_case(md, 10 + q) for q in range(B)]
