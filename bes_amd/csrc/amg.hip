@@ -77,9 +77,16 @@ struct Level {
   int *agg = nullptr;       // [n] aggregate (= next-level row), -1 removed
   unsigned char *state = nullptr;   // [n] final State of the row
   int *mptr = nullptr, *mem = nullptr;   // members of next-level row I: mem[mptr[I] .. mptr[I+1]), ascending
-  // FP32 solves, coarse levels: row-scaled FP16 copy of val for the sweeps
+  // FP32 solves, coarse levels: row-scaled FP16 copy of val for the sweeps, in
+  // CSR order (hval) or, on large levels, in slices (k_sliced)
   __half *hval = nullptr;
   float *hrm = nullptr;
+  __half2 *sval = nullptr;  // [block][NP][64] entry pairs
+  int *scol = nullptr;      // [block][64] columns
+  int *soff = nullptr;      // [nslice + 1] first block of a slice
+  int *srow = nullptr;      // [nslice][64] rows, -1 past the end
+  void *sw = nullptr;       // [nslice][nv*nv or nv][64] relaxation data (matrix type)
+  int nslice = 0;
 };
 
 struct Amg {
@@ -103,7 +110,8 @@ struct Amg {
   void *t0 = nullptr;       // level-0 residual (vector type)
   // FP32 solves: row-scaled FP16 copies of the level-0 matrix and relaxation
   // data for the cycle (the hierarchy is built from the full-precision matrix)
-  __half *Ah = nullptr, *Wh = nullptr;
+  // (entry pairs, [(K+1)][NP][N] and [WP][N])
+  __half2 *Ah = nullptr, *Wh = nullptr;
   float *rm = nullptr;      // [N] row scale m_i: A_i = m_i Ah_i, W_i = Wh_i / m_i
   std::vector<void *> owned;     // allocations outside the arena
   void *arena = nullptr;
@@ -133,19 +141,15 @@ struct EllAcc {
   __device__ int back(int i, int q, int) const { return 1 + mrev[(size_t)(q - 1) * N + i]; }
 };
 
-// level 0 from the row-scaled FP16 copy (cycle only)
+// level 0 from the row-scaled FP16 copy (cycle only): entries 2p and 2p + 1 of
+// block q of row i at A[(q*NP + p)*N + i] (the last one padded with 0)
 template <int NV>
 struct EllAccH {
-  static constexpr int NB = NV * NV;
-  const __half *A;
+  static constexpr int NP = (NV * NV + 1) / 2;
+  const __half2 *A;
   const float *rm;
   const int *nbr;
-  int N, K;
-  __device__ int len(int) const { return K + 1; }
-  __device__ int col(int i, int q) const { return q == 0 ? i : nbr[(size_t)(q - 1) * N + i]; }
-  __device__ double v(int i, int q, int e) const {
-    return (double)__half2float(A[((size_t)q * NB + e) * N + i]) * (double)rm[i];
-  }
+  int N;
 };
 
 template <typename TM, int NV>
@@ -688,6 +692,33 @@ __device__ __forceinline__ void relax_apply(const TW *__restrict__ w, const floa
   }
 }
 
+// the same from entry pairs [WP][N] (level 0's FP16 copy)
+template <int NV, int KIND>
+__device__ __forceinline__ void relax_apply(const __half2 *__restrict__ w, const float *__restrict__ ws, int i, int N,
+                                            const double *t, double *d) {
+  constexpr int WN = KIND == kBlockJacobi ? NV * NV : NV, WP = (WN + 1) / 2;
+  float v[2 * WP];
+#pragma unroll
+  for (int p = 0; p < WP; p++) {
+    const float2 h = __half22float2(w[(size_t)p * N + i]);
+    v[2 * p] = h.x;
+    v[2 * p + 1] = h.y;
+  }
+  const double inv = 1.0 / (double)ws[i];
+#pragma unroll
+  for (int r = 0; r < NV; r++) {
+    if (KIND == kBlockJacobi) {
+      double s = 0;
+#pragma unroll
+      for (int c = 0; c < NV; c++) s += (double)v[r * NV + c] * t[c];
+      d[r] = s;
+    } else {
+      d[r] = (double)v[r] * t[r];
+    }
+    d[r] *= inv;
+  }
+}
+
 // x = W f (one sweep from x = 0)
 template <int NV, int KIND, typename TW, typename TV>
 __global__ __launch_bounds__(256) void k_relax0(int n, const TW *__restrict__ w, const float *__restrict__ ws,
@@ -697,6 +728,17 @@ __global__ __launch_bounds__(256) void k_relax0(int n, const TW *__restrict__ w,
   double t[NV], d[NV];
   for (int r = 0; r < NV; r++) t[r] = (double)f[(size_t)i * NV + r];
   relax_apply<NV, KIND>(w, ws, i, t, d);
+  for (int r = 0; r < NV; r++) x[(size_t)i * NV + r] = (TV)d[r];
+}
+
+template <int NV, int KIND, typename TV>
+__global__ __launch_bounds__(256) void k_relax0_h(int n, const __half2 *__restrict__ w, const float *__restrict__ ws,
+                                                  const TV *__restrict__ f, TV *__restrict__ x) {
+  const int i = row_index();
+  if (i >= n) return;
+  double t[NV], d[NV];
+  for (int r = 0; r < NV; r++) t[r] = (double)f[(size_t)i * NV + r];
+  relax_apply<NV, KIND>(w, ws, i, n, t, d);
   for (int r = 0; r < NV; r++) x[(size_t)i * NV + r] = (TV)d[r];
 }
 
@@ -713,6 +755,43 @@ __device__ __forceinline__ void row_resid(const Acc &a, int i, const TV *__restr
     for (int r = 0; r < NV; r++) {
       double s = 0;
       for (int c = 0; c < NV; c++) s += a.v(i, q, r * NV + c) * xj[c];
+      t[r] -= s;
+    }
+  }
+}
+
+// the row of level 0's FP16 copy (NV blocks: the diagonal and NV - 1 faces): all
+// columns first, then every block's entry pairs and x, so that a row waits for
+// memory twice and not once per block
+template <int NV, typename TV>
+__device__ __forceinline__ void row_resid(const EllAccH<NV> &a, int i, const TV *__restrict__ f,
+                                          const TV *__restrict__ x, double *t) {
+  constexpr int NP = EllAccH<NV>::NP;
+  int j[NV];
+  j[0] = i;
+#pragma unroll
+  for (int q = 1; q < NV; q++) j[q] = a.nbr[(size_t)(q - 1) * a.N + i];
+  const double rm = (double)a.rm[i];
+#pragma unroll
+  for (int r = 0; r < NV; r++) t[r] = (double)f[(size_t)i * NV + r];
+#pragma unroll
+  for (int q = 0; q < NV; q++) {
+    if (j[q] < 0) continue;
+    float v[2 * NP];
+    double xj[NV];
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const float2 h = __half22float2(a.A[((size_t)q * NP + p) * a.N + i]);
+      v[2 * p] = h.x;
+      v[2 * p + 1] = h.y;
+    }
+#pragma unroll
+    for (int c = 0; c < NV; c++) xj[c] = (double)x[(size_t)j[q] * NV + c];
+#pragma unroll
+    for (int r = 0; r < NV; r++) {
+      double s = 0;
+#pragma unroll
+      for (int c = 0; c < NV; c++) s += ((double)v[r * NV + c] * rm) * xj[c];
       t[r] -= s;
     }
   }
@@ -742,13 +821,28 @@ __global__ __launch_bounds__(256) void k_relax(Acc a, int n, const TW *__restric
   for (int r = 0; r < NV; r++) xout[(size_t)i * NV + r] = (TV)((double)xin[(size_t)i * NV + r] + d[r]);
 }
 
+// x + W (f - A x) on level 0's FP16 copies
+template <int NV, int KIND, typename TV>
+__global__ __launch_bounds__(256) void k_relax_h(EllAccH<NV> a, int n, const __half2 *__restrict__ w,
+                                                 const TV *__restrict__ f, const TV *__restrict__ xin,
+                                                 TV *__restrict__ xout) {
+  const int i = row_index();
+  if (i >= n) return;
+  double t[NV], d[NV];
+  row_resid<NV>(a, i, f, xin, t);
+  relax_apply<NV, KIND>(w, a.rm, i, n, t, d);
+  for (int r = 0; r < NV; r++) xout[(size_t)i * NV + r] = (TV)((double)xin[(size_t)i * NV + r] + d[r]);
+}
+
 // row-scaled FP16 copies of the level-0 matrix and relaxation data: m_i is the
-// largest |entry| of the diagonal block; Ah = A_i / m_i, Wh = W_i m_i
+// largest |entry| of the diagonal block; Ah = A_i / m_i, Wh = W_i m_i, in entry
+// pairs (4-byte loads in the sweeps: 486k tetrahedra, residual 43 us with
+// 2-byte loads block by block)
 template <int NV, typename TM>
 __global__ __launch_bounds__(256) void k_half_copy(const TM *__restrict__ A, const TM *__restrict__ W, int N, int K,
-                                                   int wper, __half *__restrict__ Ah, __half *__restrict__ Wh,
+                                                   int wper, __half2 *__restrict__ Ah, __half2 *__restrict__ Wh,
                                                    float *__restrict__ rm, int *__restrict__ err) {
-  constexpr int NB = NV * NV;
+  constexpr int NB = NV * NV, NP = (NB + 1) / 2;
   const int i = row_index();
   if (i >= N) return;
   double m = 0;
@@ -759,15 +853,24 @@ __global__ __launch_bounds__(256) void k_half_copy(const TM *__restrict__ A, con
   const double inv = 1.0 / (double)mf;
   bool ok = true;
   for (int q = 0; q <= K; q++)
-    for (int e = 0; e < NB; e++) {
-      const float v = (float)(to_d(A[((size_t)q * NB + e) * N + i]) * inv);
-      ok &= fabsf(v) < 65000.0f;
-      Ah[((size_t)q * NB + e) * N + i] = __float2half(v);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      float v[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        v[u] = 2 * p + u < NB ? (float)(to_d(A[((size_t)q * NB + 2 * p + u) * N + i]) * inv) : 0.0f;
+        ok &= fabsf(v[u]) < 65000.0f;
+      }
+      Ah[((size_t)q * NP + p) * N + i] = __floats2half2_rn(v[0], v[1]);
     }
-  for (int e = 0; e < wper; e++) {
-    const float v = (float)(to_d(W[(size_t)i * wper + e]) * (double)mf);
-    ok &= fabsf(v) < 65000.0f;
-    Wh[(size_t)i * wper + e] = __float2half(v);
+  for (int p = 0; p < (wper + 1) / 2; p++) {
+    _Float16 v[2];   // W_i m_i rounded once (the product of two FP32 values is exact in FP64)
+    for (int u = 0; u < 2; u++) {
+      const double x = 2 * p + u < wper ? to_d(W[(size_t)i * wper + 2 * p + u]) * (double)mf : 0.0;
+      ok &= fabs(x) < 65000.0;
+      v[u] = (_Float16)x;
+    }
+    Wh[(size_t)p * N + i] = __halves2half2(__half(v[0]), __half(v[1]));
   }
   if (!ok) atomicOr(err, 16);
 }
@@ -874,27 +977,168 @@ __global__ __launch_bounds__(256) void k_restrict(int nc, const int *__restrict_
 }
 
 // row-scaled FP16 sweep copy of a coarse level: rm_i = largest |entry| of the
-// diagonal block, hval = val / rm_i (err |= 64 when out of FP16 range)
+// diagonal block, hval = val / rm_i (err |= 64 when out of FP16 range); 32 lanes
+// per row, lane e entry e of every block (a thread per row read 100 bytes apart
+// and ran one chain per row: 220-290 us on levels of 600 to 74k rows)
 template <int NV, typename TM>
 __global__ __launch_bounds__(256) void k_half_csr(int n, const int *__restrict__ rp, const int *__restrict__ dpos,
                                                   const TM *__restrict__ val, __half *__restrict__ hval,
                                                   float *__restrict__ rm, int *__restrict__ err) {
   constexpr int NB = NV * NV;
-  const int i = row_index();
-  if (i >= n) return;
-  double m = 0;
-  for (int e = 0; e < NB; e++) m = fmax(m, fabs(to_d(val[(size_t)(rp[i] + dpos[i]) * NB + e])));
+  const int i = (blockIdx.x * 256 + threadIdx.x) >> 5, l = threadIdx.x & 31;
+  if (i >= n) return;   // whole 32-lane groups
+  const size_t p0 = rp[i], p1 = rp[i + 1];
+  double m = l < NB ? fabs(to_d(val[(p0 + dpos[i]) * NB + l])) : 0.0;
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 32));
   if (!(m > 0)) m = 1.0;
   const float mf = (float)m;
-  rm[i] = mf;
+  if (l == 0) rm[i] = mf;
+  if (l >= NB) return;
   const double inv = 1.0 / (double)mf;
   bool ok = true;
-  for (size_t k = (size_t)rp[i] * NB; k < (size_t)rp[i + 1] * NB; k++) {
-    const float v = (float)(to_d(val[k]) * inv);
+#pragma unroll 4
+  for (size_t k = p0; k < p1; k++) {
+    const float v = (float)(to_d(val[k * NB + l]) * inv);
     ok &= fabsf(v) < 65000.0f;
-    hval[k] = __float2half(v);
+    hval[k * NB + l] = __float2half(v);
   }
   if (!ok) atomicOr(err, 64);
+}
+
+// ---- sliced sweep copy of a large coarse level ----
+// Windows of 1024 rows are sorted by their number of blocks (descending, stable)
+// and cut into slices of 64 rows; a slice stores as many blocks per row as its
+// longest row has, entry pairs and columns lane-interleaved, so a wave sweeps 64
+// rows with coalesced 4-byte loads.  The 32-lanes-per-row form issues about ten
+// times the instructions per block (one entry a lane, a shuffle per column) and
+// was bound by that: 74k rows with 693k blocks took 38 us a residual, 35 MB.
+constexpr int kSlicedRows = 16384;   // levels from this size on
+constexpr int kWindow = 1024;
+
+__global__ __launch_bounds__(kWindow) void k_slice_sort(int n, const int *__restrict__ rp, int *__restrict__ srow,
+                                                        int *__restrict__ width) {
+  __shared__ int len[kWindow];
+  const int t = threadIdx.x, i = blockIdx.x * kWindow + t;
+  const int my = i < n ? rp[i + 1] - rp[i] : -1;
+  len[t] = my;
+  __syncthreads();
+  int rank = 0;
+  for (int y = 0; y < kWindow; y++) rank += len[y] > my || (len[y] == my && y < t);
+  srow[blockIdx.x * kWindow + rank] = i < n ? i : -1;
+  if ((rank & 63) == 0) width[(blockIdx.x * kWindow + rank) >> 6] = max(my, 0);
+}
+
+template <int NV, typename TM>
+__global__ __launch_bounds__(256) void k_slice_fill(int nslice, int wper, const int *__restrict__ rp,
+                                                    const int *__restrict__ cl, const int *__restrict__ dpos,
+                                                    const TM *__restrict__ val, const TM *__restrict__ w,
+                                                    const int *__restrict__ srow, const int *__restrict__ soff,
+                                                    __half2 *__restrict__ sval, int *__restrict__ scol,
+                                                    float *__restrict__ rm, TM *__restrict__ sw,
+                                                    int *__restrict__ err) {
+  constexpr int NB = NV * NV, NP = (NB + 1) / 2;
+  const int s = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (s >= nslice) return;
+  const int i = srow[(size_t)s * 64 + l];
+  const int b0 = soff[s], nb = soff[s + 1] - b0;
+  const int p0 = i >= 0 ? rp[i] : 0, len = i >= 0 ? rp[i + 1] - p0 : 0;
+  double m = 0;
+  if (i >= 0)
+    for (int e = 0; e < NB; e++) m = fmax(m, fabs(to_d(val[(size_t)(p0 + dpos[i]) * NB + e])));
+  if (!(m > 0)) m = 1.0;
+  const float mf = (float)m;
+  const double inv = 1.0 / (double)mf;
+  bool ok = true;
+  if (i >= 0) rm[i] = mf;
+  for (int k = 0; k < nb; k++) {   // blocks past the row's own: zeros on its first column
+    const bool in = k < len;
+    const size_t src = (size_t)(p0 + (in ? k : 0));
+    scol[(size_t)(b0 + k) * 64 + l] = len > 0 ? cl[src] : 0;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      float v[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        v[u] = in && 2 * p + u < NB ? (float)(to_d(val[src * NB + 2 * p + u]) * inv) : 0.0f;
+        ok &= fabsf(v[u]) < 65000.0f;
+      }
+      sval[((size_t)(b0 + k) * NP + p) * 64 + l] = __floats2half2_rn(v[0], v[1]);
+    }
+  }
+  for (int e = 0; e < wper; e++)
+    sw[((size_t)s * wper + e) * 64 + l] = i >= 0 ? w[(size_t)i * wper + e] : (TM)0;
+  if (!ok) atomicOr(err, 64);
+}
+
+// k_csr_group's sweep on the sliced copy, a thread per row: entry (r, c) of the
+// row's blocks is summed over the blocks in column order, then over c, as there.
+template <int NV, int KIND, int RELAX, typename TM, typename TV>
+__global__ __launch_bounds__(256) void k_sliced(int nslice, const int *__restrict__ srow,
+                                                const int *__restrict__ soff, const int *__restrict__ scol,
+                                                const __half2 *__restrict__ sval, const float *__restrict__ rm,
+                                                const TM *__restrict__ sw, const TV *__restrict__ f,
+                                                const TV *__restrict__ x, TV *__restrict__ out) {
+  constexpr int NB = NV * NV, NP = (NB + 1) / 2, U = 2;
+  const int s = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (s >= nslice) return;
+  const int i = srow[(size_t)s * 64 + l];
+  const int b0 = soff[s], nb = soff[s + 1] - b0;
+  double acc[NB];
+#pragma unroll
+  for (int e = 0; e < NB; e++) acc[e] = 0;
+  int J[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) J[u] = u < nb ? scol[(size_t)(b0 + u) * 64 + l] : 0;
+  for (int k = 0; k < nb; k += U) {   // U blocks and the next columns in flight
+    __half2 v[U][NP];
+    TV xv[U][NV];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const size_t b = (size_t)(b0 + (k + u < nb ? k + u : k));
+#pragma unroll
+      for (int p = 0; p < NP; p++) v[u][p] = sval[(b * NP + p) * 64 + l];
+#pragma unroll
+      for (int c = 0; c < NV; c++) xv[u][c] = x[(size_t)J[u] * NV + c];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) J[u] = k + U + u < nb ? scol[(size_t)(b0 + k + U + u) * 64 + l] : 0;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k + u >= nb) break;
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        const float2 h = __half22float2(v[u][p]);
+        acc[2 * p] += (double)h.x * (double)xv[u][(2 * p) % NV];
+        if (2 * p + 1 < NB) acc[2 * p + 1] += (double)h.y * (double)xv[u][(2 * p + 1) % NV];
+      }
+    }
+  }
+  if (i < 0) return;
+  double t[NV];
+#pragma unroll
+  for (int r = 0; r < NV; r++) {
+    double q = 0;
+#pragma unroll
+    for (int c = 0; c < NV; c++) q += acc[r * NV + c];
+    q *= (double)rm[i];
+    t[r] = (double)f[(size_t)i * NV + r] - q;
+  }
+#pragma unroll
+  for (int r = 0; r < NV; r++) {
+    if (RELAX == 0) {
+      out[(size_t)i * NV + r] = (TV)t[r];
+      continue;
+    }
+    double d = 0;
+    if (KIND == kBlockJacobi) {
+#pragma unroll
+      for (int c = 0; c < NV; c++) d += to_d(sw[((size_t)s * NB + r * NV + c) * 64 + l]) * t[c];
+    } else {
+      d = to_d(sw[((size_t)s * NV + r) * 64 + l]) * t[r];
+    }
+    out[(size_t)i * NV + r] = (TV)((double)x[(size_t)i * NV + r] + d);
+  }
 }
 
 template <int NV, typename TV>
@@ -1234,6 +1478,34 @@ static CsrAcc<TM, NV> csr(const Level &L) {
   return CsrAcc<TM, NV>{L.rp, L.col, L.dpos, (const TM *)L.val};
 }
 
+// the sliced FP16 copy of a coarse level
+template <int NV, typename TM>
+static int sliced_copy(bes_ctx *c, Amg *g, Level &L) {
+  constexpr int NP = (NV * NV + 1) / 2;
+  const int nwin = blocks_for(L.n, kWindow), wper = g->prm.relax == kBlockJacobi ? NV * NV : NV;
+  L.nslice = nwin * (kWindow / 64);
+  int s;
+  if ((s = dmalloc(g, (void **)&L.srow, (size_t)L.nslice * 64 * sizeof(int))) ||
+      (s = dmalloc(g, (void **)&L.soff, (size_t)(L.nslice + 1) * sizeof(int))) ||
+      (s = dmalloc(g, &L.sw, (size_t)L.nslice * wper * 64 * sizeof(TM))))
+    return s;
+  // g->ibuf (level-0 rows + 1 ints) has room for the widths: a slice is 64 rows,
+  // and at most 15 more than the rows fill
+  hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, c->stream, g->ibuf + L.nslice, 1L, 0);
+  hipLaunchKernelGGL(k_slice_sort, dim3(nwin), dim3(kWindow), 0, c->stream, L.n, L.rp, L.srow, g->ibuf);
+  BES_HIP(hipGetLastError());
+  long nblk = 0;
+  if ((s = scan_ex(c, g, g->ibuf, L.soff, L.nslice + 1, 0, &nblk))) return s;
+  if ((s = dmalloc(g, (void **)&L.sval, (size_t)nblk * NP * 64 * sizeof(__half2))) ||
+      (s = dmalloc(g, (void **)&L.scol, (size_t)nblk * 64 * sizeof(int))))
+    return s;
+  hipLaunchKernelGGL((k_slice_fill<NV, TM>), dim3(blocks_for(L.nslice, 4)), dim3(256), 0, c->stream, L.nslice, wper,
+                     L.rp, L.col, L.dpos, (const TM *)L.val, (const TM *)L.w, L.srow, L.soff, L.sval, L.scol, L.hrm,
+                     (TM *)L.sw, g->flags + 1);
+  BES_HIP(hipGetLastError());
+  return BES_OK;
+}
+
 template <int NV, typename TM>
 static int build_t(bes_ctx *c, Impl *im, Amg *g) {
   const int N = c->N, K = c->k;
@@ -1278,8 +1550,8 @@ static int build_t(bes_ctx *c, Impl *im, Amg *g) {
     if (s) return s;
     if (l == 0 && im->prec == 32) {
       const int wper = g->prm.relax == kBlockJacobi ? NV * NV : NV;
-      if ((s = dmalloc(g, (void **)&g->Ah, (size_t)(K + 1) * NV * NV * N * sizeof(__half))) ||
-          (s = dmalloc(g, (void **)&g->Wh, (size_t)N * wper * sizeof(__half))) ||
+      if ((s = dmalloc(g, (void **)&g->Ah, (size_t)(K + 1) * EllAccH<NV>::NP * N * sizeof(__half2))) ||
+          (s = dmalloc(g, (void **)&g->Wh, (size_t)N * ((wper + 1) / 2) * sizeof(__half2))) ||
           (s = dmalloc(g, (void **)&g->rm, (size_t)N * sizeof(float))))
         return s;
       hipLaunchKernelGGL((k_half_copy<NV, TM>), dim3(blocks_for(N, 256)), dim3(256), 0, c->stream,
@@ -1310,15 +1582,20 @@ static int build_t(bes_ctx *c, Impl *im, Amg *g) {
     for (int l = 1; l < g->nlev; l++) {
       if (l == g->nlev - 1 && g->direct) break;   // the coarsest is applied as a dense inverse
       Level &Lh = g->lv[l];
-      if ((s = dmalloc(g, (void **)&Lh.hval, (size_t)Lh.nnzb * NV * NV * sizeof(__half))) ||
-          (s = dmalloc(g, (void **)&Lh.hrm, (size_t)Lh.n * sizeof(float))))
-        return s;
-      hipLaunchKernelGGL((k_half_csr<NV, TM>), dim3(blocks_for(Lh.n, 256)), dim3(256), 0, c->stream, Lh.n, Lh.rp,
-                         Lh.dpos, (const TM *)Lh.val, Lh.hval, Lh.hrm, g->flags + 1);
+      if ((s = dmalloc(g, (void **)&Lh.hrm, (size_t)Lh.n * sizeof(float)))) return s;
+      if (Lh.n >= kSlicedRows) {
+        if ((s = sliced_copy<NV, TM>(c, g, Lh))) return s;
+      } else {
+        if ((s = dmalloc(g, (void **)&Lh.hval, (size_t)Lh.nnzb * NV * NV * sizeof(__half)))) return s;
+        hipLaunchKernelGGL((k_half_csr<NV, TM>), dim3(blocks_for((long)Lh.n * 32, 256)), dim3(256), 0, c->stream, Lh.n,
+                           Lh.rp, Lh.dpos, (const TM *)Lh.val, Lh.hval, Lh.hrm, g->flags + 1);
+        BES_HIP(hipGetLastError());
+      }
       int hf[3];
       if ((s = read_flags(c, g, hf))) return s;
       if (hf[1] & 64) {   // out of FP16 range: this level sweeps its full-precision values
         Lh.hval = nullptr;
+        Lh.sval = nullptr;
         Lh.hrm = nullptr;
         hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, c->stream, g->flags + 1, 1L, hf[1] & ~64);
       }
@@ -1371,8 +1648,14 @@ static void launch_relax0_t(bes_ctx *c, int kind, int n, const TW *w, const floa
 template <int NV, typename TM, typename TV>
 static void launch_relax0(bes_ctx *c, Amg *g, int l, const TV *f, TV *x) {
   const Level &L = g->lv[l];
-  if (l == 0 && g->Ah) launch_relax0_t<NV, __half, TV>(c, g->prm.relax, L.n, g->Wh, g->rm, f, x);
-  else launch_relax0_t<NV, TM, TV>(c, g->prm.relax, L.n, (const TM *)L.w, nullptr, f, x);
+  if (l == 0 && g->Ah) {
+    if (g->prm.relax == kBlockJacobi)
+      hipLaunchKernelGGL((k_relax0_h<NV, kBlockJacobi, TV>), dim3(blocks_for(L.n, 256)), dim3(256), 0, c->stream, L.n,
+                         g->Wh, g->rm, f, x);
+    else
+      hipLaunchKernelGGL((k_relax0_h<NV, kJacobi, TV>), dim3(blocks_for(L.n, 256)), dim3(256), 0, c->stream, L.n,
+                         g->Wh, g->rm, f, x);
+  } else launch_relax0_t<NV, TM, TV>(c, g->prm.relax, L.n, (const TM *)L.w, nullptr, f, x);
 }
 
 template <int NV, typename Acc, typename TW, typename TV>
@@ -1411,11 +1694,30 @@ static void launch_sweep(bes_ctx *c, Impl *im, Amg *g, int l, bool relax, const 
   const int n = L.n, kind = g->prm.relax;
   const TM *w = (const TM *)L.w;
   if (l == 0) {
-    if (g->Ah)
-      launch_ell_sweep<NV>(c, kind, EllAccH<NV>{g->Ah, g->rm, c->dm.nbr, c->N, c->k}, n, relax,
-                           (const __half *)g->Wh, (const float *)g->rm, f, x, out);
-    else
+    if (g->Ah) {
+      const EllAccH<NV> a{g->Ah, g->rm, c->dm.nbr, c->N};
+      const dim3 nb(blocks_for(n, 256));
+      if (!relax)
+        hipLaunchKernelGGL((k_resid_lv<NV, EllAccH<NV>, TV>), nb, dim3(256), 0, c->stream, a, n, f, x, out);
+      else if (kind == kBlockJacobi)
+        hipLaunchKernelGGL((k_relax_h<NV, kBlockJacobi, TV>), nb, dim3(256), 0, c->stream, a, n, g->Wh, f, x, out);
+      else
+        hipLaunchKernelGGL((k_relax_h<NV, kJacobi, TV>), nb, dim3(256), 0, c->stream, a, n, g->Wh, f, x, out);
+    } else
       launch_ell_sweep<NV>(c, kind, ell<NV, TM>(c, im), n, relax, w, (const float *)nullptr, f, x, out);
+    return;
+  }
+  if (L.sval) {
+    const dim3 nb(blocks_for(L.nslice, 4));
+    if (!relax)
+      hipLaunchKernelGGL((k_sliced<NV, kJacobi, 0, TM, TV>), nb, dim3(256), 0, c->stream, L.nslice, L.srow, L.soff,
+                         L.scol, L.sval, L.hrm, (const TM *)L.sw, f, x, out);
+    else if (kind == kBlockJacobi)
+      hipLaunchKernelGGL((k_sliced<NV, kBlockJacobi, 1, TM, TV>), nb, dim3(256), 0, c->stream, L.nslice, L.srow,
+                         L.soff, L.scol, L.sval, L.hrm, (const TM *)L.sw, f, x, out);
+    else
+      hipLaunchKernelGGL((k_sliced<NV, kJacobi, 1, TM, TV>), nb, dim3(256), 0, c->stream, L.nslice, L.srow, L.soff,
+                         L.scol, L.sval, L.hrm, (const TM *)L.sw, f, x, out);
     return;
   }
   if (L.hval) launch_csr_sweep<NV>(c, kind, L, relax, (const __half *)L.hval, L.hrm, w, f, x, out);
@@ -1458,7 +1760,7 @@ static double level_bytes(const Amg *g, int nv, size_t es_m, size_t es_v) {
   for (int l = 0; l < g->nlev; l++) {
     const Level &L = g->lv[l];
     const double per = g->prm.relax == kBlockJacobi ? nv * nv : nv;
-    const double em = ((l == 0 && g->Ah) || (l > 0 && L.hval)) ? 2.0 : (double)es_m;
+    const double em = ((l == 0 && g->Ah) || (l > 0 && (L.hval || L.sval))) ? 2.0 : (double)es_m;
     b += 2.0 * L.nnzb * nv * nv * em + 2.0 * L.n * per * em + 8.0 * L.n * nv * es_v;
   }
   if (g->direct) b += (double)g->ndense * g->ndense * 8.0;
