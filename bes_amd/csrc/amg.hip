@@ -99,7 +99,8 @@ struct Amg {
   int nlev = 0;
   bool direct = false;
   int ndense = 0;           // scalar rows of the coarsest system when direct
-  double *dense = nullptr, *dense2 = nullptr, *inv = nullptr;
+  double *dense = nullptr, *dense2 = nullptr, *inv = nullptr;   // [A | I], multipliers of its elimination, inverse
+  int *gjpiv = nullptr;     // pivot rows
   // scratch sized for level 0
   double *s = nullptr, *dia = nullptr;
   unsigned char *strong = nullptr, *sym = nullptr, *near = nullptr;
@@ -836,8 +837,8 @@ __global__ __launch_bounds__(256) void k_relax_h(EllAccH<NV> a, int n, const __h
 
 // row-scaled FP16 copies of the level-0 matrix and relaxation data: m_i is the
 // largest |entry| of the diagonal block; Ah = A_i / m_i, Wh = W_i m_i, in entry
-// pairs (4-byte loads in the sweeps: 486k tetrahedra, residual 43 us with
-// 2-byte loads block by block)
+// pairs (4-byte loads, a row's columns first: 486k tetrahedra, residual 43 -> 35
+// us, post-sweep 47 -> 37; 4 TB/s)
 template <int NV, typename TM>
 __global__ __launch_bounds__(256) void k_half_copy(const TM *__restrict__ A, const TM *__restrict__ W, int N, int K,
                                                    int wper, __half2 *__restrict__ Ah, __half2 *__restrict__ Wh,
@@ -1012,7 +1013,9 @@ __global__ __launch_bounds__(256) void k_half_csr(int n, const int *__restrict__
 // longest row has, entry pairs and columns lane-interleaved, so a wave sweeps 64
 // rows with coalesced 4-byte loads.  The 32-lanes-per-row form issues about ten
 // times the instructions per block (one entry a lane, a shuffle per column) and
-// was bound by that: 74k rows with 693k blocks took 38 us a residual, 35 MB.
+// was bound by that: 74k rows with 693k blocks took 38 us a residual and 34 a
+// post-sweep (35 MB), now 21 and 19: about one wave per SIMD, four blocks of a row
+// in flight (two: 24 and 19), waiting for memory.
 constexpr int kSlicedRows = 16384;   // levels from this size on
 constexpr int kWindow = 1024;
 
@@ -1079,7 +1082,7 @@ __global__ __launch_bounds__(256) void k_sliced(int nslice, const int *__restric
                                                 const __half2 *__restrict__ sval, const float *__restrict__ rm,
                                                 const TM *__restrict__ sw, const TV *__restrict__ f,
                                                 const TV *__restrict__ x, TV *__restrict__ out) {
-  constexpr int NB = NV * NV, NP = (NB + 1) / 2, U = 2;
+  constexpr int NB = NV * NV, NP = (NB + 1) / 2, U = 4;
   const int s = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
   if (s >= nslice) return;
   const int i = srow[(size_t)s * 64 + l];
@@ -1167,66 +1170,114 @@ __global__ __launch_bounds__(256) void k_dense_apply(int m, const double *__rest
 // ---------------------------------------------------------------------------
 // coarsest system: dense [A | I] (m x 2m) and Gauss-Jordan steps
 // ---------------------------------------------------------------------------
-template <int NV, typename Acc>
-__global__ void k_densify(Acc a, int n, double *__restrict__ M) {
-  const int m = n * NV;
-  const int I = row_index();
-  if (I >= n) return;
-  for (int r = 0; r < NV; r++) {
-    double *row = M + (size_t)(I * NV + r) * 2 * m;
-    for (int c = 0; c < 2 * m; c++) row[c] = 0.0;
-    row[m + I * NV + r] = 1.0;
-  }
-  const int L = a.len(I);
-  for (int q = 0; q < L; q++) {
-    const int J = a.col(I, q);
-    if (J < 0) continue;
-    for (int r = 0; r < NV; r++)
-      for (int c = 0; c < NV; c++) M[(size_t)(I * NV + r) * 2 * m + J * NV + c] = a.v(I, q, r * NV + c);
+__global__ __launch_bounds__(256) void k_dense_identity(int m, double *__restrict__ M) {
+  const long total = (long)m * 2 * m;
+  for (long id = (long)blockIdx.x * 256 + threadIdx.x; id < total; id += (long)gridDim.x * 256) {
+    const int r = (int)(id / (2 * m));
+    M[id] = id - (long)r * 2 * m == m + r ? 1.0 : 0.0;
   }
 }
 
-// one elimination step on column k: rows swapped with the pivot row (largest
-// |entry| at or below k, first on ties), pivot row scaled, column k cleared.
-// Reads Min, writes Mout (no in-place hazards across blocks).
-__global__ __launch_bounds__(256) void k_gj_step(const double *__restrict__ Min, double *__restrict__ Mout, int m,
-                                                 int k, int *__restrict__ err) {
-  __shared__ double bv[256];
-  __shared__ int bi[256];
-  const int t = threadIdx.x;
-  double best = -1.0;
-  int bidx = k;
-  for (int r = k + t; r < m; r += 256) {
-    const double a = fabs(Min[(size_t)r * 2 * m + k]);
-    if (a > best) { best = a; bidx = r; }
+// the matrix entries of [A | I], a block per block row
+template <int NV, typename Acc>
+__global__ __launch_bounds__(64) void k_densify(Acc a, int n, double *__restrict__ M) {
+  const int m = n * NV, I = blockIdx.x;
+  if (I >= n) return;
+  for (int id = threadIdx.x; id < a.len(I) * NV * NV; id += 64) {
+    const int q = id / (NV * NV), e = id - q * (NV * NV), r = e / NV, c = e - r * NV;
+    const int J = a.col(I, q);
+    if (J >= 0) M[(size_t)(I * NV + r) * 2 * m + J * NV + c] = a.v(I, q, e);
   }
-  bv[t] = best;
-  bi[t] = bidx;
+}
+
+// Gauss-Jordan on [A | I] in panels of kGjP columns, one elimination step per
+// column k: rows k and p (largest |entry| at or below k, first on ties) swap, row
+// k is divided by the pivot, every other row r loses its entry of column k times
+// row k.  k_gj_panel runs a panel's steps on its own columns and keeps each step's
+// pivot row, pivot and multipliers; k_gj_update applies the steps in order to the
+// columns right of the panel, so every entry goes through the operations of the
+// column-by-column form.  That one took a launch of 4.9 us a column (58 block rows:
+// 290 launches, 1.42 ms; this 38, 1.05 ms); bound by the panels' chain of steps.
+constexpr int kGjP = 16;
+constexpr int kGjThreads = 512;
+__global__ __launch_bounds__(kGjThreads) void k_gj_panel(const double *__restrict__ M, int m, int k0, int np,
+                                                         double *__restrict__ mul, int *__restrict__ piv,
+                                                         int *__restrict__ err) {
+  extern __shared__ double A[];   // [np][m], the panel by columns
+  __shared__ double prow[2][kGjP], krow[2][kGjP];
+  const int t = threadIdx.x, lane = t & 63;
+  for (int id = t; id < m * np; id += kGjThreads) {
+    const int r = id / np, c = id - r * np;
+    A[(size_t)c * m + r] = M[(size_t)r * 2 * m + k0 + c];
+  }
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (t < o) {
-      if (bv[t + o] > bv[t] || (bv[t + o] == bv[t] && bi[t + o] < bi[t])) { bv[t] = bv[t + o]; bi[t] = bi[t + o]; }
+  for (int s = 0; s < np; s++) {
+    const int k = k0 + s, h = s & 1;
+    // every wave looks for the pivot itself: two barriers a step
+    double best = -1.0;
+    int p = m;
+    for (int r = k + lane; r < m; r += 64) {
+      const double a = fabs(A[(size_t)s * m + r]);
+      if (a > best) { best = a; p = r; }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const double v = __shfl_xor(best, o, 64);
+      const int i = __shfl_xor(p, o, 64);
+      if (v > best || (v == best && i < p)) { best = v; p = i; }
+    }
+    if (p >= m) p = k;   // no candidate (NaN): the row itself
+    double pv = A[(size_t)s * m + p];
+    if (pv == 0.0) {   // singular: reported, the steps go on with 1
+      if (t == 0) atomicAdd(err, 1);
+      pv = 1.0;
+    }
+    if (t < np) { prow[h][t] = A[(size_t)t * m + p] / pv; krow[h][t] = A[(size_t)t * m + k]; }
+    if (t == 0) piv[k] = p;
+    __syncthreads();
+    for (int r = t; r < m; r += kGjThreads) {
+      // the row's entry of column k after the swap
+      const double f = r == p ? krow[h][s] : A[(size_t)s * m + r];
+      mul[(size_t)k * m + r] = r == k ? pv : f;
+#pragma unroll 4
+      for (int c = s + 1; c < np; c++) {
+        const double a = r == p ? krow[h][c] : A[(size_t)c * m + r];
+        A[(size_t)c * m + r] = r == k ? prow[h][c] : a - f * prow[h][c];
+      }
     }
     __syncthreads();
   }
-  const int p = bi[0];
-  const double piv = Min[(size_t)p * 2 * m + k];
-  const long total = (long)m * 2 * m;
-  for (long id = (long)blockIdx.x * 256 + t; id < total; id += (long)gridDim.x * 256) {
-    const int r = (int)(id / (2 * m)), cidx = (int)(id - (long)r * 2 * m);
-    if (piv == 0.0) {
-      Mout[id] = Min[id];
-      if (id == 0) atomicAdd(err, 1);
-      continue;
+}
+
+// the steps of panel k0 on the columns right of it, in place: a wave per column,
+// kept in LDS beside the panel's multipliers, no barrier between steps
+constexpr int kGjC = 4;
+__global__ __launch_bounds__(64 * kGjC) void k_gj_update(double *__restrict__ M, int m, int k0, int np,
+                                                         const double *__restrict__ mul,
+                                                         const int *__restrict__ piv) {
+  extern __shared__ double sm[];   // [np][m] multipliers, [kGjC][m] columns
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63, c = k0 + np + blockIdx.x * kGjC + w;
+  double *A = sm + (size_t)(np + w) * m;
+  for (int id = t; id < np * m; id += 64 * kGjC) sm[id] = mul[(size_t)k0 * m + id];
+  if (c < 2 * m)
+    for (int r = lane; r < m; r += 64) A[r] = M[(size_t)r * 2 * m + c];
+  __syncthreads();
+  if (c >= 2 * m) return;
+  for (int s = 0; s < np; s++) {
+    const int k = k0 + s, p = piv[k];
+    const double *f = sm + (size_t)s * m;
+    const double prow = A[p] / f[k], krow = A[k];
+    // both rows are read by every lane before any lane writes
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int r = lane; r < m; r += 64) {
+      const double a = r == p ? krow : A[r];
+      A[r] = r == k ? prow : a - f[r] * prow;
     }
-    const double pc = Min[(size_t)p * 2 * m + cidx] / piv;
-    if (r == k) {
-      Mout[id] = pc;
-    } else {
-      const int src = (r == p) ? k : r;
-      Mout[id] = Min[(size_t)src * 2 * m + cidx] - Min[(size_t)src * 2 * m + k] * pc;
-    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
+  for (int r = lane; r < m; r += 64) M[(size_t)r * 2 * m + c] = A[r];
 }
 
 __global__ void k_take_inverse(int m, const double *__restrict__ M, double *__restrict__ inv) {
@@ -1263,6 +1314,7 @@ static void free_levels(Amg *g) {
   g->lv.clear();
   g->scan_tmp.clear();
   g->dense = g->dense2 = g->inv = nullptr;
+  g->gjpiv = nullptr;
   g->Ah = g->Wh = nullptr;
   g->rm = nullptr;
   g->s = g->dia = nullptr;
@@ -1605,22 +1657,28 @@ static int build_t(bes_ctx *c, Impl *im, Amg *g) {
     const int m = Cl.n * NV;
     g->ndense = m;
     if ((s = dmalloc(g, (void **)&g->dense, (size_t)m * 2 * m * sizeof(double))) ||
-        (s = dmalloc(g, (void **)&g->dense2, (size_t)m * 2 * m * sizeof(double))) ||
+        (s = dmalloc(g, (void **)&g->dense2, (size_t)m * m * sizeof(double))) ||
+        (s = dmalloc(g, (void **)&g->gjpiv, (size_t)m * sizeof(int))) ||
         (s = dmalloc(g, (void **)&g->inv, (size_t)m * m * sizeof(double))))
       return s;
+    hipLaunchKernelGGL(k_dense_identity, dim3(blocks_for((long)m * 2 * m, 256)), dim3(256), 0, c->stream, m, g->dense);
     if (g->nlev == 1)
-      hipLaunchKernelGGL((k_densify<NV, EllAcc<TM, NV>>), dim3(blocks_for(Cl.n, 64)), dim3(64), 0, c->stream,
-                         ell<NV, TM>(c, im), Cl.n, g->dense);
+      hipLaunchKernelGGL((k_densify<NV, EllAcc<TM, NV>>), dim3(Cl.n), dim3(64), 0, c->stream, ell<NV, TM>(c, im), Cl.n,
+                         g->dense);
     else
-      hipLaunchKernelGGL((k_densify<NV, CsrAcc<TM, NV>>), dim3(blocks_for(Cl.n, 64)), dim3(64), 0, c->stream,
-                         csr<NV, TM>(Cl), Cl.n, g->dense);
-    double *a = g->dense, *b = g->dense2;
-    const int gb = blocks_for((long)m * 2 * m, 256);
-    for (int k = 0; k < m; k++) {
-      hipLaunchKernelGGL(k_gj_step, dim3(gb), dim3(256), 0, c->stream, a, b, m, k, g->flags + 2);
-      std::swap(a, b);
+      hipLaunchKernelGGL((k_densify<NV, CsrAcc<TM, NV>>), dim3(Cl.n), dim3(64), 0, c->stream, csr<NV, TM>(Cl), Cl.n,
+                         g->dense);
+    // a panel's multipliers and an update block's columns fit 64 KB of LDS (m <= kDenseMax)
+    static_assert(kDenseMax * (kGjC + 1) * sizeof(double) <= 65536, "one panel column and an update block in LDS");
+    const int P = std::min(kGjP, std::max(1, 8192 / m - kGjC));
+    for (int k0 = 0; k0 < m; k0 += P) {
+      const int np = std::min(P, m - k0);
+      hipLaunchKernelGGL(k_gj_panel, dim3(1), dim3(kGjThreads), (size_t)np * m * sizeof(double), c->stream, g->dense, m,
+                         k0, np, g->dense2, g->gjpiv, g->flags + 2);
+      hipLaunchKernelGGL(k_gj_update, dim3(blocks_for(2 * m - k0 - np, kGjC)), dim3(64 * kGjC),
+                         (size_t)(np + kGjC) * m * sizeof(double), c->stream, g->dense, m, k0, np, g->dense2, g->gjpiv);
     }
-    hipLaunchKernelGGL(k_take_inverse, dim3(blocks_for((long)m * m, 256)), dim3(256), 0, c->stream, m, a, g->inv);
+    hipLaunchKernelGGL(k_take_inverse, dim3(blocks_for((long)m * m, 256)), dim3(256), 0, c->stream, m, g->dense, g->inv);
     BES_HIP(hipGetLastError());
   }
   int h[3];
