@@ -333,6 +333,10 @@ __global__ __launch_bounds__(256) void k_decode(const uint16_t *__restrict__ H, 
   const int N = dm.N;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
   const int base = (blockIdx.x * 4 + w) * 32;
+  // blends of the block's 128 nodes, then the blocks by node: written by the lanes
+  // that hold the logits (NV of 32 columns, a node per store) the operator's
+  // planes were 4-byte stores far apart, 176 us for 83k tetrahedra; now 51
+  __shared__ float Gs[K][NV][128];
   bf4 b[8];
   load_run<32>(net.wb + OFF_WE + col * 64 + 32 * h, true, b);
   const float ce = net.theta[OFF_CE + col];
@@ -346,15 +350,24 @@ __global__ __launch_bounds__(256) void k_decode(const uint16_t *__restrict__ H, 
     f16v acc = mma_run<8>(a, b, zero16());
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int nd = base + 8 * t + 2 * (q >> 2) + h, s = q & 3;
-      if (nd >= N || s >= K || col >= NV) continue;
-      const bool e = dm.nbr[(size_t)s * N + nd] >= 0;
-      const float G = e ? 1.f / (1.f + __expf(-(acc[q] + ce))) : 0.f;
-      Gb[((size_t)nd * SL + s) * 8 + col] = G;
+      const int ln = 8 * t + 2 * (q >> 2) + h, s = q & 3;
+      if (base + ln >= N || s >= K || col >= NV) continue;
+      Gs[s < K ? s : 0][col < NV ? col : 0][32 * w + ln] = 1.f / (1.f + __expf(-(acc[q] + ce)));
+    }
+  }
+  __syncthreads();
+  const int ln = threadIdx.x & 127, nd = blockIdx.x * 128 + ln;
+  if (nd >= N) return;
+  for (int s = threadIdx.x >> 7; s < K; s += 2) {
+    const bool e = dm.nbr[(size_t)s * N + nd] >= 0;
+#pragma unroll
+    for (int r = 0; r < NV; r++) {
+      const float G = e ? Gs[s][r][ln] : 0.f;
+      Gb[((size_t)nd * SL + s) * 8 + r] = G;
 #pragma unroll
       for (int cc = 0; cc < NV; cc++) {
-        const size_t e_ = (size_t)(s * NB + col * NV + cc);
-        LM[((size_t)(1 + s) * NB + col * NV + cc) * N + nd] = (TM)(e ? -G * P[e_ * N + nd] : 0.f);
+        const size_t e_ = (size_t)(s * NB + r * NV + cc);
+        LM[((size_t)NB + e_) * N + nd] = (TM)(e ? -G * P[e_ * N + nd] : 0.f);
       }
     }
   }
@@ -369,52 +382,108 @@ __global__ void k_to_half(const float *__restrict__ x, __half *__restrict__ y, s
 // ---------------------------------------------------------------------------
 // loss: Richardson chains and their adjoint (vectors [N][nv], float)
 // ---------------------------------------------------------------------------
-// (A^T x)_j = A_jj^T x_j + sum_m A_(i, 1+mrev(j,m))^T x_i, i = nbr(j,m)
-template <int ND, typename TM, typename TV>
-__global__ __launch_bounds__(256) void k_spmv_t(const TM *__restrict__ A, DevMesh dm, const int *__restrict__ mrev,
-                                                const TV *__restrict__ x, TV *__restrict__ y) {
+// y_q = A x_q or, with SUB, z_q - A x_q (the product rounded to float first) for
+// QV probe vectors at xs, zs, ys apart, each row's blocks read once for all of
+// them; every product sums as k_spmv's.  With a launch per probe the matrices
+// (41 MB each on 83k tetrahedra) were read for every one: 10.5 us a product
+// (23 transposed); four together take 17 to 22 us (29).
+template <int ND, typename TM, int QV, bool SUB>
+__global__ __launch_bounds__(256) void k_spmv_q(const TM *__restrict__ A, DevMesh dm, const float *__restrict__ x,
+                                                size_t xs, const float *z, size_t zs, float *y, size_t ys) {
+  constexpr int NV = ND + 2, K = ND + 1, NB = NV * NV;
+  const int N = dm.N;
+  const int i = cell_index();
+  if (i >= N) return;
+  double acc[QV][NV];
+#pragma unroll
+  for (int m = -1; m < K; m++) {
+    const int j = m < 0 ? i : dm.nbr[(size_t)(m < 0 ? 0 : m) * N + i];
+    if (j < 0) continue;
+    double xv[QV][NV];
+#pragma unroll
+    for (int q = 0; q < QV; q++)
+#pragma unroll
+      for (int c = 0; c < NV; c++) xv[q][c] = (double)x[q * xs + (size_t)j * NV + c];
+    const TM *Ao = A + (size_t)(1 + m) * NB * N + i;
+#pragma unroll
+    for (int r = 0; r < NV; r++) {
+      double av[NV];
+#pragma unroll
+      for (int c = 0; c < NV; c++) av[c] = (double)Ao[(size_t)(r * NV + c) * N];
+#pragma unroll
+      for (int q = 0; q < QV; q++) {
+        double s = 0;
+#pragma unroll
+        for (int c = 0; c < NV; c++) s += av[c] * xv[q][c];
+        if (m < 0) acc[q][r] = s;
+        else acc[q][r] += s;
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < QV; q++)
+#pragma unroll
+    for (int r = 0; r < NV; r++) {
+      const size_t at = (size_t)i * NV + r;
+      y[q * ys + at] = SUB ? z[q * zs + at] - (float)acc[q][r] : (float)acc[q][r];
+    }
+}
+
+// the same with A^T: (A^T x)_j = A_jj^T x_j + sum_m A_(i, 1+mrev(j,m))^T x_i, i = nbr(j,m)
+template <int ND, typename TM, int QV, bool SUB>
+__global__ __launch_bounds__(256) void k_spmv_tq(const TM *__restrict__ A, DevMesh dm, const int *__restrict__ mrev,
+                                                 const float *__restrict__ x, size_t xs, const float *z, size_t zs,
+                                                 float *y, size_t ys) {
   constexpr int NV = ND + 2, K = ND + 1, NB = NV * NV;
   const int N = dm.N;
   const int j = cell_index();
   if (j >= N) return;
-  double acc[NV], xv[NV];
+  double acc[QV][NV];
 #pragma unroll
-  for (int c = 0; c < NV; c++) xv[c] = (double)x[(size_t)j * NV + c];
-#pragma unroll
-  for (int r = 0; r < NV; r++) {
-    double s = 0;
-#pragma unroll
-    for (int c = 0; c < NV; c++) s += (double)A[((size_t)(c * NV + r)) * N + j] * xv[c];
-    acc[r] = s;
-  }
-#pragma unroll
-  for (int m = 0; m < K; m++) {
-    const int i = dm.nbr[(size_t)m * N + j];
+  for (int m = -1; m < K; m++) {
+    const int i = m < 0 ? j : dm.nbr[(size_t)(m < 0 ? 0 : m) * N + j];
     if (i < 0) continue;
-    const int mm = mrev[(size_t)m * N + j];
+    const int slot = m < 0 ? 0 : 1 + mrev[(size_t)(m < 0 ? 0 : m) * N + j];
+    double xv[QV][NV];
 #pragma unroll
-    for (int c = 0; c < NV; c++) xv[c] = (double)x[(size_t)i * NV + c];
-    const TM *Ao = A + (size_t)(1 + mm) * NB * N;
+    for (int q = 0; q < QV; q++)
+#pragma unroll
+      for (int c = 0; c < NV; c++) xv[q][c] = (double)x[q * xs + (size_t)i * NV + c];
+    const TM *Ao = A + (size_t)slot * NB * N + i;
 #pragma unroll
     for (int r = 0; r < NV; r++) {
-      double s = 0;
+      double av[NV];
 #pragma unroll
-      for (int c = 0; c < NV; c++) s += (double)Ao[((size_t)(c * NV + r)) * N + i] * xv[c];
-      acc[r] += s;
+      for (int c = 0; c < NV; c++) av[c] = (double)Ao[(size_t)(c * NV + r) * N];
+#pragma unroll
+      for (int q = 0; q < QV; q++) {
+        double s = 0;
+#pragma unroll
+        for (int c = 0; c < NV; c++) s += av[c] * xv[q][c];
+        if (m < 0) acc[q][r] = s;
+        else acc[q][r] += s;
+      }
     }
   }
 #pragma unroll
-  for (int r = 0; r < NV; r++) y[(size_t)j * NV + r] = (TV)acc[r];
+  for (int q = 0; q < QV; q++)
+#pragma unroll
+    for (int r = 0; r < NV; r++) {
+      const size_t at = (size_t)j * NV + r;
+      y[q * ys + at] = SUB ? z[q * zs + at] - (float)acc[q][r] : (float)acc[q][r];
+    }
 }
 
-// out = x - y (r_{k+1} = r_k - A M r_k), or out = x - y scaled
-__global__ void k_sub(const float *__restrict__ x, const float *__restrict__ y, float *__restrict__ out, size_t n) {
+// one factor per probe
+struct CoefQ {
+  float a[16];
+};
+// out_q = a_q x_q, probe q = blockIdx.y
+__global__ void k_scale_q(const float *__restrict__ x, size_t xs, CoefQ a, float *__restrict__ out, size_t os,
+                          size_t n) {
+  const int p = blockIdx.y;
   for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
-    out[q] = x[q] - y[q];
-}
-__global__ void k_scale_f(const float *__restrict__ x, float a, float *__restrict__ out, size_t n) {
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
-    out[q] = a * x[q];
+    out[p * os + q] = a.a[p] * x[p * xs + q];
 }
 __global__ void k_from_double(const double *__restrict__ x, float *__restrict__ out, size_t n) {
   for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
@@ -441,8 +510,11 @@ __global__ void k_randn(unsigned long long seed, float *__restrict__ out, size_t
   }
 }
 
-// sum of squares, per-block partials (double)
-__global__ void k_sumsq(const float *__restrict__ x, size_t n, double *__restrict__ part) {
+// sums of squares of the first (even blockIdx.y) and last vector of each probe's
+// chain, per-block partials (double)
+__global__ void k_sumsq(const float *__restrict__ x, size_t probe, size_t last, size_t n, double *__restrict__ part) {
+  const int v = blockIdx.y;
+  x += (v >> 1) * probe + ((v & 1) ? last : 0);
   double s = 0;
   for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
     s += (double)x[q] * x[q];
@@ -450,41 +522,52 @@ __global__ void k_sumsq(const float *__restrict__ x, size_t n, double *__restric
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+  if (threadIdx.x == 0) part[(size_t)v * gridDim.x + blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
 }
 __global__ void k_sum_parts(const double *__restrict__ part, int nblk, double *__restrict__ out) {
+  part += (size_t)blockIdx.x * nblk;
   double s = 0;
   for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += part[b];
   __shared__ double sh[4];
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) out[0] = sh[0] + sh[1] + sh[2] + sh[3];
+  if (threadIdx.x == 0) out[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
 }
 
-// dMe_im -= at_i (x) r_j   (at = A^T g, one (probe, step) term)
+// dMe_im = -sum over probes and steps (probe by probe, last step first) of
+// at_i (x) r_j, at = A^T g; a thread per (cell, face m = blockIdx.y), the sum in
+// registers: 33 us for the 12 terms of a training step on 83k tetrahedra.  (One
+// launch per term read and wrote all of dMe each time, 29 us each.)
 template <int ND>
-__global__ __launch_bounds__(256) void k_dme(const float *__restrict__ at, const float *__restrict__ rk, DevMesh dm,
-                                             float *__restrict__ dMe) {
-  constexpr int NV = ND + 2, K = ND + 1, NB = NV * NV;
-  const int N = dm.N;
-  const int i = cell_index();
+__global__ __launch_bounds__(256) void k_dme(const float *__restrict__ at, const float *__restrict__ chain, int Q,
+                                             int steps, DevMesh dm, float *__restrict__ dMe) {
+  constexpr int NV = ND + 2, NB = NV * NV;
+  const int N = dm.N, m = blockIdx.y;
+  const int i = xcd_block_of(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (i >= N) return;
-  float ai[NV];
+  const size_t n = (size_t)N * NV;
+  const int j = dm.nbr[(size_t)m * N + i];
+  float d[NB];
 #pragma unroll
-  for (int r = 0; r < NV; r++) ai[r] = at[(size_t)i * NV + r];
+  for (int e = 0; e < NB; e++) d[e] = 0.f;
+  if (j >= 0)
+    for (int q = 0; q < Q; q++)
+#pragma unroll 3
+      for (int k = steps - 1; k >= 0; k--) {
+        float ai[NV], rj[NV];
 #pragma unroll
-  for (int m = 0; m < K; m++) {
-    const int j = dm.nbr[(size_t)m * N + i];
-    if (j < 0) continue;
-    float rj[NV];
+        for (int r = 0; r < NV; r++) {
+          ai[r] = at[((size_t)q * steps + k) * n + (size_t)i * NV + r];
+          rj[r] = chain[((size_t)q * (steps + 1) + k) * n + (size_t)j * NV + r];
+        }
 #pragma unroll
-    for (int cc = 0; cc < NV; cc++) rj[cc] = rk[(size_t)j * NV + cc];
+        for (int r = 0; r < NV; r++)
 #pragma unroll
-    for (int r = 0; r < NV; r++)
+          for (int cc = 0; cc < NV; cc++) d[r * NV + cc] -= ai[r] * rj[cc];
+      }
 #pragma unroll
-      for (int cc = 0; cc < NV; cc++) dMe[((size_t)m * NB + r * NV + cc) * N + i] -= ai[r] * rj[cc];
-  }
+  for (int e = 0; e < NB; e++) dMe[((size_t)m * NB + e) * N + i] = d[e];
 }
 
 // dL/ds_im = -sum_c dMe_im[r][c] P_im[r][c] * G (1 - G), as bf16 rows of 32
@@ -758,8 +841,18 @@ __global__ __launch_bounds__(256) void k_encode_bwd(const float *__restrict__ dH
 __global__ void k_grad_reduce(const float *__restrict__ gpart, int nrow, float *__restrict__ grad) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= NPARAM) return;
+  // the rows are added in order; 32 of their loads in flight (one at a time took
+  // 338 us, a chain of 1024 memory latencies; now 40)
   float s = 0.f;
-  for (int r = 0; r < nrow; r++) s += gpart[(size_t)r * NPARAM + p];
+  int r = 0;
+  for (; r + 32 <= nrow; r += 32) {
+    float v[32];
+#pragma unroll
+    for (int u = 0; u < 32; u++) v[u] = gpart[(size_t)(r + u) * NPARAM + p];
+#pragma unroll
+    for (int u = 0; u < 32; u++) s += v[u];
+  }
+  for (; r < nrow; r++) s += gpart[(size_t)r * NPARAM + p];
   grad[p] = s;
 }
 
@@ -819,7 +912,8 @@ struct Lp {
   float *dH = nullptr, *dH2 = nullptr, *dA = nullptr, *dnb = nullptr, *dMe = nullptr;
   uint16_t *dlog = nullptr;
   float *chain = nullptr;                // [Q][K+1][n]
-  float *tv1 = nullptr, *tv2 = nullptr, *gv = nullptr;
+  float *tv = nullptr, *gv = nullptr;    // [Q][n] M r_k, g_k
+  float *at = nullptr;                   // [Q][K][n] A^T g_(k+1)
   double *part = nullptr, *dsum = nullptr;
   int qcap = 0, kcap = 0;
   bool train_ready = false;
@@ -876,7 +970,7 @@ int lp_release(Impl *im) {
   if (!L) return BES_OK;
   void *ptrs[] = {L->theta, L->grad, L->m1, L->m2, L->gpart, L->wb, L->wt, L->bbits, L->efeat, L->X, L->Aed, L->H,
                   L->Msg, L->Agg, L->Rr, L->P, L->G, L->dH, L->dH2, L->dA, L->dnb, L->dMe, L->dlog, L->chain,
-                  L->tv1, L->tv2, L->gv, L->part, L->dsum};
+                  L->tv, L->at, L->gv, L->part, L->dsum};
   for (void *p : ptrs)
     if (p) hipFree(p);
   delete L;
@@ -932,7 +1026,7 @@ static int lp_alloc(bes_ctx *c, Impl *im, uint64_t seed) {
 static int lp_alloc_train(bes_ctx *c, Lp *L, int Q, int K) {
   if (L->train_ready && Q <= L->qcap && K <= L->kcap) return BES_OK;
   const size_t Np = (size_t)L->ntile * 32, n = (size_t)L->N * L->nv;
-  void *old[] = {L->dH, L->dH2, L->dA, L->dnb, L->dMe, L->dlog, L->chain, L->tv1, L->tv2, L->gv, L->part, L->dsum,
+  void *old[] = {L->dH, L->dH2, L->dA, L->dnb, L->dMe, L->dlog, L->chain, L->tv, L->at, L->gv, L->part, L->dsum,
                  L->gpart};
   for (void *p : old)
     if (p) hipFree(p);
@@ -940,8 +1034,9 @@ static int lp_alloc_train(bes_ctx *c, Lp *L, int Q, int K) {
   if ((s = lalloc(&L->dH, Np * WD)) || (s = lalloc(&L->dH2, Np * WD)) || (s = lalloc(&L->dA, Np * WD)) ||
       (s = lalloc(&L->dnb, Np * SL * WD)) || (s = lalloc(&L->dMe, (size_t)L->k * L->nv * L->nv * L->N)) ||
       (s = lalloc(&L->dlog, Np * SL * WD)) || (s = lalloc(&L->chain, (size_t)Q * (K + 1) * n)) ||
-      (s = lalloc(&L->tv1, n)) || (s = lalloc(&L->tv2, n)) || (s = lalloc(&L->gv, n)) ||
-      (s = lalloc(&L->part, kDotBlocks)) || (s = lalloc(&L->dsum, 1)) ||
+      (s = lalloc(&L->tv, (size_t)Q * n)) || (s = lalloc(&L->at, (size_t)Q * K * n)) ||
+      (s = lalloc(&L->gv, (size_t)Q * n)) ||
+      (s = lalloc(&L->part, (size_t)2 * Q * kDotBlocks)) || (s = lalloc(&L->dsum, (size_t)2 * Q)) ||
       (s = lalloc(&L->gpart, (size_t)kTrainWaves * NPARAM)))
     return s;
   BES_HIP(hipMemset(L->dH, 0, Np * WD * sizeof(float)));
@@ -1003,29 +1098,35 @@ int lp_build(bes_ctx *c, Impl *im) {
   return BES_OK;
 }
 
-static double read_sumsq(bes_ctx *c, Lp *L, const float *x, size_t n, int *st) {
-  hipLaunchKernelGGL(k_sumsq, dim3(kDotBlocks), dim3(256), 0, c->stream, x, n, L->part);
-  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, c->stream, L->part, kDotBlocks, L->dsum);
-  double v = 0;
-  hipError_t e = hipMemcpyAsync(&v, L->dsum, sizeof(double), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  *st = e == hipSuccess ? BES_OK : hip_fail(e, "sum of squares");
-  return v;
-}
-
+// y_q = A x_q or z_q - A x_q (z given; A^T with trans) for Q probe vectors, four
+// or fewer per launch
 template <typename TM>
-static void spmv_f(bes_ctx *c, const TM *A, const float *x, float *y) {
-  const int bs = 256;
-  if (c->nd == 2) hipLaunchKernelGGL((k_spmv<2, TM, float>), dim3(grid_for(c->N, bs)), dim3(bs), 0, c->stream, A, c->dm, x, y, 0);
-  else hipLaunchKernelGGL((k_spmv<3, TM, float>), dim3(grid_for(c->N, bs)), dim3(bs), 0, c->stream, A, c->dm, x, y, 0);
-}
-template <typename TM>
-static void spmv_t_f(bes_ctx *c, Impl *im, const TM *A, const float *x, float *y) {
-  const int bs = 256;
-  if (c->nd == 2)
-    hipLaunchKernelGGL((k_spmv_t<2, TM, float>), dim3(grid_for(c->N, bs)), dim3(bs), 0, c->stream, A, c->dm, im->fd.mrev, x, y);
-  else
-    hipLaunchKernelGGL((k_spmv_t<3, TM, float>), dim3(grid_for(c->N, bs)), dim3(bs), 0, c->stream, A, c->dm, im->fd.mrev, x, y);
+static void spmv_probes(bes_ctx *c, Impl *im, const TM *A, bool trans, int Q, const float *x, size_t xs, const float *z,
+                        size_t zs, float *y, size_t ys) {
+  const dim3 grid(grid_for(c->N, 256)), block(256);
+  auto go = [&](auto nd, auto qv, auto sub, int q0) {
+    constexpr int ND = decltype(nd)::value, QV = decltype(qv)::value;
+    constexpr bool SUB = decltype(sub)::value;
+    const float *xq = x + q0 * xs, *zq = SUB ? z + q0 * zs : nullptr;
+    if (trans)
+      hipLaunchKernelGGL((k_spmv_tq<ND, TM, QV, SUB>), grid, block, 0, c->stream, A, c->dm, im->fd.mrev, xq, xs, zq, zs,
+                         y + q0 * ys, ys);
+    else
+      hipLaunchKernelGGL((k_spmv_q<ND, TM, QV, SUB>), grid, block, 0, c->stream, A, c->dm, xq, xs, zq, zs, y + q0 * ys,
+                         ys);
+  };
+  auto group = [&](auto qv, int q0) {
+    auto dim = [&](auto nd) {
+      if (z) go(nd, qv, std::true_type{}, q0);
+      else go(nd, qv, std::false_type{}, q0);
+    };
+    if (c->nd == 2) dim(std::integral_constant<int, 2>{});
+    else dim(std::integral_constant<int, 3>{});
+  };
+  int q = 0;
+  for (; q + 4 <= Q; q += 4) group(std::integral_constant<int, 4>{}, q);
+  if (q + 2 <= Q) { group(std::integral_constant<int, 2>{}, q); q += 2; }
+  if (q < Q) group(std::integral_constant<int, 1>{}, q);
 }
 
 // one forward + loss + backward on the current system; probes already in
@@ -1039,33 +1140,38 @@ static int lp_loss_grad_t(bes_ctx *c, Impl *im, int Q, int K, double *loss) {
   if ((s = lp_build_t<TM>(c, im))) return s;
   const TM *A = (const TM *)im->A, *M = (const TM *)im->LM;
   ProfScope ps(c, kProfLearned, 0.0);
-  hipLaunchKernelGGL(k_fill_f, dim3(1024), dim3(256), 0, c->stream, L->dMe, 0.f, (size_t)c->k * NB * N);
+  // r_{k+1} = r_k - A M r_k of every probe's chain
+  const size_t cs = (size_t)(K + 1) * n;
+  for (int kk = 0; kk < K; kk++) {
+    spmv_probes<TM>(c, im, M, false, Q, L->chain + kk * n, cs, nullptr, 0, L->tv, n);
+    spmv_probes<TM>(c, im, A, false, Q, L->tv, n, L->chain + kk * n, cs, L->chain + (kk + 1) * n, cs);
+  }
+  hipLaunchKernelGGL(k_sumsq, dim3(kDotBlocks, 2 * Q), dim3(256), 0, c->stream, L->chain, cs, K * n, n, L->part);
+  hipLaunchKernelGGL(k_sum_parts, dim3(2 * Q), dim3(256), 0, c->stream, L->part, kDotBlocks, L->dsum);
+  double sums[32];   // probes <= 16
+  BES_HIP(hipMemcpyAsync(sums, L->dsum, (size_t)2 * Q * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  BES_HIP(hipStreamSynchronize(c->stream));
   double Lsum = 0;
+  CoefQ gc;
   for (int q = 0; q < Q; q++) {
-    float *ch = L->chain + (size_t)q * (K + 1) * n;
-    for (int kk = 0; kk < K; kk++) {
-      spmv_f<TM>(c, M, ch + kk * n, L->tv1);
-      spmv_f<TM>(c, A, L->tv1, L->tv2);
-      hipLaunchKernelGGL(k_sub, dim3(1024), dim3(256), 0, c->stream, ch + kk * n, L->tv2, ch + (kk + 1) * n, n);
-    }
-    const double vv = read_sumsq(c, L, ch, n, &s);
-    if (s) return s;
-    const double rr = read_sumsq(c, L, ch + K * n, n, &s);
-    if (s) return s;
+    const double vv = sums[2 * q], rr = sums[2 * q + 1];
     if (!(vv > 0)) { set_error("zero probe vector"); return BES_ERR_ARG; }
     Lsum += rr / vv / Q;
-    // adjoint: g_K = 2 r_K / (Q vv); dMe -= (A^T g_{k+1}) (x) r_k; g_k = g_{k+1} - M^T A^T g_{k+1}
-    hipLaunchKernelGGL(k_scale_f, dim3(1024), dim3(256), 0, c->stream, ch + K * n, (float)(2.0 / (Q * vv)), L->gv, n);
-    for (int kk = K - 1; kk >= 0; kk--) {
-      spmv_t_f<TM>(c, im, A, L->gv, L->tv1);
-      if (c->nd == 2) hipLaunchKernelGGL(k_dme<2>, dim3(grid_for(N, 256)), dim3(256), 0, c->stream, L->tv1, ch + kk * n, c->dm, L->dMe);
-      else hipLaunchKernelGGL(k_dme<3>, dim3(grid_for(N, 256)), dim3(256), 0, c->stream, L->tv1, ch + kk * n, c->dm, L->dMe);
-      if (kk > 0) {
-        spmv_t_f<TM>(c, im, M, L->tv1, L->tv2);
-        hipLaunchKernelGGL(k_sub, dim3(1024), dim3(256), 0, c->stream, L->gv, L->tv2, L->gv, n);
-      }
-    }
+    gc.a[q] = (float)(2.0 / (Q * vv));
   }
+  // adjoint: g_K = 2 r_K / (Q vv); dMe -= (A^T g_{k+1}) (x) r_k; g_k = g_{k+1} - M^T A^T g_{k+1}
+  hipLaunchKernelGGL(k_scale_q, dim3(1024, Q), dim3(256), 0, c->stream, L->chain + K * n, cs, gc, L->gv, n, n);
+  const size_t as = (size_t)K * n;
+  for (int kk = K - 1; kk >= 0; kk--) {
+    spmv_probes<TM>(c, im, A, true, Q, L->gv, n, nullptr, 0, L->at + kk * n, as);
+    if (kk > 0) spmv_probes<TM>(c, im, M, true, Q, L->at + kk * n, as, L->gv, n, L->gv, n);
+  }
+  if (c->nd == 2)
+    hipLaunchKernelGGL(k_dme<2>, dim3(grid_for(N, 256), 3), dim3(256), 0, c->stream, L->at, L->chain, Q, K, c->dm,
+                       L->dMe);
+  else
+    hipLaunchKernelGGL(k_dme<3>, dim3(grid_for(N, 256), 4), dim3(256), 0, c->stream, L->at, L->chain, Q, K, c->dm,
+                       L->dMe);
   *loss = Lsum;
   // back through the decoder, the layers and the encoder
   const Net net = net_of(L);
@@ -1087,7 +1193,7 @@ static int lp_loss_grad_t(bes_ctx *c, Impl *im, int Q, int K, double *loss) {
                        im->fd.mrev, c->k, N, L->dH);
   }
   hipLaunchKernelGGL(k_encode_bwd, dim3(nblk), dim3(256), 0, c->stream, L->dH, L->H, L->X, N, L->ntile, L->gpart);
-  hipLaunchKernelGGL(k_grad_reduce, dim3(grid_for(NPARAM, 256)), dim3(256), 0, c->stream, L->gpart, kTrainWaves,
+  hipLaunchKernelGGL(k_grad_reduce, dim3(grid_for(NPARAM, 64)), dim3(64), 0, c->stream, L->gpart, kTrainWaves,
                      L->grad);
   BES_HIP(hipGetLastError());
   return BES_OK;
