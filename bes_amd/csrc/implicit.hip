@@ -305,6 +305,65 @@ __global__ __launch_bounds__(256) void k_spmv_pos(const TM *__restrict__ A, cons
   for (int r = 0; r < NV; r++) y[((size_t)p * NV + r) * B + b] = (TV)acc[r];
 }
 
+// y = A x as k_spmv / k_spmv_pos with a thread per (block of a row, cell,
+// condition): wave w of a block takes slot w (0 the diagonal, w the neighbour
+// w - 1; 1 + K = NV of them) of the block's 64 units u = cell*B + condition, then
+// component w of their sums, the products added in slot order.  An absent
+// neighbour adds -0.0, which changes nothing.
+// Bound by memory latency where a thread per cell is too few waves (its four
+// gathers follow one another) and by the last-level cache above: per product 31k
+// tetrahedra FP64 11.7 -> 7.0 us, 83k 20.4 -> 16, 249k 61.6 -> 55.1 (FP32 32.6 ->
+// 28.7), 590k 138 -> 127; 12.8k triangles 7.1 -> 4.3, 490k 60.9 -> 54.2.  (A
+// thread per row of the block repeats the gathers in every row: 18.6, 81.5, 190.)
+template <int ND, typename TM, typename TV>
+__device__ __forceinline__ void block_product(const TM *__restrict__ Am, size_t es, const TV *__restrict__ xs, int lgB,
+                                              double s[ND + 2]) {
+  constexpr int NV = ND + 2;
+  TV xv[NV];
+  TM av[NV][NV];
+#pragma unroll
+  for (int c = 0; c < NV; c++) xv[c] = xs[(size_t)c << lgB];
+#pragma unroll
+  for (int r = 0; r < NV; r++)
+#pragma unroll
+    for (int c = 0; c < NV; c++) av[r][c] = Am[(size_t)(r * NV + c) * es];
+#pragma unroll
+  for (int r = 0; r < NV; r++) {
+    double t = 0;
+#pragma unroll
+    for (int c = 0; c < NV; c++) t += to_d(av[r][c]) * (double)xv[c];
+    s[r] = t;
+  }
+}
+
+template <int ND, typename TM, typename TV>
+__global__ __launch_bounds__(64 * (ND + 2)) void k_spmv_slots(const TM *__restrict__ A, const int *__restrict__ nbr,
+                                                              int N, const TV *__restrict__ x, TV *__restrict__ y,
+                                                              int lgB) {
+  constexpr int NV = ND + 2, NB = NV * NV;
+  __shared__ double sh[NV][NV][64];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = threadIdx.x & 63;
+  const int u = blockIdx.x * 64 + t;
+  const int p = u >> lgB, b = u & ((1 << lgB) - 1);
+  const size_t es = (size_t)N << lgB;
+  double s[NV];
+#pragma unroll
+  for (int r = 0; r < NV; r++) s[r] = -0.0;
+  if (p < N) {
+    const int q = w == 0 ? p : nbr[(size_t)(w - 1) * N + p];
+    if (q >= 0)
+      block_product<ND, TM, TV>(A + (size_t)w * NB * es + u, es, x + (((size_t)q * NV) << lgB) + b, lgB, s);
+  }
+#pragma unroll
+  for (int r = 0; r < NV; r++) sh[w][r][t] = s[r];
+  __syncthreads();
+  if (p >= N) return;
+  double acc = sh[0][w][t];
+#pragma unroll
+  for (int m = 1; m < NV; m++) acc += sh[m][w][t];
+  y[(((size_t)p * NV + w) << lgB) + b] = (TV)acc;
+}
+
 // rows between cell order and colour order (each row nv*B contiguous values):
 // to_colour: dst[p] = src[crow[p]], else dst[crow[p]] = src[p]
 template <typename T>
@@ -557,6 +616,71 @@ __global__ __launch_bounds__(256) void k_ilu_upper(const TM *__restrict__ LU, in
 #pragma unroll
     for (int c = 0; c < NV; c++) s += (double)Lr[(a * NV + c) * es] * acc[c];
     x[((size_t)p * NV + a) * B + b] = (TV)s;
+  }
+}
+
+// The sweeps as k_ilu_lower / k_ilu_upper with a thread per (neighbour, row p,
+// condition): wave m of a block takes neighbour m of the block's 64 units (the
+// last wave has none), then component m of their rows, the products subtracted in
+// the order of the neighbours; one not in the sweep subtracts 0.0, which changes
+// nothing.  INV: the product with inv(U_pp), whose factor is rounded to TV first
+// in the forward sweep.
+// Bound as k_spmv_slots; a colour is a third of the mesh, so it pays further up:
+// backward, a colour of 29k tetrahedra FP64 8.9 -> 5.3 us, 80k 12.8 -> 8.8, 240k
+// 29.2 -> 26.1; forward 9.0 -> 6.6, 22.3 -> 19.7, 43.8 -> 45.8; 15k triangles
+// forward 6.3 -> 4.0, backward 5.8 -> 4.1.
+template <int ND, typename TM, typename TV, bool UPPER, bool INV>
+__global__ __launch_bounds__(64 * (ND + 2)) void k_ilu_slots(const TM *__restrict__ LU, int N,
+                                                             const int *__restrict__ cnp,
+                                                             const unsigned char *__restrict__ clow, int p0, int nrows,
+                                                             const TV *__restrict__ r, const TV *y, int y0end,
+                                                             const TV *x, TV *out, int lgB) {
+  constexpr int NV = ND + 2, K = ND + 1, NB = NV * NV;
+  __shared__ double sh[K][NV][64];
+  __shared__ double sa[INV ? NV : 1][64];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = threadIdx.x & 63;
+  const int u = blockIdx.x * 64 + t;
+  const bool ok = u < (nrows << lgB);
+  const int p = p0 + (u >> lgB), b = u & ((1 << lgB) - 1);
+  const size_t es = (size_t)N << lgB, at = (((size_t)p * NV + w) << lgB) + b;
+  const TM *Lr = LU + ((size_t)p << lgB) + b;
+  TV own = 0;
+  TM d[INV ? NV : 1];
+  if (ok) {
+    own = (UPPER && p >= y0end ? y : r)[at];
+    if constexpr (INV)
+#pragma unroll
+      for (int c = 0; c < NV; c++) d[c] = Lr[(size_t)(w * NV + c) * es];
+  }
+  if (w < K) {
+    double s[NV];
+#pragma unroll
+    for (int c = 0; c < NV; c++) s[c] = 0.0;
+    if (ok) {
+      const int q = cnp[(size_t)w * N + p];
+      const bool low = (clow[p] >> w) & 1;
+      if (UPPER ? q >= 0 && !low : low) {
+        const TV *src = UPPER ? x : (q < y0end ? r : y);
+        block_product<ND, TM, TV>(Lr + (size_t)(1 + w) * NB * es, es, src + (((size_t)q * NV) << lgB) + b, lgB, s);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NV; c++) sh[w][c][t] = s[c];
+  }
+  __syncthreads();
+  double acc = (double)own;
+#pragma unroll
+  for (int m = 0; m < K; m++) acc -= sh[m][w][t];
+  if constexpr (INV) {
+    sa[w][t] = UPPER ? acc : (double)(TV)acc;
+    __syncthreads();
+    if (!ok) return;
+    double s = 0;
+#pragma unroll
+    for (int c = 0; c < NV; c++) s += (double)d[c] * sa[c][t];
+    out[at] = (TV)s;
+  } else {
+    if (ok) out[at] = (TV)acc;
   }
 }
 
@@ -1643,6 +1767,30 @@ static int factor(bes_ctx *c, Impl *im) {
 }
 
 // z = M^-1 r (B conditions at once for the block Jacobi and ILU(0) forms)
+// A thread per block (k_spmv_slots, k_ilu_slots) or per cell and condition.  One
+// condition gathers its neighbours' values 40 bytes apart and a colour of a small
+// mesh is a few waves, so the split pays while a launch does not fill the chip
+// with loads: at 1M cells 4 to 8 % are left, at 2M both take the same time.  A
+// batch fills it earlier and its gathers are contiguous: FP64 gains 5 % and FP32
+// nothing at 250k cell-conditions, both lose 1 to 3 % at 500k.
+static bool slot_split(const bes_ctx *c) { return (size_t)c->N * c->B <= (c->B == 1 ? 1u << 20 : 1u << 18); }
+
+// y = A x, matrix and vectors in cell order
+template <typename TM, typename TV>
+static void spmv_cells(bes_ctx *c, const TM *A, const TV *x, TV *y, int bs) {
+  auto go = [&](auto ndc) {
+    constexpr int ND = decltype(ndc)::value;
+    if (slot_split(c))
+      hipLaunchKernelGGL((k_spmv_slots<ND, TM, TV>), dim3(grid_for(c->N * c->B, 64)), dim3(64 * (ND + 2)), 0, c->stream, A,
+                         c->dm.nbr, c->N, x, y, c->lgB);
+    else
+      hipLaunchKernelGGL((k_spmv<ND, TM, TV>), dim3(grid_for(c->N * c->B, bs)), dim3(bs), 0, c->stream, A, c->dm, x, y,
+                         c->lgB);
+  };
+  if (c->nd == 2) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 3>{});
+}
+
 template <typename TM, typename TV>
 static int precond_apply(bes_ctx *c, Impl *im, const TV *r, TV *z, TV *tmp) {
   if (im->precond == 4) return amg_apply<TV>(c, im, r, z, tmp);
@@ -1661,11 +1809,9 @@ static int precond_apply(bes_ctx *c, Impl *im, const TV *r, TV *z, TV *tmp) {
   if (im->precond == 0) {
     hipLaunchKernelGGL((k_scale<TV, TV>), dim3(kRedBlocks), dim3(256), 0, c->stream, r, 1.0, z, n);
   } else if (im->precond == 3 && im->prec == 32) {   // learned operator, FP16 copy: one block SpMV
-    if (c->nd == 2) hipLaunchKernelGGL((k_spmv<2, __half, TV>), dim3(grid_for(N, bs)), dim3(bs), 0, c->stream, (const __half *)im->LMh, c->dm, r, z, 0);
-    else hipLaunchKernelGGL((k_spmv<3, __half, TV>), dim3(grid_for(N, bs)), dim3(bs), 0, c->stream, (const __half *)im->LMh, c->dm, r, z, 0);
+    spmv_cells(c, (const __half *)im->LMh, r, z, bs);
   } else if (im->precond == 3) {   // learned operator: one block SpMV
-    if (c->nd == 2) hipLaunchKernelGGL((k_spmv<2, TM, TV>), dim3(grid_for(N, bs)), dim3(bs), 0, c->stream, (const TM *)im->LM, c->dm, r, z, 0);
-    else hipLaunchKernelGGL((k_spmv<3, TM, TV>), dim3(grid_for(N, bs)), dim3(bs), 0, c->stream, (const TM *)im->LM, c->dm, r, z, 0);
+    spmv_cells(c, (const TM *)im->LM, r, z, bs);
   } else if (im->precond == 1) {
     if (c->nd == 2) hipLaunchKernelGGL((k_bj_apply<2, TM, TV>), dim3(grid_for(N * B, bs)), dim3(bs), 0, c->stream, (const TM *)im->LU, N, r, z, lgB);
     else hipLaunchKernelGGL((k_bj_apply<3, TM, TV>), dim3(grid_for(N * B, bs)), dim3(bs), 0, c->stream, (const TM *)im->LU, N, r, z, lgB);
@@ -1673,35 +1819,40 @@ static int precond_apply(bes_ctx *c, Impl *im, const TV *r, TV *z, TV *tmp) {
     // colour 0 needs no forward sweep (y = r); the last colour's backward step
     // is fused into its forward sweep
     const int y0end = nc > 0 ? im->color_start[1] : 0;
-    for (int col = 1; col < nc; col++) {
-      const int r0 = im->color_start[col], nr = im->color_start[col + 1] - r0;
-      if (nr == 0) continue;
-      const dim3 g(grid_for(nr * B, bs));
-      if (col == nc - 1) {
-        if (c->nd == 2)
-          hipLaunchKernelGGL((k_ilu_lower<2, TM, TV, true>), g, dim3(bs), 0, c->stream, (const TM *)im->LU, N, im->cnp,
-                             im->clow, r0, nr, r, tmp, y0end, z, lgB);
+    const TM *LU = (const TM *)im->LU;
+    const bool slots = slot_split(c);
+    auto sweeps = [&](auto ndc) {
+      constexpr int ND = decltype(ndc)::value;
+      auto lower = [&](auto fuse, int r0, int nr) {
+        constexpr bool FUSE = decltype(fuse)::value;
+        TV *x = FUSE ? z : nullptr;
+        if (slots)
+          hipLaunchKernelGGL((k_ilu_slots<ND, TM, TV, false, FUSE>), dim3(grid_for(nr * B, 64)), dim3(64 * (ND + 2)), 0,
+                             c->stream, LU, N, im->cnp, im->clow, r0, nr, r, tmp, y0end, (const TV *)nullptr,
+                             FUSE ? z : tmp, lgB);
         else
-          hipLaunchKernelGGL((k_ilu_lower<3, TM, TV, true>), g, dim3(bs), 0, c->stream, (const TM *)im->LU, N, im->cnp,
-                             im->clow, r0, nr, r, tmp, y0end, z, lgB);
-      } else if (c->nd == 2) {
-        hipLaunchKernelGGL((k_ilu_lower<2, TM, TV, false>), g, dim3(bs), 0, c->stream, (const TM *)im->LU, N, im->cnp,
-                           im->clow, r0, nr, r, tmp, y0end, (TV *)nullptr, lgB);
-      } else {
-        hipLaunchKernelGGL((k_ilu_lower<3, TM, TV, false>), g, dim3(bs), 0, c->stream, (const TM *)im->LU, N, im->cnp,
-                           im->clow, r0, nr, r, tmp, y0end, (TV *)nullptr, lgB);
+          hipLaunchKernelGGL((k_ilu_lower<ND, TM, TV, FUSE>), dim3(grid_for(nr * B, bs)), dim3(bs), 0, c->stream, LU, N,
+                             im->cnp, im->clow, r0, nr, r, tmp, y0end, x, lgB);
+      };
+      for (int col = 1; col < nc; col++) {
+        const int r0 = im->color_start[col], nr = im->color_start[col + 1] - r0;
+        if (nr == 0) continue;
+        if (col == nc - 1) lower(std::true_type{}, r0, nr);
+        else lower(std::false_type{}, r0, nr);
       }
-    }
-    for (int col = nc > 1 ? nc - 2 : nc - 1; col >= 0; col--) {
-      const int r0 = im->color_start[col], nr = im->color_start[col + 1] - r0;
-      if (nr == 0) continue;
-      if (c->nd == 2)
-        hipLaunchKernelGGL((k_ilu_upper<2, TM, TV>), dim3(grid_for(nr * B, bs)), dim3(bs), 0, c->stream,
-                           (const TM *)im->LU, N, im->cnp, im->clow, r0, nr, tmp, z, r, y0end, lgB);
-      else
-        hipLaunchKernelGGL((k_ilu_upper<3, TM, TV>), dim3(grid_for(nr * B, bs)), dim3(bs), 0, c->stream,
-                           (const TM *)im->LU, N, im->cnp, im->clow, r0, nr, tmp, z, r, y0end, lgB);
-    }
+      for (int col = nc > 1 ? nc - 2 : nc - 1; col >= 0; col--) {
+        const int r0 = im->color_start[col], nr = im->color_start[col + 1] - r0;
+        if (nr == 0) continue;
+        if (slots)
+          hipLaunchKernelGGL((k_ilu_slots<ND, TM, TV, true, true>), dim3(grid_for(nr * B, 64)), dim3(64 * (ND + 2)), 0,
+                             c->stream, LU, N, im->cnp, im->clow, r0, nr, r, tmp, y0end, z, z, lgB);
+        else
+          hipLaunchKernelGGL((k_ilu_upper<ND, TM, TV>), dim3(grid_for(nr * B, bs)), dim3(bs), 0, c->stream, LU, N,
+                             im->cnp, im->clow, r0, nr, tmp, z, r, y0end, lgB);
+      }
+    };
+    if (c->nd == 2) sweeps(std::integral_constant<int, 2>{});
+    else sweeps(std::integral_constant<int, 3>{});
   }
   BES_HIP(hipGetLastError());
   return BES_OK;
@@ -1713,17 +1864,21 @@ static int spmv(bes_ctx *c, Impl *im, const TV *x, TV *y) {
   // stored blocks, x and y once, neighbour ids
   ProfScope ps(c, kProfSpmv, (double)(c->N + 2 * im->ninternal) * c->nv * c->nv * sizeof(TM) * B +
                                  2.0 * c->N * c->nv * sizeof(TV) * B + 4.0 * c->N * c->k);
-  if (im->precond == 2) {   // ILU(0) solves run in colour order
-    if (c->nd == 2)
-      hipLaunchKernelGGL((k_spmv_pos<2, TM, TV>), dim3(grid_for(c->N * B, bs)), dim3(bs), 0, c->stream,
-                         (const TM *)im->Ac, im->cnp, c->N, x, y, lgB);
-    else
-      hipLaunchKernelGGL((k_spmv_pos<3, TM, TV>), dim3(grid_for(c->N * B, bs)), dim3(bs), 0, c->stream,
-                         (const TM *)im->Ac, im->cnp, c->N, x, y, lgB);
-  } else if (c->nd == 2) {
-    hipLaunchKernelGGL((k_spmv<2, TM, TV>), dim3(grid_for(c->N * B, bs)), dim3(bs), 0, c->stream, (const TM *)im->A, c->dm, x, y, lgB);
-  } else {
-    hipLaunchKernelGGL((k_spmv<3, TM, TV>), dim3(grid_for(c->N * B, bs)), dim3(bs), 0, c->stream, (const TM *)im->A, c->dm, x, y, lgB);
+  if (im->precond != 2) {
+    spmv_cells(c, (const TM *)im->A, x, y, bs);
+  } else {   // ILU(0) solves run in colour order
+    auto go = [&](auto ndc) {
+      constexpr int ND = decltype(ndc)::value;
+      const TM *A = (const TM *)im->Ac;
+      if (slot_split(c))
+        hipLaunchKernelGGL((k_spmv_slots<ND, TM, TV>), dim3(grid_for(c->N * B, 64)), dim3(64 * (ND + 2)), 0, c->stream,
+                           A, im->cnp, c->N, x, y, lgB);
+      else
+        hipLaunchKernelGGL((k_spmv_pos<ND, TM, TV>), dim3(grid_for(c->N * B, bs)), dim3(bs), 0, c->stream, A, im->cnp,
+                           c->N, x, y, lgB);
+    };
+    if (c->nd == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 3>{});
   }
   BES_HIP(hipGetLastError());
   return BES_OK;
