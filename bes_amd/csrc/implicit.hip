@@ -1899,7 +1899,7 @@ static void sum_lanes(bes_ctx *c, Impl *im, int nqb, double *out, int qnorm, Gat
 
 // dots h_q = V_q^T w (q < cnt) and ||w||^2 of every condition, reduced to row
 // at of the dots buffer (the deterministic lane reductions).  With defer, one
-// condition's last level may be left to k_orth_update: returns its S2 through
+// condition's last level may be left to the update kernels: returns its S2 through
 // *S2 (null: the dots are done).
 template <typename TV>
 static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, const TV *w, int at = 0,
