@@ -952,7 +952,7 @@ __global__ void k_jacobian_batch(int kind, int n, const double *__restrict__ UL,
   int col = dir < NV ? dir : dir - NV;
   if (!J) return;
 #pragma unroll
-  for (int o = 0; o < NV; o++) J[((size_t)f * NV + o) * NV + col] = out[o].d;
+  for (int o = 0; o < NV; o++) J[((size_t)f * NV + o) * NV + col] = out[o].d[0];
 }
 
 // ---------------------------------------------------------------------------

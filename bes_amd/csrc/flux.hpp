@@ -9,14 +9,15 @@
 //   Roe + Harten fix     FluxRoe.tpp:61-333
 //   far field            FluxFreestream.tpp:34-226
 //   slip wall            FluxSlipWall.tpp:32-53
-// The scalar type T is double, or Dual (value + one directional derivative)
+// The scalar type T is double, or DualN (value + M directional derivatives)
 // whose rules are those of the reference's Jacobian machinery (Eigen 3.3.4
 // AutoDiffScalar: product, quotient, sqrt, abs with sign(0)=+1, comparisons
-// on values), so one thread per Jacobian column reproduces the reference
-// Jacobian exactly.
+// on values), so every Jacobian column is the reference's exactly.
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "kernels_common.hpp"
 
@@ -26,33 +27,86 @@ struct GasConst {
   double gamma, R, harten, cv, cp;
 };
 
-struct Dual {
-  double v, d;
-  __device__ __forceinline__ Dual() {}
-  __device__ __forceinline__ Dual(double x) : v(x), d(0.0) {}
-  __device__ __forceinline__ Dual(double x, double dx) : v(x), d(dx) {}
+// M derivatives share the value, and with it every division and square root (the
+// quotient's and the root's derivatives scale by factors of the values only)
+template <int M>
+struct DualN {
+  double v, d[M];
+  __device__ __forceinline__ DualN() {}
+  __device__ __forceinline__ DualN(double x) : v(x) {
+#pragma unroll
+    for (int k = 0; k < M; k++) d[k] = 0.0;
+  }
+  __device__ __forceinline__ DualN(double x, double dx) : v(x) {   // derivative 0
+    static_assert(M == 1, "one derivative");
+    d[0] = dx;
+  }
+  // value v, derivatives f(k)
+  template <typename F>
+  static __device__ __forceinline__ DualN make(double v, F f) {
+    DualN r;
+    r.v = v;
+#pragma unroll
+    for (int k = 0; k < M; k++) r.d[k] = f(k);
+    return r;
+  }
+  friend __device__ __forceinline__ DualN operator+(const DualN &a, const DualN &b) {
+    return make(a.v + b.v, [&](int k) { return a.d[k] + b.d[k]; });
+  }
+  friend __device__ __forceinline__ DualN operator-(const DualN &a, const DualN &b) {
+    return make(a.v - b.v, [&](int k) { return a.d[k] - b.d[k]; });
+  }
+  friend __device__ __forceinline__ DualN operator-(const DualN &a) {
+    return make(-a.v, [&](int k) { return -a.d[k]; });
+  }
+  friend __device__ __forceinline__ DualN operator*(const DualN &a, const DualN &b) {
+    return make(a.v * b.v, [&](int k) { return a.d[k] * b.v + b.d[k] * a.v; });
+  }
+  friend __device__ __forceinline__ DualN operator/(const DualN &a, const DualN &b) {
+    const double i2 = 1.0 / (b.v * b.v);
+    return make(a.v / b.v, [&](int k) { return (a.d[k] * b.v - b.d[k] * a.v) * i2; });
+  }
+  friend __device__ __forceinline__ DualN operator+(const DualN &a, double s) {
+    return make(a.v + s, [&](int k) { return a.d[k]; });
+  }
+  friend __device__ __forceinline__ DualN operator+(double s, const DualN &a) {
+    return make(s + a.v, [&](int k) { return a.d[k]; });
+  }
+  friend __device__ __forceinline__ DualN operator-(const DualN &a, double s) {
+    return make(a.v - s, [&](int k) { return a.d[k]; });
+  }
+  friend __device__ __forceinline__ DualN operator-(double s, const DualN &a) {
+    return make(s - a.v, [&](int k) { return -a.d[k]; });
+  }
+  friend __device__ __forceinline__ DualN operator*(const DualN &a, double s) {
+    return make(a.v * s, [&](int k) { return a.d[k] * s; });
+  }
+  friend __device__ __forceinline__ DualN operator*(double s, const DualN &a) {
+    return make(a.v * s, [&](int k) { return a.d[k] * s; });
+  }
+  friend __device__ __forceinline__ DualN operator/(const DualN &a, double s) {
+    const double i = 1.0 / s;
+    return make(a.v / s, [&](int k) { return a.d[k] * i; });
+  }
+  friend __device__ __forceinline__ DualN operator/(double s, const DualN &a) {
+    const double i = (-s) / (a.v * a.v);
+    return make(s / a.v, [&](int k) { return a.d[k] * i; });
+  }
+  friend __device__ __forceinline__ DualN &operator+=(DualN &a, const DualN &b) { a = a + b; return a; }
+  friend __device__ __forceinline__ DualN &operator-=(DualN &a, const DualN &b) { a = a - b; return a; }
+  friend __device__ __forceinline__ DualN &operator+=(DualN &a, double s) { a = a + s; return a; }
+  friend __device__ __forceinline__ DualN &operator/=(DualN &a, double s) { a = a / s; return a; }
+  friend __device__ __forceinline__ DualN dsqrt(const DualN &a) {
+    const double s = ::sqrt(a.v), h = 0.5 / s;
+    return make(s, [&](int k) { return a.d[k] * h; });
+  }
+  friend __device__ __forceinline__ DualN dabs(const DualN &a) {
+    const double sg = a.v < 0 ? -1.0 : 1.0;
+    return make(::fabs(a.v), [&](int k) { return a.d[k] * sg; });
+  }
+  friend __device__ __forceinline__ double val(const DualN &a) { return a.v; }
 };
-__device__ __forceinline__ Dual operator+(Dual a, Dual b) { return Dual(a.v + b.v, a.d + b.d); }
-__device__ __forceinline__ Dual operator-(Dual a, Dual b) { return Dual(a.v - b.v, a.d - b.d); }
-__device__ __forceinline__ Dual operator-(Dual a) { return Dual(-a.v, -a.d); }
-__device__ __forceinline__ Dual operator*(Dual a, Dual b) { return Dual(a.v * b.v, a.d * b.v + b.d * a.v); }
-__device__ __forceinline__ Dual operator/(Dual a, Dual b) {
-  return Dual(a.v / b.v, (a.d * b.v - b.d * a.v) * (1.0 / (b.v * b.v)));
-}
-__device__ __forceinline__ Dual operator+(Dual a, double s) { return Dual(a.v + s, a.d); }
-__device__ __forceinline__ Dual operator+(double s, Dual a) { return Dual(s + a.v, a.d); }
-__device__ __forceinline__ Dual operator-(Dual a, double s) { return Dual(a.v - s, a.d); }
-__device__ __forceinline__ Dual operator-(double s, Dual a) { return Dual(s - a.v, -a.d); }
-__device__ __forceinline__ Dual operator*(Dual a, double s) { return Dual(a.v * s, a.d * s); }
-__device__ __forceinline__ Dual operator*(double s, Dual a) { return Dual(a.v * s, a.d * s); }
-__device__ __forceinline__ Dual operator/(Dual a, double s) { return Dual(a.v / s, a.d * (1.0 / s)); }
-__device__ __forceinline__ Dual operator/(double s, Dual a) { return Dual(s / a.v, a.d * ((-s) / (a.v * a.v))); }
-__device__ __forceinline__ Dual &operator+=(Dual &a, Dual b) { a = a + b; return a; }
-__device__ __forceinline__ Dual &operator-=(Dual &a, Dual b) { a = a - b; return a; }
-__device__ __forceinline__ Dual &operator/=(Dual &a, double s) { a = a / s; return a; }
-__device__ __forceinline__ Dual dsqrt(Dual a) { double s = ::sqrt(a.v); return Dual(s, a.d * (0.5 / s)); }
-__device__ __forceinline__ Dual dabs(Dual a) { return Dual(::fabs(a.v), a.d * (a.v < 0 ? -1.0 : 1.0)); }
-__device__ __forceinline__ double val(Dual a) { return a.v; }
+using Dual = DualN<1>;
 __device__ __forceinline__ double dsqrt(double a) { return ::sqrt(a); }
 __device__ __forceinline__ double dabs(double a) { return ::fabs(a); }
 __device__ __forceinline__ double val(double a) { return a; }
@@ -119,13 +173,19 @@ struct Gas {
   }
 };
 
-// Quotients by one divisor: for double the shared-reciprocal form (RcpDiv,
-// bitwise the division), for Dual the division itself.
+// Quotients by one divisor: the shared-reciprocal form (RcpDiv, bitwise the
+// division) for values, one factor 1 / b^2 for derivatives.
 template <typename T>
-struct Divider {
-  T b;
-  __device__ __forceinline__ explicit Divider(const T &b_) : b(b_) {}
-  __device__ __forceinline__ T operator()(const T &a) const { return a / b; }
+struct Divider;
+template <int M>
+struct Divider<DualN<M>> {
+  DualN<M> b;
+  RcpDiv r;
+  double i2;
+  __device__ __forceinline__ explicit Divider(const DualN<M> &b_) : b(b_), r(b_.v), i2(1.0 / (b_.v * b_.v)) {}
+  __device__ __forceinline__ DualN<M> operator()(const DualN<M> &a) const {
+    return DualN<M>::make(r(a.v), [&](int k) { return (a.d[k] * b.v - b.d[k] * a.v) * i2; });
+  }
 };
 template <>
 struct Divider<double> {
@@ -160,22 +220,27 @@ __device__ __forceinline__ T harten_fix(const T &lam, const T &delta) {
 }
 
 // Roe flux per unit area, left/right conserved states, unit normal left->right.
-template <int ND, typename T>
-__device__ __forceinline__ void roe_flux(const GasConst &gc, const T *UL, const T *UR,
+// With derivatives to one side only (TL or TR a DualN, the other double) the
+// products with that side's zero derivatives fall away.
+template <int ND, typename TL, typename TR = TL, typename T = std::conditional_t<std::is_same_v<TL, double>, TR, TL>>
+__device__ __forceinline__ void roe_flux(const GasConst &gc, const TL *UL, const TR *UR,
                                          const double *n, T *F) {
   constexpr int NV = ND + 2, IP = ND + 1;
-  Gas<ND, T> g(gc);
+  Gas<ND, TL> gl(gc);
+  Gas<ND, TR> gr(gc);
   // extended primitive states: [rho, u_d, p, T] + H, V (c and q^2 of the
   // sides enter only through the deltas, which the dissipation never uses)
-  T PL[ND + 3], PR[ND + 3], HL, HR, VL, VR;
-  roe_side<ND, T>(g, UL, n, PL, HL, VL);
-  roe_side<ND, T>(g, UR, n, PR, HR, VR);
+  TL PL[ND + 3], HL, VL;
+  TR PR[ND + 3], HR, VR;
+  roe_side<ND, TL>(gl, UL, n, PL, HL, VL);
+  roe_side<ND, TR>(gr, UR, n, PR, HR, VR);
   T dRho = PR[0] - PL[0], dP = PR[IP] - PL[IP], dV = VR - VL;
   T du[ND];
 #pragma unroll
   for (int d = 0; d < ND; d++) du[d] = PR[1 + d] - PL[1 + d];
   // Roe averages
-  T sl = dsqrt(PL[0]), sr = dsqrt(PR[0]);
+  const TL sl = dsqrt(PL[0]);
+  const TR sr = dsqrt(PR[0]);
   T den = sl + sr;
   const Divider<T> by_den(den);
   T aRho = dsqrt(PL[0] * PR[0]);
@@ -190,15 +255,16 @@ __device__ __forceinline__ void roe_flux(const GasConst &gc, const T *UL, const 
   T aH = by_den(HL * dsqrt(PL[0]) + HR * dsqrt(PR[0]));
   T aC = dsqrt((T(gc.gamma) - 1.0) * (aH - aQ / 2.0));
   // central part
-  T tmp[NV];
 #pragma unroll
   for (int i = 0; i < NV; i++) F[i] = 0.0;
-  g.flux(PL, n, tmp);
+  TL fl[NV];
+  gl.flux(PL, n, fl);
 #pragma unroll
-  for (int i = 0; i < NV; i++) F[i] += tmp[i];
-  g.flux(PR, n, tmp);
+  for (int i = 0; i < NV; i++) F[i] += fl[i];
+  TR fr[NV];
+  gr.flux(PR, n, fr);
 #pragma unroll
-  for (int i = 0; i < NV; i++) F[i] += tmp[i];
+  for (int i = 0; i < NV; i++) F[i] += fr[i];
   T delta = dabs(aC * gc.harten);
   const Divider<T> by_2c2(2.0 * aC * aC);
   {  // acoustic wave V - c

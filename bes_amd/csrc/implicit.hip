@@ -3,9 +3,9 @@
 // One backward-Euler pseudo-time step (SolverImplicit.cpp:293-345):
 //   k_timestep + k_gradlim          (explicit.hip)
 //   k_face_jacobian   first-order flux Jacobians dF/dU_L, dF/dU_R per face by
-//                     one-direction dual numbers with the reference's Eigen AD
-//                     rules (FluxJacobianWrapper.tpp:32-82), one thread per
-//                     (face, input column)
+//                     dual numbers with the reference's Eigen AD rules
+//                     (FluxJacobianWrapper.tpp:32-82), one thread per (face,
+//                     side), its nv derivatives sharing the values
 //   k_assemble        row-owned assembly: second-order fluxes give the right-
 //                     hand side b = -dt/V sum +-F*A; the block row gets
 //                     I + sum nV x (dt/V*A*J) in the reference's accumulation
@@ -67,45 +67,72 @@ struct JRec {
   static constexpr int P = (NB * (int)sizeof(TJ) + 15) / 16 * 16 / (int)sizeof(TJ);
 };
 
+// Both blocks of a face, a thread per side (and condition).  Bound by FP64
+// arithmetic: the values' divisions and square roots, which a thread per input
+// column repeated for each of the 2 nv columns, and then the derivatives, whose
+// registers leave one wave per SIMD in 3D (346; capped at 256 it spills: 2042 us).
+// 4M faces FP64 1820 -> 1294 us, 64k faces x 16 conditions FP32 444 -> 258, 60k
+// triangle faces 26 -> 14; two columns to a thread 1536 and 328.
 template <int ND, typename TJ>
 __global__ __launch_bounds__(256) void k_face_jacobian(const double *__restrict__ U, int N, FaceDev fd,
                                                        GasConst gc, const double *__restrict__ finf,
                                                        TJ *__restrict__ JF, int lgB) {
   constexpr int NV = ND + 2, NB = NV * NV, JP = JRec<TJ, NB>::P;
-  // groups of 64 lanes x 2nv input directions: the lanes of a wave take 64/B
-  // consecutive faces x B conditions of one direction, and the group's waves
-  // reuse the same face states through the cache and fill the same face
-  // records; a face's two blocks sit side by side in one record [2][JP] (JL,
+  using D = DualN<NV>;
+  // groups of 64 lanes x 2 sides: the lanes of a wave take 64/B consecutive faces
+  // x B conditions and all nv derivatives to one side, which share the values'
+  // arithmetic; a face's two blocks sit side by side in one record [2][JP] (JL,
   // then JR, row-major), entry e of condition b at (rec + e)*B + b
   const int B = 1 << lgB;
   const int t = xcd_block() * blockDim.x + threadIdx.x;
-  const int grp = t / (64 * 2 * NV), rem = t - grp * (64 * 2 * NV);
-  const int dir = rem >> 6, l = rem & 63;
-  const int f = grp * (64 >> lgB) + (l >> lgB), b = l & (B - 1);
+  const bool right = __builtin_amdgcn_readfirstlane((t >> 6) & 1);
+  const int l = t & 63;
+  const int f = (t >> 7) * (64 >> lgB) + (l >> lgB), b = l & (B - 1);
   if (f >= fd.F) return;
   const int o = fd.fo[f], j = fd.fn[f];
-  if (j < 0 && dir >= NV) return;   // boundary faces: left Jacobian only
+  if (j < 0 && right) return;   // boundary faces: left Jacobian only
   double nn[ND];
 #pragma unroll
   for (int d = 0; d < ND; d++) nn[d] = fd.fnrm[(size_t)d * fd.F + f];
-  Dual ul[NV], ur[NV + 1], F[NV];
+  D F[NV];
+  double xl[NV], xr[NV + 1];
 #pragma unroll
-  for (int v = 0; v < NV; v++) ul[v] = Dual(U[((size_t)v * N + o) * B + b], dir == v ? 1.0 : 0.0);
+  for (int v = 0; v < NV; v++) xl[v] = U[((size_t)v * N + o) * B + b];
   if (j >= 0) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) ur[v] = Dual(U[((size_t)v * N + j) * B + b], dir == NV + v ? 1.0 : 0.0);
-    roe_flux<ND, Dual>(gc, ul, ur, nn, F);
+    for (int v = 0; v < NV; v++) xr[v] = U[((size_t)v * N + j) * B + b];
+  }
+  D u[NV];   // the state differentiated by: its value's derivatives are the unit vectors
+#pragma unroll
+  for (int v = 0; v < NV; v++)
+    u[v] = D::make(right ? xr[v] : xl[v], [&](int k) { return k == v ? 1.0 : 0.0; });
+  if (j >= 0) {
+    if (right) roe_flux<ND, double, D>(gc, xl, u, nn, F);
+    else roe_flux<ND, D, double>(gc, u, xr, nn, F);
   } else if (j == -1) {
-    slip_flux<ND, Dual>(gc, ul, nn, F);
+    slip_flux<ND, D>(gc, u, nn, F);
+  } else {
+    D ui[NV + 1];
+#pragma unroll
+    for (int v = 0; v < NV + 1; v++) ui[v] = D(finf[b * (NV + 1) + v]);
+    freestream_flux<ND, D>(gc, u, ui, nn, F);
+  }
+  TJ *rec = JF + ((size_t)f * 2 + right) * JP * B;
+  if (lgB == 0) {   // 16-byte stores of the record
+    constexpr int W = 16 / (int)sizeof(TJ);
+    TJ out[JP];
+#pragma unroll
+    for (int e = 0; e < JP; e++) out[e] = e < NB ? (TJ)F[e < NB ? e / NV : 0].d[e < NB ? e % NV : 0] : (TJ)0;
+#pragma unroll
+    for (int q = 0; q < JP / W; q++) {
+      uint4 w;
+      __builtin_memcpy(&w, out + q * W, 16);
+      reinterpret_cast<uint4 *>(rec)[q] = w;
+    }
   } else {
 #pragma unroll
-    for (int v = 0; v < NV + 1; v++) ur[v] = Dual(finf[b * (NV + 1) + v]);
-    freestream_flux<ND, Dual>(gc, ul, ur, nn, F);
+    for (int e = 0; e < NB; e++) rec[(size_t)e * B + b] = (TJ)F[e / NV].d[e % NV];
   }
-  const int side = dir < NV ? 0 : 1, col = dir < NV ? dir : dir - NV;
-  TJ *rec = JF + ((size_t)f * 2 + side) * JP * B;
-#pragma unroll
-  for (int r = 0; r < NV; r++) rec[(size_t)(r * NV + col) * B + b] = (TJ)F[r].d;
 }
 
 // one padded block record (16-byte aligned, JP entries) into registers as doubles
@@ -1685,7 +1712,7 @@ static int launch_assemble(bes_ctx *c, Impl *im) {
     ProfScope ps(c, kProfJacobian, (double)im->fd.F * (16.0 * c->nv * B + 8.0 * c->nd + 8.0) +
                                        (double)(im->fd.F + im->ninternal) * nbl * sizeof(TM) * B);
     const int groups = (im->fd.F + (64 >> lgB) - 1) / (64 >> lgB);   // groups of 64 lanes
-    const int nt = groups * 64 * 2 * c->nv;
+    const int nt = groups * 64 * 2;
     if (c->nd == 2)
       hipLaunchKernelGGL((k_face_jacobian<2, TM>), dim3(grid_for(nt, bsj)), dim3(bsj), 0, c->stream, c->U0, c->N,
                          im->fd, c->gc, c->dfinf, (TM *)im->JF, lgB);
