@@ -1793,13 +1793,13 @@ static int factor(bes_ctx *c, Impl *im) {
   return BES_OK;
 }
 
-// z = M^-1 r (B conditions at once for the block Jacobi and ILU(0) forms)
 // A thread per block (k_spmv_slots, k_ilu_slots) or per cell and condition.  One
 // condition gathers its neighbours' values 40 bytes apart and a colour of a small
 // mesh is a few waves, so the split pays while a launch does not fill the chip
-// with loads: at 1M cells 4 to 8 % are left, at 2M both take the same time.  A
-// batch fills it earlier and its gathers are contiguous: FP64 gains 5 % and FP32
-// nothing at 250k cell-conditions, both lose 1 to 3 % at 500k.
+// with loads: at 590k cells a product still takes 8 % less (FP32 6), at 2M both
+// take the same time and the line lies between.  A batch fills it earlier and its
+// gathers are contiguous: FP64 gains 5 % and FP32 nothing at 250k cell-conditions;
+// at 500k FP64 gains 2 % and FP32 loses up to 3 %.
 static bool slot_split(const bes_ctx *c) { return (size_t)c->N * c->B <= (c->B == 1 ? 1u << 20 : 1u << 18); }
 
 // y = A x, matrix and vectors in cell order
@@ -1818,6 +1818,7 @@ static void spmv_cells(bes_ctx *c, const TM *A, const TV *x, TV *y, int bs) {
   else go(std::integral_constant<int, 3>{});
 }
 
+// z = M^-1 r (B conditions at once for the block Jacobi and ILU(0) forms)
 template <typename TM, typename TV>
 static int precond_apply(bes_ctx *c, Impl *im, const TV *r, TV *z, TV *tmp) {
   if (im->precond == 4) return amg_apply<TV>(c, im, r, z, tmp);
