@@ -902,8 +902,7 @@ __device__ __forceinline__ void ld_lanes(const TV *__restrict__ v, size_t e, siz
 
 // Dot products <V_q, w>, q < cnt, and ||w||^2 (row cnt) per lane, all chunks
 // of Q vectors in one launch (blockIdx.y; w is read once per chunk).  A thread
-// is one lane of VB neighbouring conditions (VB = 4 where the batch allows it:
-// 16-byte loads).  One condition: the block's lanes (lane_of) are summed here
+// is one lane of VB neighbouring conditions (quad_of).  One condition: the block's lanes (lane_of) are summed here
 // as level 1 of the lane sums does, out is S2[row][G][4]; a batch stores the
 // lane sums S[row*B + b][L].
 // Bound by HBM on the 2M wing; on small meshes by the number of waves (L is
@@ -1925,10 +1924,19 @@ static void sum_lanes(bes_ctx *c, Impl *im, int nqb, double *out, int qnorm, Gat
   }
 }
 
+// Four conditions a thread in the dot products and the thread-per-lane update,
+// where their values are one 16-byte load.  FP64 takes two, 32 bytes a thread
+// apart, on a quarter of the threads: solves of 250k tetrahedra x 4 took 7.58 ms
+// so and 6.79 with a condition a thread (with DGKS 9.32 and 7.82), 486k x 8 28.7
+// and 27.8, 120k x 16 13.05 and 12.82, 31k x 64 10.22 and 10.16.  FP32: 250k x 4
+// 4.01 and 3.97, 31k x 16 1.69 and 1.78, 83k x 32 8.05 and 8.24.
+template <typename TV>
+static bool quad_of(int lgB) { return sizeof(TV) == 4 && lgB >= 2; }
+
 // dots h_q = V_q^T w (q < cnt) and ||w||^2 of every condition, reduced to row
-// at of the dots buffer (the deterministic lane reductions).  With defer, one
-// condition's last level may be left to the update kernels: returns its S2 through
-// *S2 (null: the dots are done).
+// at of the dots buffer (the deterministic lane reductions).  With S2 given, one
+// condition's last level may be left to the update kernels: *S2 is then its
+// level-1 sums (null: the dots are done).
 template <typename TV>
 static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, const TV *w, int at = 0,
                     Gate gate = Gate(), const double **S2 = nullptr) {
@@ -1936,7 +1944,7 @@ static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, c
   const size_t n1 = (size_t)c->N * c->nv;
   if (S2) *S2 = nullptr;
   if (cnt > im->restart + 1) { set_error("too many basis vectors"); return BES_ERR_ARG; }
-  const bool quad = lgB >= 2;
+  const bool quad = quad_of<TV>(lgB);
   // vectors per thread: as many as leave about four waves on every SIMD
   const size_t units = (size_t)L * (quad ? B / 4 : B);
   int qmax = quad ? 2 : 8;
@@ -1952,8 +1960,10 @@ static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, c
   };
   using std::integral_constant;
   if (quad) {
-    if (Q == 1) go(integral_constant<int, 4>{}, integral_constant<int, 1>{});
-    else go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+    if constexpr (sizeof(TV) == 4) {
+      if (Q == 1) go(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+      else go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+    }
   } else {
     const integral_constant<int, 1> one;
     switch (Q) {
@@ -1975,8 +1985,8 @@ static int multidot(bes_ctx *c, Impl *im, const TV *V, size_t stride, int cnt, c
   return BES_OK;
 }
 
-// Up to this many lanes (times conditions over the kernel's VB) the update runs
-// a thread per lane group: past it a thread per lane gives at least a wave for
+// Up to this many lanes (times conditions, over four where a batch has as many)
+// the update runs a thread per lane group: past it a thread per lane gives at least a wave for
 // every other SIMD, and the sixteenfold blocks with their barrier cost more (486k
 // tetrahedra, 2^16 lanes, FP32: 79 us against 34; the 2M wing 371 against 232).
 constexpr size_t kSlotUnits = 16384;
@@ -2015,13 +2025,18 @@ static int orthogonalise(bes_ctx *c, Impl *im, const TV *V, size_t stride, int c
     else go(std::integral_constant<int, 1>{});
     hipLaunchKernelGGL(k_sum_lanes, dim3(1), dim3(256), 0, c->stream, im->S, G, out, -1, 0, gate, keep);
   } else {
-    const dim3 grid((unsigned)((units + 255) / 256));
-    if (lgB >= 2)
-      hipLaunchKernelGGL((k_orth_lanes<TV, 4, 1>), grid, dim3(256), lds, c->stream, V, stride, cnt, S2, G, d, w, n1,
-                         lgB, L, im->S, gate);
-    else
-      hipLaunchKernelGGL((k_orth_lanes<TV, 1, 1>), grid, dim3(256), lds, c->stream, V, stride, cnt, S2, G, d, w, n1,
-                         lgB, L, im->S, gate);
+    auto go = [&](auto vb) {
+      constexpr int VB = decltype(vb)::value;
+      const size_t nt = (size_t)L * (B / VB);
+      hipLaunchKernelGGL((k_orth_lanes<TV, VB, 1>), dim3((unsigned)((nt + 255) / 256)), dim3(256), lds, c->stream, V,
+                         stride, cnt, S2, G, d, w, n1, lgB, L, im->S, gate);
+    };
+    if constexpr (sizeof(TV) == 4) {
+      if (quad_of<TV>(lgB)) go(std::integral_constant<int, 4>{});
+      else go(std::integral_constant<int, 1>{});
+    } else {
+      go(std::integral_constant<int, 1>{});
+    }
     sum_lanes(c, im, B, out, -1, gate, keep);
   }
   BES_HIP(hipGetLastError());

@@ -63,6 +63,8 @@ def test_iterate_matches_numpy(ni, nj, eta):
 
 # a condition's iterates are the same bits in a batch as alone: scalar loads
 # (B = 2), four conditions a thread (B >= 4), either form of the update
+# (both forms for B = 2, the thread-per-group one for larger batches: the other,
+# and their lane sums in two launches, are in test_gpu_batch_reductions.py)
 @pytest.mark.parametrize("precision", [64, 32])
 @pytest.mark.parametrize("ni,nj,B", [(20, 11, 2), (20, 11, 4), (64, 33, 8), (90, 47, 64), (300, 221, 2)])
 @pytest.mark.parametrize("eta", [0.0, 0.7])
