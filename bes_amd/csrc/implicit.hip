@@ -2056,6 +2056,19 @@ static int fetch_dots(bes_ctx *c, Impl *im, size_t ndbl) {
   return BES_OK;
 }
 
+// Whether a step queues the next one's preconditioner and product before the host
+// has read h and ||w||: it saves the device the host's turn (10 to 20 us a step)
+// and costs one application and product at the end of a cycle, discarded.
+// Without DGKS every step does.  With it (queue / wait, ms, DGKS 0.7): 83k
+// tetrahedra FP64 7 iterations 1.04 / 1.05, 46 iterations 6.39 / 6.68; 31k x 8
+// FP32 4 iterations 0.81 / 0.78, 19 iterations 3.29 / 3.36; 250k x 4 FP64 6
+// iterations 5.33 / 4.91, 23 iterations 23.6 / 23.3; 2M FP64 17 iterations 31.8 /
+// 30.9.  An AMG cycle costs more than it hides: 83k 9 iterations 1.80 / 1.76, 486k 12
+// iterations 5.07 / 4.86.
+static bool queue_ahead(const bes_ctx *c, const Impl *im) {
+  return im->reorth_eta <= 0 || (im->precond != 4 && (size_t)c->N * c->B <= (1u << 17));
+}
+
 // GMRES(m), right-preconditioned, for the B conditions of the batch at once
 // (one launch per kernel for all of them).  Each condition keeps its own
 // Arnoldi process, Givens rotations, iteration count and stopping point: a
@@ -2086,6 +2099,7 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
   const double *hd = im->hdots;
   const double eta = im->reorth_eta;
   auto hdot = [&](int row, int q, int b) { return hd[(size_t)(row + dot_row(q)) * B + b]; };
+  const bool ahead = queue_ahead(c, im);
   const int scale_blocks = (int)std::min<size_t>(kRedBlocks, (n / 4 + 255) / 256 + 1);
   // ||b|| per condition
   hipLaunchKernelGGL((k_scale<double, TV>), dim3(kRedBlocks), dim3(256), 0, c->stream, bb, 1.0, Z, n);
@@ -2169,11 +2183,11 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
       BES_HIP(hipGetLastError());
       BES_HIP(hipEventRecord(im->ev_dots, c->stream));
       // the next step's preconditioner and product need only the normalised w:
-      // queue them before waiting, so the device works while the host reads h
-      // and ||w|| (their results are discarded for conditions this step ends)
+      // queued before waiting (queue_ahead), they run while the host reads h and
+      // ||w|| (their results are discarded for conditions this step ends)
       bool more = false;
       for (int b = 0; b < B; b++) if (active[b] && total[b] + 1 < im->maxiter) more = true;
-      if (j + 1 < m && more) {
+      if (ahead && j + 1 < m && more) {
         if ((s = precond_apply<TM, TV>(c, im, w, Z, Z1))) return s;
         if ((s = spmv<TM, TV>(c, im, Z, V + (size_t)(j + 2) * vs))) return s;
         queued = true;
