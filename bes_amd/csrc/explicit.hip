@@ -1223,10 +1223,11 @@ void by_mesh(const bes_ctx *c, Fn &&f) {
   else forms(std::integral_constant<int, 3>{});
 }
 
-// algorithmic HBM bytes of one gradient+limiter launch: state, geometry, pack
-double gradlim_bytes(const bes_ctx *c) {
+// algorithmic HBM bytes of one gradient+limiter launch: state, geometry, pack;
+// with the time step in it, the projected areas and dt
+double gradlim_bytes(const bes_ctx *c, bool dt = false) {
   const double N = c->N, B = c->B, nv = c->nv, nd = c->nd, k = c->k;
-  return N * (8 * nv * B + k * (4 + 16 * nd + 8) + 16 + 8.0 * c->pw * B);
+  return N * (8 * nv * B + k * (4 + 16 * nd + 8) + 16 + 8.0 * c->pw * B + (dt ? 8 * nd + 8 * B : 0));
 }
 
 // Up to this many (cell, condition) units a pass is bound by the length of a
@@ -1249,7 +1250,7 @@ static int xcd_order(const bes_ctx *c) { return (long)c->N * c->B <= (1 << 20); 
 // for the split form only
 int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout, const StageAux *aux = nullptr) {
   const int bs = tuned_bs(c, kProfGradlim), nb = grid_for(c->N * c->B, bs);
-  ProfScope ps(c, kProfGradlim, gradlim_bytes(c));
+  ProfScope ps(c, kProfGradlim, gradlim_bytes(c, aux && aux->dt));
   CoefB fm;
   for (int b = 0; b < bes_ctx::kMaxBatch; b++)
     fm.c[b] = (b < (int)c->lim_frozen.size() && c->lim_frozen[b]) ? 1.0 : 0.0;
@@ -1303,18 +1304,25 @@ double residual_bytes(const bes_ctx *c, bool update, bool rout) {
          (double)c->dm.F * 8 * c->fs * B;
 }
 
+// the same from the packs (k_residual_faces): face geometry and packs once, the
+// neighbours and face order of each cell, no face fluxes in memory
+double residual_faces_bytes(const bes_ctx *c, bool update, bool rout) {
+  const double F = c->dm.F, N = c->N, B = c->B, nd = c->nd, k = c->k;
+  return residual_bytes(c, update, rout) - F * 8 * c->fs * B + N * (4 * k + 4 + 8.0 * c->pw * B) +
+         F * (c->common ? 8 : 24) * nd;
+}
+
 // residual of the packs of the last gradient pass; with U0/Ud the stage update
 int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int local, double *Rout,
                     unsigned long long *linf_bits) {
   const double *dtg = local ? nullptr : c->dtg;
   if (split_pass(c)) {
-    // the packs of both sides and the face records per cell face
-    ProfScope ps(c, kProfResidual, residual_bytes(c, U0 != nullptr, Rout != nullptr) + faceflux_bytes(c));
+    ProfScope ps(c, kProfResidual, residual_faces_bytes(c, U0 != nullptr, Rout != nullptr));
     by_mesh(c, [&](auto nd, auto one, auto rc) {
       constexpr int ND = decltype(nd)::value;
       hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual_faces<ND, decltype(one)::value, decltype(rc)::value>),
-                         dim3(grid_for(c->N * c->B, 64)), dim3(64 * (ND + 2)), 0, c->stream, c->LG, c->dm, c->gc, c->dfinf, U0, Ud, c->dt, dtg, alpha,
-                         Rout, linf_bits, c->err, c->lgB);
+                         dim3(grid_for(c->N * c->B, 64)), dim3(64 * (ND + 2)), 0, c->stream, c->LG, c->dm, c->gc,
+                         c->dfinf, U0, Ud, c->dt, dtg, alpha, Rout, linf_bits, c->err, c->lgB);
     });
     BES_HIP(hipGetLastError());
     return BES_OK;
