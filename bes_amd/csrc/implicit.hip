@@ -2169,12 +2169,15 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
       // pass (its kernels look up which conditions need it) and the
       // normalisation are queued back to back and the host waits once, for h
       // and ||w||
+      size_t ev2 = 0, ev2_end = 0;   // profile records of the second pass
       if (eta > 0) {
         if ((s = orthogonalise<TV>(c, im, V, vs, j + 1, w, 0, kDotNorm1))) return s;
         Gate gate;
         gate.eta = eta;
         gate.dots = im->dots;
+        ev2 = c->ev_pending.size();
         if ((s = orthogonalise<TV>(c, im, V, vs, j + 1, w, kDots2, kDotNorm, gate))) return s;
+        ev2_end = c->ev_pending.size();
       } else if ((s = orthogonalise<TV>(c, im, V, vs, j + 1, w, 0, kDotNorm))) {
         return s;
       }
@@ -2193,10 +2196,17 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
         queued = true;
       }
       BES_HIP(hipEventSynchronize(im->ev_dots));
+      auto second = [&](int b) {
+        return eta > 0 && std::sqrt(hd[(size_t)kDotNorm1 * B + b]) < eta * std::sqrt(hd[(size_t)8 * B + b]);
+      };
+      bool any = false;
+      for (int b = 0; b < B; b++) any = any || second(b);
+      if (!any)   // its kernels returned at once
+        for (size_t e = ev2; e < ev2_end; e++) c->ev_pending[e].bytes = 0.0;
       for (int b = 0; b < B; b++) {
         if (!active[b]) continue;
         const double hn = std::sqrt(hd[(size_t)kDotNorm * B + b]);
-        const bool re = eta > 0 && std::sqrt(hd[(size_t)kDotNorm1 * B + b]) < eta * std::sqrt(hd[(size_t)8 * B + b]);
+        const bool re = second(b);
         for (int q = 0; q <= j; q++) hcol[q] = re ? hdot(0, q, b) + hdot(kDots2, q, b) : hdot(0, q, b);
         if (re) im->reorths++;
         hcol[j + 1] = hn;

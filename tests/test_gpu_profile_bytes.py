@@ -1,6 +1,6 @@
 """Algorithmic bytes that the profile reports for the explicit passes: every
 array a launch touches, once, in the split passes of small meshes and the
-separate ones of larger meshes."""
+separate ones of larger meshes; and for the Gram-Schmidt passes that did work."""
 import numpy as np
 import pytest
 
@@ -51,3 +51,28 @@ def test_bytes_of_the_explicit_passes(mesh, B, split, local, mode):
         assert got["residual"] == cell + F * 8 * fs * B
     if "timestep" in p:
         assert got["timestep"] == step
+
+
+# a second pass that no condition needs moves nothing
+@pytest.mark.parametrize("ni,nj,B", [(40, 20, 1), (40, 20, 4), (331, 299, 1)])
+def test_bytes_of_an_idle_second_pass(ni, nj, B):
+    md = mg.bump_channel(ni, nj)
+    P = core.freestream_primitive((0.5, 0.0), 2)
+    rng = np.random.default_rng(1)
+    U = core.conserved_from_primitive(P, 2) * (1.0 + 0.01 * rng.uniform(-1, 1, (B, md.ncell, 4)))
+    print("case", md.ncell, B, flush=True)
+    bytes_of, reorths = {}, {}
+    for eta in (0.0, 1e-9, 1.0):
+        with core.Context(md) as c:
+            c.set_batch(B)
+            c.set_freestream(np.tile(P, (B, 1)) if B > 1 else P)
+            c.set_state(U if B > 1 else U[0])
+            c.implicit_setup(64, "ilu0", maxiter=8, rtol=1e-14)
+            c.implicit_set_reorth(eta)
+            c.implicit_assemble(20.0)
+            c.set_profiling(True)
+            c.linear_solve(allow_unconverged=True)
+            bytes_of[eta] = c.profile()["krylov"]["bytes"]
+            reorths[eta] = c.implicit_stats()["reorths"]
+    assert reorths == {0.0: 0, 1e-9: 0, 1.0: 8 * B}
+    assert bytes_of[1e-9] == bytes_of[0.0] < bytes_of[1.0]
