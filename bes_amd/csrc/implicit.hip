@@ -817,8 +817,9 @@ __device__ __forceinline__ void st_group(TV *__restrict__ v, size_t e, size_t n1
 // Rows of the reduced values in the dots buffer (B conditions each): the dot
 // products of the first Gram-Schmidt pass from row 0 and of the second from row
 // kDots2, product q at 9*(q/8) + q%8 with ||w||^2 at row 8 of each; ||w||^2
-// after the update the step ends with, and after its first pass.
-constexpr int kDots2 = 48, kDotNorm = 40, kDotNorm1 = 41, kDotRows = 96;
+// after the update the step ends with, and after its first pass; on the host,
+// whether the second pass was taken (1.0 or 0.0).
+constexpr int kDots2 = 48, kDotNorm = 40, kDotNorm1 = 41, kDotSecond = 42, kDotRows = 96;
 __host__ __device__ constexpr int dot_row(int q) { return 9 * (q / 8) + q % 8; }
 
 // DGKS: condition b takes a second pass when the first left less than eta of
@@ -1317,16 +1318,20 @@ __device__ __forceinline__ void st4(T *p, const double x[4]) {
 // w = w / sqrt(||w||^2) per condition when that is > 0, the norm (row kDotNorm
 // of dots) read on the device, so the launch need not wait for the host.  Block 0
 // hands the host the first ndots values of dots (a copy of its own took 2.7 us
-// a step and its gap).  (Summing the lane norms here too, by every block, took
-// 8.6 us where the sum and this take 7.3: 40k triangles.)
+// a step and its gap), with the gate's decision in row kDotSecond, so that the
+// host adds a second pass's products exactly where the kernels used them.
+// (Summing the lane norms here too, by every block, took 8.6 us where the sum and
+// this take 7.3: 40k triangles.)
 template <typename TV>
 __global__ __launch_bounds__(256) void k_scale_norm(TV *__restrict__ w, const double *__restrict__ dots,
-                                                    double *__restrict__ hdots, int ndots, size_t n, int lgB) {
+                                                    double *__restrict__ hdots, int ndots, size_t n, int lgB,
+                                                    Gate gate) {
   const size_t B = (size_t)1 << lgB, tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x,
                nt = (size_t)gridDim.x * blockDim.x, ng = n / 4;
   const double *n2 = dots + kDotNorm * B;
   if (blockIdx.x == 0)
-    for (int q = threadIdx.x; q < ndots; q += blockDim.x) hdots[q] = dots[q];
+    for (int q = threadIdx.x; q < ndots; q += blockDim.x)
+      hdots[q] = q >> lgB != kDotSecond ? dots[q] : (gate.second(q & ((int)B - 1), (int)B) ? 1.0 : 0.0);
   double a[4];
   bool on[4];
 #pragma unroll
@@ -2170,9 +2175,9 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
       // normalisation are queued back to back and the host waits once, for h
       // and ||w||
       size_t ev2 = 0, ev2_end = 0;   // profile records of the second pass
+      Gate gate;
       if (eta > 0) {
         if ((s = orthogonalise<TV>(c, im, V, vs, j + 1, w, 0, kDotNorm1))) return s;
-        Gate gate;
         gate.eta = eta;
         gate.dots = im->dots;
         ev2 = c->ev_pending.size();
@@ -2182,7 +2187,7 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
         return s;
       }
       hipLaunchKernelGGL((k_scale_norm<TV>), dim3(scale_blocks), dim3(256), 0, c->stream, w, im->dots,
-                         im->hdots, (eta > 0 ? kDotRows : kDotNorm + 1) * B, n, lgB);
+                         im->hdots, (eta > 0 ? kDotRows : kDotNorm + 1) * B, n, lgB, gate);
       BES_HIP(hipGetLastError());
       BES_HIP(hipEventRecord(im->ev_dots, c->stream));
       // the next step's preconditioner and product need only the normalised w:
@@ -2196,9 +2201,7 @@ static int gmres(bes_ctx *c, Impl *im, int *iters_out, double *relres_out) {
         queued = true;
       }
       BES_HIP(hipEventSynchronize(im->ev_dots));
-      auto second = [&](int b) {
-        return eta > 0 && std::sqrt(hd[(size_t)kDotNorm1 * B + b]) < eta * std::sqrt(hd[(size_t)8 * B + b]);
-      };
+      auto second = [&](int b) { return eta > 0 && hd[(size_t)kDotSecond * B + b] != 0.0; };
       bool any = false;
       for (int b = 0; b < B; b++) any = any || second(b);
       if (!any)   // its kernels returned at once
