@@ -1237,7 +1237,7 @@ double gradlim_bytes(const bes_ctx *c, bool dt = false) {
 // 48k 80 / 105, 83k 122 / 138, 105k 147 / 150, 132k 171 / 178, 179k 215 / 192;
 // batches: 8 x 10k tetrahedra 119 / 121, 32 x 3k 128 / 123, 64 x 2.4k triangles
 // 105 / 111, 64 x 4k 148 / 138.
-static bool split_pass(const bes_ctx *c) { return (long)c->N * c->B <= (c->nd == 2 ? 196608 : 90112); }
+bool split_pass(const bes_ctx *c) { return (long)c->N * c->B <= (c->nd == 2 ? 196608 : 90112); }
 
 // Block order of the per-pass kernels: up to this many units each XCD takes one
 // range of cells in every pass, so part of what a pass reads is still in its L2

@@ -43,6 +43,7 @@ namespace bes {
 int launch_timestep(bes_ctx *c, const double *U, double cfl, int local, const double *cfl_b = nullptr);
 int launch_face_flux(bes_ctx *c);
 struct StageAux;   // explicit.hip
+bool split_pass(const bes_ctx *c);
 int launch_gradlim(bes_ctx *c, const double *U, double *Gout, double *Pout, const StageAux *aux = nullptr);
 int launch_residual(bes_ctx *c, const double *U0, double *Ud, double alpha, int local, double *Rout,
                     unsigned long long *linf_bits);
@@ -2840,7 +2841,10 @@ int bes_autotune(bes_ctx *c, int flags, int *chosen, double *best_us, int *color
   double best[bes_ctx::kProfKinds];
   for (int k = 0; k < bes_ctx::kProfKinds; k++) best[k] = 0;
   int s = BES_OK;
-  auto tune = [&](int kind, auto fn) -> int {
+  // fixed: the launch does not take the kind's block size at the context's size
+  // (it is timed, the size kept)
+  auto tune = [&](int kind, auto fn, bool fixed = false) -> int {
+    if (fixed) return time_us(c, 5, fn, &best[kind]);
     double bt = 1e300;
     int bb = 256;
     for (int bs : cand) {
@@ -2863,14 +2867,15 @@ int bes_autotune(bes_ctx *c, int flags, int *chosen, double *best_us, int *color
     if (!s) s = tune(kProfFactor, fact);
     if (!s) {
       const size_t vs = im->vstride;
+      const bool slots = slot_split(c), sweeps = im->precond == 2 && slots;
       if (p64) {
         double *V = (double *)im->V, *Z = (double *)im->Z;
-        s = tune(kProfSpmv, [&]() { return spmv<double, double>(c, im, V, V + vs); });
-        if (!s) s = tune(kProfPrecond, [&]() { return precond_apply<double, double>(c, im, V, Z, Z + vs); });
+        s = tune(kProfSpmv, [&]() { return spmv<double, double>(c, im, V, V + vs); }, slots);
+        if (!s) s = tune(kProfPrecond, [&]() { return precond_apply<double, double>(c, im, V, Z, Z + vs); }, sweeps);
       } else {
         float *V = (float *)im->V, *Z = (float *)im->Z;
-        s = tune(kProfSpmv, [&]() { return spmv<float, float>(c, im, V, V + vs); });
-        if (!s) s = tune(kProfPrecond, [&]() { return precond_apply<float, float>(c, im, V, Z, Z + vs); });
+        s = tune(kProfSpmv, [&]() { return spmv<float, float>(c, im, V, V + vs); }, slots);
+        if (!s) s = tune(kProfPrecond, [&]() { return precond_apply<float, float>(c, im, V, Z, Z + vs); }, sweeps);
       }
     }
     im->factored = false;
@@ -2893,10 +2898,12 @@ int bes_autotune(bes_ctx *c, int flags, int *chosen, double *best_us, int *color
   }
   if (!s && (flags & 1)) {   // explicit kernels on the current state, last: the time step it leaves is at CFL 1
     // (U0 is read, never written; the next assembly or explicit step recomputes dt)
-    s = tune(kProfGradlim, [&]() { return launch_gradlim(c, c->U0, nullptr, nullptr); });
+    s = tune(kProfGradlim, [&]() { return launch_gradlim(c, c->U0, nullptr, nullptr); }, split_pass(c));
     if (!s) s = tune(kProfTimestep, [&]() { return launch_timestep(c, c->U0, 1.0, 1); });
     if (!s) s = tune(kProfFaceFlux, [&]() { return launch_face_flux(c); });
-    if (!s) s = tune(kProfResidual, [&]() { return launch_residual(c, nullptr, nullptr, 0.0, 1, nullptr, nullptr); });
+    if (!s)
+      s = tune(kProfResidual, [&]() { return launch_residual(c, nullptr, nullptr, 0.0, 1, nullptr, nullptr); },
+               split_pass(c));
   }
   if (!s) BES_HIP(hipStreamSynchronize(c->stream));
   c->prof = prof;

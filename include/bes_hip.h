@@ -369,7 +369,8 @@ int bes_set_profiling(bes_ctx *ctx, int on);
 /* autotuner (no reference counterpart; the reference's counterpart is its
  * OpenMP schedule, SolverExplicit.cpp:285): times each tunable kernel kind at
  * block sizes 64, 128 and 256 on the context's current data with HIP events
- * and keeps the fastest.  flags: 1 the explicit kernels (gradient and
+ * and keeps the fastest (a kind whose kernel has one block size at the
+ * context's cells and conditions is timed only).  flags: 1 the explicit kernels (gradient and
  * limiter, time step, face flux, residual) on the current state; 2 the implicit kernels (Jacobians, assembly,
  * factorisation, SpMV, preconditioner, update) on the assembled system, which
  * is assembled and factored again (same values); 4 the ILU(0) colouring order

@@ -40,3 +40,21 @@ def test_autotune_keeps_results():
         c.set_state(U)
         linf = c.explicit_run(2, 0.8)
         assert np.array_equal(c.get_state(), Uref) and np.array_equal(linf, lref)
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_kernels_of_one_block_size_keep_it(precision):
+    """On a small mesh the gradient, residual, product and ILU(0) kernels have one
+    block size each: timing three settings of it would pick one by chance."""
+    md = mg.bump_channel(40, 20, seed=5)
+    finf = orc.freestream_primitive((0.5, 0.0), 2)
+    print("case", md.ncell, precision, flush=True)
+    for _ in range(4):
+        with core.Context(md) as c:
+            c.set_freestream(finf)
+            c.set_state(orc.perturbed_state(md.ncell, 2, (0.5, 0.0), seed=17))
+            c.implicit_setup(precision, "ilu0")
+            c.implicit_assemble(20.0)
+            tuned, _ = c.autotune(explicit=True, implicit=True)
+        for kind in ("gradlim", "residual", "spmv", "precond"):
+            assert tuned[kind][0] == 256 and tuned[kind][1] > 0, kind
