@@ -60,6 +60,26 @@ FORM_KERNEL_NAMES = {
 }
 
 
+# Sizes up to which the library splits a cell's work over threads: explicit
+# passes by cells x conditions in 2D and 3D; of one condition, products and
+# ILU(0) sweeps by cells, the Gram-Schmidt update by values of a vector (64 a lane).
+SPLIT_PASS = {2: 196608, 3: 90112}
+SLOT_SPLIT = 1 << 20
+ORTH_SLOTS = 16384 * 64
+
+
+def form_names(nd, ncell, nbatch=1):
+    """Names of the kernels that the sizes select, where they are not KERNEL_NAMES'."""
+    names = {}
+    if ncell * nbatch <= SPLIT_PASS[nd]:
+        names.update(gradlim="k_gradlim_split", residual="k_residual_faces")
+    if nbatch == 1 and ncell <= SLOT_SPLIT:
+        names.update(spmv="k_spmv_slots", precond="k_ilu_slots")
+    if nbatch == 1 and ncell * (nd + 2) <= ORTH_SLOTS:
+        names["krylov"] = "k_mdot+k_orth_slots"
+    return names
+
+
 def roofline(prof, names=None):
     names = {**KERNEL_NAMES, **(names or {})}
     kern = {k: v for k, v in prof.items() if v["ms"] > 0}
@@ -67,7 +87,7 @@ def roofline(prof, names=None):
     d = kern[dom]
     avg_ms = d["ms"] / d["launches"]
     name = names.get(dom, dom)
-    tr = traffic_from_profiles(name)
+    tr = traffic_from_profiles(name, d["bytes"] / d["launches"])
     return {"bound": "hbm", "kernel": name, "achieved": round(d["GBps"], 1),
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(d["GBps"] / HBM_PEAK_GBS, 4),
             "traffic": tr["bytes_per_launch"] if tr else None,
@@ -233,7 +253,7 @@ def implicit_workload(args):
         log(f"timed {args.steps} steps in {wall:.3f}s (CFL {hist[0, 10]:.1f} -> {hist[-1, 10]:.1f}, "
             f"{int(hist[:, 11].sum())} Krylov iterations)")
         value = md.ncell * args.steps / wall
-        out["roofline"] = roofline(prof, FORM_KERNEL_NAMES.get(args.timed_form))
+        out["roofline"] = roofline(prof, {**form_names(3, md.ncell), **FORM_KERNEL_NAMES.get(args.timed_form, {})})
         out["timed_steps"] = {"ramp_steps_to_cap": nramp, "warmup_steps": args.warmup,
                               "cfl_first": float(hist[0, 10]), "cfl_last": float(hist[-1, 10]),
                               "cfl_min": float(hist[:, 10].min()),
@@ -525,7 +545,7 @@ def explicit_workload(args):
     out = {"metric": METRIC, "value": md.ncell * args.steps / wall, "unit": "cell-updates/s", "n_gpus": 1,
            "steps": args.steps, "warmup": args.warmup, "ms_per_step": wall * 1e3 / args.steps,
            "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f64",
-           "data": "synthetic", "config": cfg, "roofline": roofline(prof),
+           "data": "synthetic", "config": cfg, "roofline": roofline(prof, form_names(nd, md.ncell)),
            "residual_linf_last": [float(x) for x in linf[-1]]}
     if not args.no_cpu:
         out["cpu_baseline"] = cpu_baseline_explicit(args, nd)
@@ -584,7 +604,7 @@ def sweep_workload(args):
     out = {"metric": METRIC, "value": md.ncell * B * args.steps / wall, "unit": "cell-updates/s",
            "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": wall * 1e3 / args.steps,
            "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f64",
-           "data": "synthetic", "config": cfg, "roofline": roofline(prof),
+           "data": "synthetic", "config": cfg, "roofline": roofline(prof, form_names(3, md.ncell, B)),
            "residual_linf_last_max": float(np.max(linf[-1]))}
     if not args.no_cpu:
         out["cpu_baseline"] = cpu_baseline_explicit(args, 3)
@@ -875,14 +895,18 @@ def copy_probe():
                       "ms_per_sum": ms_read, "GBps_read": n * 4 / (ms_read * 1e-3) / 1e9}))
 
 
-def traffic_from_profiles(kernel):
-    """HBM bytes per launch of a kernel as measured by the committed counter runs."""
+def traffic_from_profiles(kernel, alg_bytes):
+    """HBM bytes per launch of a kernel as measured by the committed counter runs;
+    None where those ran another size or form of it: their algorithmic bytes
+    are not this run's (within a twentieth: Gram-Schmidt launches vary)."""
     path = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     if not os.path.exists(path):
         return None
     with open(path) as fh:
         table = json.load(fh)
-    return table.get(kernel)
+    tr = table.get(kernel)
+    ref = tr.get("algorithmic_bytes") if tr else None
+    return None if ref and abs(alg_bytes - ref) > 0.05 * ref else tr
 
 
 def main():
