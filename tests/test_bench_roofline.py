@@ -29,6 +29,15 @@ def test_traffic_is_of_the_same_launch(kind, kernel):
         assert r["traffic"] is None and r["traffic_source"] is None
 
 
+def test_traffic_table_names_kernels_of_the_bench():
+    names = set(bench.KERNEL_NAMES.values()) | {n for f in bench.FORM_KERNEL_NAMES.values() for n in f.values()}
+    with open(os.path.join(ROOT, "profiles", "hbm_traffic_pmc.md")) as fh:
+        source = fh.read()
+    for kernel, row in _table().items():
+        assert kernel in names
+        assert f"| `{kernel}` | {row['what']} |" in source, kernel
+
+
 def test_small_meshes_name_their_kernels():
     p = _prof("residual", 1e6)
     assert bench.roofline(p, bench.form_names(2, 40000))["kernel"] == "k_residual_faces"
