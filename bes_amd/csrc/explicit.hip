@@ -1441,6 +1441,12 @@ static void drop_graph(bes_ctx *c) {
   c->graph = nullptr;
 }
 
+// the state slots change places after a one-stage step (a capture holds the old ones)
+static void swap_slots(bes_ctx *c) {
+  std::swap(c->U0, c->Ua);
+  drop_graph(c);
+}
+
 // (Re)allocate every per-condition array for a batch of B conditions
 static int resize_batch(bes_ctx *c, int B) {
   if (c->stream) BES_HIP(hipStreamSynchronize(c->stream));
@@ -1765,7 +1771,7 @@ static int explicit_iteration(bes_ctx *c, int nstage, const double *alpha, doubl
                          it_host < 0 ? 0 : it_host, c->linf_cap, it_host < 0 ? c->dit : nullptr);
       BES_HIP(hipGetLastError());
     }
-    if (last && nstage == 1) std::swap(c->U0, c->Ua);
+    if (last && nstage == 1) swap_slots(c);
   }
   return BES_OK;
 }
@@ -1843,7 +1849,7 @@ static int explicit_run_persistent(bes_ctx *c, int niter, int nstage, const doub
   const int grid = std::max(1, std::min(per_cu * ncu, want));   // all blocks resident: the barriers complete
   void *args[] = {&a, &c->dm, &c->gc, &fm};
   BES_HIP(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(bs), args, (unsigned)lds, c->stream));
-  if (nstage == 1 && niter % 2 == 1) std::swap(c->U0, c->Ua);
+  if (nstage == 1 && niter % 2 == 1) swap_slots(c);
   return BES_OK;
 }
 
