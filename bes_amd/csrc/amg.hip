@@ -1197,7 +1197,9 @@ __global__ __launch_bounds__(64) void k_densify(Acc a, int n, double *__restrict
 // pivot row, pivot and multipliers; k_gj_update applies the steps in order to the
 // columns right of the panel, so every entry goes through the operations of the
 // column-by-column form.  That one took a launch of 4.9 us a column (58 block rows:
-// 290 launches, 1.42 ms; this 38, 1.05 ms); bound by the panels' chain of steps.
+// 290 launches, 1.42 ms; this 38, 1.05 ms; assembly and build with a coarsest
+// system of the largest size, 1024 rows in panels of 4: 23.6 ms, now 11.9); bound
+// by the panels' chain of steps.
 constexpr int kGjP = 16;
 constexpr int kGjThreads = 512;
 __global__ __launch_bounds__(kGjThreads) void k_gj_panel(const double *__restrict__ M, int m, int k0, int np,

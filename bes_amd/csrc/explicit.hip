@@ -4,15 +4,16 @@
 //   k_timestep   local dt per cell + global minimum (TimeStepCalculator*.cpp)
 //   per stage:
 //     k_gradlim  Green-Gauss gradient fused with the Venkatakrishnan limiter,
-//                writes the limited gradient phi*grad (GradientGreenGauss.cpp:21-135,
-//                LimiterVenkatakrishnan.cpp:21-128)
-//     k_residual second-order face fluxes gathered per cell, summed in the
-//                reference face order, fused with the stage update
-//                U = U0 - alpha*dt/V*R and the Linf monitor
-//                (SolverExplicit.cpp:285-378, Solver.cpp:69-121)
-// One thread per cell; every cell computes the fluxes of its own faces, so no
-// atomics touch the residual and the result is deterministic.  Blocks are
-// remapped so that each XCD walks a contiguous range of Morton-ordered cells.
+//                writes the reconstructed state or the limited gradient
+//                (GradientGreenGauss.cpp:21-135, LimiterVenkatakrishnan.cpp:21-128)
+//     k_face_flux      second-order flux of every face (Solver.cpp:69-121)
+//     k_cell_residual  fluxes gathered per cell, summed in the reference face
+//                order, fused with the stage update U = U0 - alpha*dt/V*R and
+//                the Linf monitor (SolverExplicit.cpp:285-378)
+// On small meshes k_gradlim_split (with the time step) and k_residual_faces (both
+// of the last) deal a cell's work over several threads (split_pass).  A cell's
+// residual is summed by one thread, so no atomics touch it and the result is
+// deterministic.
 #include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
 
