@@ -1401,7 +1401,9 @@ static int move_rows(bes_ctx *c, double *dev, size_t sq, size_t si, int ncomp, d
     const std::vector<int> ip(c->iperm.begin(), c->iperm.end());
     if ((s = upload(&c->diperm, ip))) return s;
   }
-  const size_t ct = kMoveRows / B, cells = std::max<size_t>(c->stage_bytes / (B * row) / ct, 1) * ct;
+  // the whole mesh where it fits (one copy), else whole blocks of cells
+  const size_t ct = kMoveRows / B, room = c->stage_bytes / (B * row);
+  const size_t cells = room >= N ? N : std::max<size_t>(room / ct, 1) * ct;
   for (size_t e0 = 0; e0 < N; e0 += cells) {
     const size_t ne = std::min(cells, N - e0);
     auto kernel = [&]() {

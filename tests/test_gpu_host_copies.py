@@ -1,5 +1,7 @@
 """Host copies of per-cell arrays: the device-side permutation between the
 callers' order and the device layout, against the values themselves."""
+import time
+
 import numpy as np
 import pytest
 
@@ -58,3 +60,26 @@ def test_gradient_and_limiter_values(n, B):
         assert np.array_equal(P, single[0][1] if B == 1 else np.stack([s[1] for s in single]))
         c.freeze_limiter_values(0.5 * P)
         assert np.array_equal(c.gradient_limiter()[1], 0.5 * P)
+
+
+@pytest.mark.parametrize("B", [16, 64])
+def test_ragged_counts_copy_in_one_piece(B):
+    """A cell count that no block of the permutation divides takes about what its
+    neighbour does (cut in two chunks, every condition's part would be a copy of its
+    own)."""
+    took = {}
+    for ni in (640, 641):   # 3,840 cells: whole blocks; 3,846: not
+        md = mg.bump_channel(ni, 3)
+        U = np.tile(_states(md, 1, 7), (B, 1, 1))
+        with core.Context(md) as c:
+            c.set_batch(B)
+            c.set_state(U)
+            ts = []
+            for _ in range(15):
+                t = time.perf_counter()
+                out = c.get_state()
+                ts.append(time.perf_counter() - t)
+            assert np.array_equal(out, U)
+            took[md.ncell] = sorted(ts)[7]
+    print("seconds", took)
+    assert took[3846] < 3 * took[3840]
