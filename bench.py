@@ -61,7 +61,7 @@ FORM_KERNEL_NAMES = {
 
 
 # Sizes up to which the library splits a cell's work over threads: explicit
-# passes by cells x conditions in 2D and 3D; of one condition, products and
+# passes by cells x conditions in 2D and 3D (the default geometry mode); of one condition, products and
 # ILU(0) sweeps by cells, the Gram-Schmidt update by values of a vector (64 a lane).
 SPLIT_PASS = {2: 196608, 3: 90112}
 SLOT_SPLIT = 1 << 20

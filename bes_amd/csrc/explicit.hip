@@ -1237,8 +1237,15 @@ double gradlim_bytes(const bes_ctx *c, bool dt = false) {
 // 97, 160k 112 / 123, 250k 152 / 154, 360k 200 / 192; tetrahedra 25k 60 / 88,
 // 48k 80 / 105, 83k 122 / 138, 105k 147 / 150, 132k 171 / 178, 179k 215 / 192;
 // batches: 8 x 10k tetrahedra 119 / 121, 32 x 3k 128 / 123, 64 x 2.4k triangles
-// 105 / 111, 64 x 4k 148 / 138.
-bool split_pass(const bes_ctx *c) { return (long)c->N * c->B <= (c->nd == 2 ? 196608 : 90112); }
+// 105 / 111, 64 x 4k 148 / 138.  With a reconstruction vector per face the packs,
+// which the split form reads from both cells of a face, are three times as long
+// and the line lies lower: tetrahedra 35k 92 / 100, 46k 100 / 108, 56k 122 / 114,
+// 79k 151 / 146, 8 x 5.4k 89 / 94, 8 x 6.6k 118 / 97; triangles 100k 107 / 106,
+// 130k 123 / 113, 64 x 1.6k 87 / 91, 64 x 2k 104 / 102.
+bool split_pass(const bes_ctx *c) {
+  const long line = c->common ? (c->nd == 2 ? 196608 : 90112) : (c->nd == 2 ? 98304 : 49152);
+  return (long)c->N * c->B <= line;
+}
 
 // Block order of the per-pass kernels: up to this many units each XCD takes one
 // range of cells in every pass, so part of what a pass reads is still in its L2

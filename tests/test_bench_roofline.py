@@ -53,8 +53,7 @@ def test_size_lines_are_the_library_s():
         with open(os.path.join(ROOT, "bes_amd", "csrc", name)) as fh:
             return fh.read()
 
-    m = re.search(r"split_pass\(const bes_ctx \*c\) \{ return \(long\)c->N \* c->B <= \(c->nd == 2 \? (\d+) : (\d+)\)",
-                  source("explicit.hip"))
+    m = re.search(r"line = c->common \? \(c->nd == 2 \? (\d+) : (\d+)\)", source("explicit.hip"))
     assert bench.SPLIT_PASS == {2: int(m[1]), 3: int(m[2])}
     imp = source("implicit.hip")
     m = re.search(r"slot_split\(const bes_ctx \*c\) \{ return [^}]*c->B == 1 \? 1u << (\d+)", imp)
